@@ -7,10 +7,11 @@
 //
 //  plan (once per LOR set; geometry only):
 //    kRayPrep     resolve every (LOR, ray) once into the ray table
-//    kBin<COUNT>  walk every ray, count tile entries per tile (LDS counters,
-//                 one global atomic per tile and workgroup)
+//    kBin<COUNT>  cut every ray at its tiles (sidPieces), count tile entries
+//                 per tile (LDS counters, one global atomic per tile and
+//                 workgroup)
 //    host         prefix sum -> tile ranges, chunk table
-//    kBin<FILL>   walk again, write one record per tile entry into its
+//    kBin<FILL>   cut again, write one record per tile entry into its
 //                 tile's range: key = lor * R + ray, the alpha where the
 //                 walk enters the tile, the voxel it enters and the ray's
 //                 plane shift (sidPlaneShift); a DD record is the LOR alone
@@ -100,10 +101,11 @@ __global__ void __launch_bounds__(256) kRayPrep(KArgs a, float4* __restrict__ ta
 	}
 }
 
-// Walks ray t of the ray table and calls onRecord(tile, alpha, packed
-// entry, segments) for each tile the walk passes through, once the walk has
-// left it (so the piece's number of segments is known).  A plane shift
-// beyond the record's range sets *err (the ray is not binned).
+// The pieces of ray t of the ray table: onRecord(tile, alpha, packed entry,
+// segments) for each tile its walk passes through.  FP32 set-up: cut tile by
+// tile (sidPieces); FP64: by walking it (its first planes have the set-up's
+// own alphas).  A plane shift beyond the record's range sets *err (the ray
+// is not binned).
 template <bool TOF, bool S64, class Fn>
 __device__ __forceinline__ void binRay(const DImage& im, const DTof& tof, const DTiles& T,
                                        const float4* __restrict__ tab, uint32_t t, int* err,
@@ -118,12 +120,25 @@ __device__ __forceinline__ void binRay(const DImage& im, const DTof& tof, const 
 	SidRay s;
 	if (!sidSetup<TOF, S64>(im, q1, q2, tof, Bq.z, s))
 		return;
-	int dx, dy, dz;
-	if (!sidPlaneShift<S64>(im, s, dx, dy, dz))
+	int ex, ey, ez, dx, dy, dz;
+	if (!sidFirst<S64>(im, s, ex, ey, ez, dx, dy, dz))
 		return;
 	if (abs(dx) > kMaxShift || abs(dy) > kMaxShift || abs(dz) > kMaxShift)
 	{
 		atomicOr(err, 2);
+		return;
+	}
+	if constexpr (!S64)
+	{
+		bool first = true;
+		sidPieces(im, s, T.lx, T.ly, T.lz, ex, ey, ez, dx, dy, dz,
+		          [&](float a0, int vx, int vy, int vz, int segs) {
+			          onRecord(tileOf(T, frame, vx, vy, vz), a0,
+			                   packEntry(vx & (T.tx - 1), vy & (T.ty - 1), vz & (T.tz - 1), dx,
+			                             dy, dz, first),
+			                   segs);
+			          first = false;
+		          });
 		return;
 	}
 	int last = -1, start = 0, nseg = 0;
