@@ -1563,7 +1563,6 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	const int64_t tabBytes = tabVec * (int64_t)sizeof(float4) * l->n * (int64_t)R;
 	if (o.max_bytes > 0 && (int64_t)sizeof(float) * l->n + tabBytes > o.max_bytes)
 		return fail(YRTMI_ENOMEM, "plan: the ray table exceeds the memory budget");
-	const int CH = o.chunk_records > 0 ? o.chunk_records : 4096;
 	DTiles T{};
 	T.shape = o.tile_shape;
 	T.tx = tileDim(T.shape, 0);
@@ -1602,8 +1601,8 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	q->T = T;
 	q->persistent = o.persistent;
 	// [0] next chunk, [1] finished workgroups (persistent launches),
-	// [2] fixed-point scale exponent of the current launch, [3] unused,
-	// [4 .. 259] exponent histogram of its values
+	// [2] fixed-point scale exponent of the current launch, [3] workgroups
+	// done counting, [4 .. 259] exponent histogram of its values (kVExpScale)
 	if (hipMalloc(&q->queue, 260 * sizeof(unsigned int)) != hipSuccess ||
 	    hipMemset(q->queue, 0, 260 * sizeof(unsigned int)) != hipSuccess)
 	{
@@ -1711,6 +1710,10 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	std::vector<int64_t> off(nB);
 	std::vector<TileChunk> chunks;
 	int64_t total = 0;
+	for (int64_t b = 0; b < nB; b++)
+		total += (int64_t)cnt[b];
+	const int CH = o.chunk_records > 0 ? o.chunk_records : chunkRecords(total);
+	total = 0;
 	for (int64_t t = 0; t < nT; t++)
 	{
 		const int64_t begin = total;
