@@ -6,6 +6,7 @@
 #include "yrtmi_tiles.hpp"
 #include "yrtmi_f64.hpp"
 #include "yrtmi_order.hpp"
+#include "yrtmi_pool.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -271,7 +272,7 @@ int ensurePartials(yrtmi_ctx* c, int64_t n)
 	HIP_TRY(hipFree(c->part));
 	c->part = nullptr;
 	c->partStride = 0;
-	HIP_TRY(hipMalloc(&c->part, sizeof(float) * stride * c->nxcc));
+	HIP_TRY(poolMalloc(c->device, &c->part, sizeof(float) * stride * c->nxcc));
 	HIP_TRY(hipMemset(c->part, 0, sizeof(float) * stride * c->nxcc));
 	c->partStride = stride;
 	return YRTMI_OK;
@@ -291,7 +292,7 @@ int ensureBrick(yrtmi_ctx* c, int64_t need)
 		HIP_TRY(hipFree(c->brick));
 		c->brick = nullptr;
 		c->brickCap = 0;
-		HIP_TRY(hipMalloc(&c->brick, sizeof(float) * need));
+		HIP_TRY(poolMalloc(c->device, &c->brick, sizeof(float) * need));
 		c->brickCap = need;
 	}
 	return YRTMI_OK;
@@ -379,6 +380,7 @@ int yrtmi_ctx_create(int device, void* stream, yrtmi_ctx** out)
 		delete c;
 		return hipFail(e, "yrtmi_ctx_create");
 	}
+	poolRetain(device);
 	*out = c;
 	return YRTMI_OK;
 }
@@ -400,6 +402,7 @@ int yrtmi_ctx_destroy(yrtmi_ctx* c)
 	(void)hipFree(c->brick);
 	if (c->owned != nullptr)
 		(void)hipStreamDestroy(c->owned);
+	poolRelease(c->device);
 	delete c;
 	return YRTMI_OK;
 }
@@ -1454,11 +1457,13 @@ namespace
 
 void freePlan(yrtmi_plan* q)
 {
-	hipFree(q->rec);
-	hipFree(q->ray);
-	hipFree(q->chunks);
-	hipFree(q->v);
-	hipFree(q->queue);
+	// calls on any stream, and graphs, may still be using it
+	const bool idle = poolQuiesce(q->device);
+	poolFree(q->device, q->rec, idle);
+	poolFree(q->device, q->ray, idle);
+	poolFree(q->device, q->chunks, idle);
+	poolFree(q->device, q->v, idle);
+	poolFree(q->device, q->queue, idle);
 	delete q;
 }
 
@@ -1603,14 +1608,14 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	// [0] next chunk, [1] finished workgroups (persistent launches),
 	// [2] fixed-point scale exponent of the current launch, [3] workgroups
 	// done counting, [4 .. 259] exponent histogram of its values (kVExpScale)
-	if (hipMalloc(&q->queue, 260 * sizeof(unsigned int)) != hipSuccess ||
-	    hipMemset(q->queue, 0, 260 * sizeof(unsigned int)) != hipSuccess)
+	if (poolAlloc(c->device, &q->queue, 260 * sizeof(unsigned int)) != hipSuccess ||
+	    hipMemsetAsync(q->queue, 0, 260 * sizeof(unsigned int), c->stream) != hipSuccess)
 	{
 		freePlan(q);
 		return fail(YRTMI_ENOMEM, "plan: chunk queue");
 	}
 	if (l->n > 0)
-		if (hipMalloc(&q->v, sizeof(float) * l->n) != hipSuccess)
+		if (poolAlloc(c->device, &q->v, sizeof(float) * l->n) != hipSuccess)
 		{
 			freePlan(q);
 			return fail(YRTMI_ENOMEM, "plan: value buffer");
@@ -1624,11 +1629,13 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	int64_t* dOff = nullptr;
 	int* dErr = nullptr;
 	auto cleanup = [&](int rc) {
-		hipFree(dCount);
-		hipFree(dCursor);
-		hipFree(dBlockCnt);
-		hipFree(dOff);
-		hipFree(dErr);
+		// (a plan is returned after its stream has been waited for)
+		const bool idle = rc == YRTMI_OK || poolQuiesce(c->device);
+		poolFree(c->device, dCount, idle);
+		poolFree(c->device, dCursor, idle);
+		poolFree(c->device, dBlockCnt, idle);
+		poolFree(c->device, dOff, idle);
+		poolFree(c->device, dErr, idle);
 		if (rc != YRTMI_OK)
 			freePlan(q);
 		else
@@ -1670,13 +1677,13 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	const int64_t nB = nT * pl.C;
 	const int64_t rays = l->n * (int64_t)R;
 	const int grid = (int)std::min<int64_t>((rays + 255) / 256, 2048);
-	if (hipMalloc(&dCount, sizeof(unsigned long long) * nB) != hipSuccess ||
-	    hipMalloc(&dCursor, sizeof(unsigned int) * nB) != hipSuccess ||
-	    hipMalloc(&dBlockCnt, sizeof(unsigned int) * nB * grid) != hipSuccess ||
-	    hipMalloc(&dOff, sizeof(int64_t) * nB) != hipSuccess ||
-	    hipMalloc(&dErr, sizeof(int)) != hipSuccess)
+	if (poolAlloc(c->device, &dCount, sizeof(unsigned long long) * nB) != hipSuccess ||
+	    poolAlloc(c->device, &dCursor, sizeof(unsigned int) * nB) != hipSuccess ||
+	    poolAlloc(c->device, &dBlockCnt, sizeof(unsigned int) * nB * grid) != hipSuccess ||
+	    poolAlloc(c->device, &dOff, sizeof(int64_t) * nB) != hipSuccess ||
+	    poolAlloc(c->device, &dErr, sizeof(int)) != hipSuccess)
 		return cleanup(fail(YRTMI_ENOMEM, "plan: build scratch"));
-	if (hipMalloc(&q->ray, tabVec * sizeof(float4) * rays) != hipSuccess)
+	if (poolAlloc(c->device, &q->ray, tabVec * sizeof(float4) * rays) != hipSuccess)
 		return cleanup(fail(YRTMI_ENOMEM, "plan: ray table"));
 	q->bytes += rays * tabVec * (int64_t)sizeof(float4);
 	hipError_t e = hipMemsetAsync(dCount, 0, sizeof(unsigned long long) * nB, c->stream);
@@ -1752,8 +1759,8 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	if (total > 0)
 	{
 		// records of 12 B (Siddon) / 8 B (DD: no alpha)
-		if (hipMalloc(&q->rec, sizeof(uint32_t) * recWords(dd) * total) != hipSuccess ||
-		    hipMalloc(&q->chunks, sizeof(TileChunk) * chunks.size()) != hipSuccess)
+		if (poolAlloc(c->device, &q->rec, sizeof(uint32_t) * recWords(dd) * total) != hipSuccess ||
+		    poolAlloc(c->device, &q->chunks, sizeof(TileChunk) * chunks.size()) != hipSuccess)
 			return cleanup(fail(YRTMI_ENOMEM, "plan: records"));
 		q->bytes += total * (dd ? 8 : 12) + (int64_t)(sizeof(TileChunk) * chunks.size());
 		e = hipMemcpyAsync(dOff, off.data(), sizeof(int64_t) * nB,
@@ -1981,6 +1988,8 @@ int yrtmi_mem_info(yrtmi_ctx* c, int64_t* free_bytes, int64_t* total_bytes)
 	int r = setDev(c);
 	if (r)
 		return r;
+	// what the library keeps for reuse counts as free: it goes back first
+	poolTrim(c->device);
 	size_t fr = 0, tot = 0;
 	HIP_TRY(hipMemGetInfo(&fr, &tot));
 	if (free_bytes != nullptr)
@@ -2003,7 +2012,7 @@ int yrtmi_device_alloc(yrtmi_ctx* c, int64_t bytes, void** out)
 	*out = nullptr;
 	if (bytes == 0)
 		return YRTMI_OK;
-	if (hipMalloc(out, (size_t)bytes) != hipSuccess)
+	if (poolMalloc(c->device, out, (size_t)bytes) != hipSuccess)
 	{
 		*out = nullptr;
 		return fail(YRTMI_ENOMEM, "device_alloc: out of device memory");
@@ -2089,12 +2098,13 @@ int yrtmi_histo_subset_nonzero(yrtmi_ctx* c, const float* values, int S, int s,
 	int* dCnt = nullptr;
 	int64_t* dOff = nullptr;
 	auto done = [&](int rc) {
-		hipFree(dCnt);
-		hipFree(dOff);
+		// (the stream has been waited for, but for an error)
+		poolFree(c->device, dCnt, rc == YRTMI_OK);
+		poolFree(c->device, dOff, rc == YRTMI_OK);
 		return rc;
 	};
-	if (hipMalloc(&dCnt, sizeof(int) * nb) != hipSuccess ||
-	    hipMalloc(&dOff, sizeof(int64_t) * nb) != hipSuccess)
+	if (poolAlloc(c->device, &dCnt, sizeof(int) * nb) != hipSuccess ||
+	    poolAlloc(c->device, &dOff, sizeof(int64_t) * nb) != hipSuccess)
 		return done(fail(YRTMI_ENOMEM, "histo_subset_nonzero: scratch"));
 	std::vector<int> hc(nb);
 	std::vector<int64_t> ho(nb);
@@ -2266,16 +2276,17 @@ int yrtmi_autotune(yrtmi_ctx* c, yrtmi_proj* p, const yrtmi_image* im,
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 	const int64_t ny = a.im.nvox * a.im.nt;
 	auto done = [&](int rc) {
-		hipFree(v);
-		hipFree(y);
+		// (the last timing has been waited for, but for an error)
+		poolFree(c->device, v, rc == YRTMI_OK);
+		poolFree(c->device, y, rc == YRTMI_OK);
 		if (e0)
 			hipEventDestroy(e0);
 		if (e1)
 			hipEventDestroy(e1);
 		return rc;
 	};
-	if (hipMalloc(&v, sizeof(float) * l->n) != hipSuccess ||
-	    hipMalloc(&y, sizeof(float) * ny) != hipSuccess)
+	if (poolAlloc(c->device, &v, sizeof(float) * l->n) != hipSuccess ||
+	    poolAlloc(c->device, &y, sizeof(float) * ny) != hipSuccess)
 		return done(fail(YRTMI_ENOMEM, "autotune: temporaries"));
 	if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
 		return done(fail(YRTMI_EHIP, "autotune: events"));

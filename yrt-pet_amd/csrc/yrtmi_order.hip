@@ -9,6 +9,7 @@
 // midpoint and tilt) at neighbouring transaxial angles and offsets, and the
 // voxels a window of concurrent waves reads fit in L2.
 #include "yrtmi_order.hpp"
+#include "yrtmi_pool.hpp"
 
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -91,11 +92,14 @@ hipError_t lorOrder(const DScanner& S, const DLors& L, const DImage& im, uint32_
 	uint32_t* iin = nullptr;
 	void* tmp = nullptr;
 	size_t tmpBytes = 0;
-	hipError_t e = hipMalloc(&kin, sizeof(uint64_t) * n);
+	int dev = 0;
+	hipError_t e = hipGetDevice(&dev);
 	if (e == hipSuccess)
-		e = hipMalloc(&kout, sizeof(uint64_t) * n);
+		e = poolAlloc(dev, &kin, sizeof(uint64_t) * n);
 	if (e == hipSuccess)
-		e = hipMalloc(&iin, sizeof(uint32_t) * n);
+		e = poolAlloc(dev, &kout, sizeof(uint64_t) * n);
+	if (e == hipSuccess)
+		e = poolAlloc(dev, &iin, sizeof(uint32_t) * n);
 	if (e == hipSuccess)
 	{
 		kLorKey<<<gridFor(n), 256, 0, st>>>(S, L, im, kin, iin);
@@ -105,17 +109,17 @@ hipError_t lorOrder(const DScanner& S, const DLors& L, const DImage& im, uint32_
 		e = rocprim::radix_sort_pairs(nullptr, tmpBytes, kin, kout, iin, perm, (size_t)n, 0,
 		                              60, st);
 	if (e == hipSuccess)
-		e = hipMalloc(&tmp, std::max<size_t>(tmpBytes, 1));
+		e = poolAlloc(dev, &tmp, std::max<size_t>(tmpBytes, 1));
 	if (e == hipSuccess)
 		e = rocprim::radix_sort_pairs(tmp, tmpBytes, kin, kout, iin, perm, (size_t)n, 0, 60,
 		                              st);
 	if (e == hipSuccess)
 		e = hipStreamSynchronize(st);
-	// hipFree waits for the device; the buffers are released on every path
-	(void)hipFree(kin);
-	(void)hipFree(kout);
-	(void)hipFree(iin);
-	(void)hipFree(tmp);
+	// the stream has been waited for, but for an error
+	poolFree(dev, kin, e == hipSuccess);
+	poolFree(dev, kout, e == hipSuccess);
+	poolFree(dev, iin, e == hipSuccess);
+	poolFree(dev, tmp, e == hipSuccess);
 	return e;
 }
 
