@@ -1676,7 +1676,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	}
 	const int64_t nB = nT * pl.C;
 	const int64_t rays = l->n * (int64_t)R;
-	const int grid = (int)std::min<int64_t>((rays + 255) / 256, 2048);
+	const int grid = (int)std::min<int64_t>((rays + kBinThreads - 1) / kBinThreads, 2048);
 	if (poolAlloc(c->device, &dCount, sizeof(unsigned long long) * nB) != hipSuccess ||
 	    poolAlloc(c->device, &dCursor, sizeof(unsigned int) * nB) != hipSuccess ||
 	    poolAlloc(c->device, &dBlockCnt, sizeof(unsigned int) * nB * grid) != hipSuccess ||
@@ -1700,7 +1700,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	pl.tileOff = dOff;
 	pl.err = dErr;
 	pl.ray = q->ray;
-	e = launchRayPrep(a, q->ray, c->stream);
+	e = launchRayPrep(a, q->ray, dErr, c->stream);
 	if (e == hipSuccess)
 		e = launchBin(0, a, T, pl, grid, c->stream);
 	std::vector<unsigned long long> cnt(nB);

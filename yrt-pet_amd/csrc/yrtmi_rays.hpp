@@ -328,17 +328,17 @@ __device__ __forceinline__ bool sidSetup(const DImage& P, float3 p1, float3 p2,
 }
 
 // The part of an FP32 set-up (sidSetup<TOF, false>) that a walk re-entered
-// at a tile record needs beyond the ray's end points, in two float4 (a
-// plan's ray table): the per-axis reciprocals, the exit alpha, the length
-// and the TOF constants.  sidLoad rebuilds the SidRay from the end points
-// and them: every field sidRestart and sidWalk read equals the set-up's
-// (the planes are recomputed by sidRestart, with the set-up's own
-// expression in the FP32 set-up, so kx/ky/kz are set to never match and
-// every non-flat axis is recomputed).
+// at a tile record and the plan's tile cut need beyond the ray's end points,
+// in two float4 (a plan's ray table): the per-axis reciprocals, the entry
+// and exit alphas and the TOF constants.  sidLoad rebuilds the SidRay from
+// the end points and them: every field sidRestart, sidWalk and sidPieces
+// read equals the set-up's (the planes are recomputed by sidRestart, with
+// the set-up's own expression in the FP32 set-up, so kx/ky/kz are set to
+// never match and every non-flat axis is recomputed).
 __device__ __forceinline__ void sidStore(float4* e, const SidRay& r)
 {
 	e[0] = make_float4(r.invx, r.invy, r.invz, r.amax);
-	e[1] = make_float4(r.dnorm, r.tA, r.tB, r.ws);
+	e[1] = make_float4(r.a_cur, r.tA, r.tB, r.ws);
 }
 
 __device__ __forceinline__ void sidLoad(float3 p1, float3 p2, const float4& s0,
@@ -351,10 +351,11 @@ __device__ __forceinline__ void sidLoad(float3 p1, float3 p2, const float4& s0,
 	r.invy = s0.y;
 	r.invz = s0.z;
 	r.amax = s0.w;
-	r.dnorm = s1.x;
+	r.a_cur = s1.x;
 	r.tA = s1.y;
 	r.tB = s1.z;
 	r.ws = s1.w;
+	r.dnorm = 0.f;
 	r.dirx = (r.invx >= 0.0f) ? 1 : -1;
 	r.diry = (r.invy >= 0.0f) ? 1 : -1;
 	r.dirz = (r.invz >= 0.0f) ? 1 : -1;
@@ -363,7 +364,6 @@ __device__ __forceinline__ void sidLoad(float3 p1, float3 p2, const float4& s0,
 	r.azn = FMAX;
 	r.xc = r.yc = r.zc = 0.f;
 	r.kx = r.ky = r.kz = -0x40000000;
-	r.a_cur = 0.f;
 	r.x1d = r.y1d = r.z1d = r.ddx = r.ddy = r.ddz = 0.0;
 }
 
@@ -479,101 +479,108 @@ __device__ __forceinline__ bool sidPlaneShift(const DImage& P, const SidRay& r, 
 // A tile is left at the nearest of its three far faces; an axis whose face
 // lies further has crossed the planes at or before that alpha (the walk's
 // rule: planes at one alpha advance together), found from the ray's position
-// there and corrected by the planes' own alphas, so the voxel entered is the
-// one whose far faces all lie ahead.  Planes take sidRestart's expression,
-// start + k dir v: a record's re-entered walk starts on the very planes its
-// piece was cut at.  The walk accumulates them, the same on voxel sizes that
-// are short binary fractions and within an ulp otherwise.
+// there and corrected by the alphas of the two planes around it, so the voxel
+// entered is the one whose far faces all lie ahead.  (The position is good to
+// 1e-6 of the image in voxels: one plane either way, but for voxels below a
+// millionth of the scanner, `coarse`, which search on.)  Planes take
+// sidRestart's expression, start + k dir v: a record's re-entered walk starts
+// on the very planes its piece was cut at.  The walk accumulates them, the
+// same on voxel sizes that are short binary fractions and within an ulp
+// otherwise.  A flat axis (origin -FMAX, factor 1, as in sidWalk) has every
+// plane at FMAX.
 //
-// Some 6 crossings of ~100 instructions per ray replace the walk's ~130 to
-// 250 segments of ~40: a plan's count and fill passes, bound by the walk's
-// VALU issue before, took 9.5 and 16.0 ms and take 2.7 and 4.2 ms for the
+// Some 6 crossings per ray replace the walk's ~130 to 250 segments of ~40
+// instructions: a plan's count and fill passes, bound by the walk's VALU
+// issue before, took 9.5 and 16.0 ms and take 0.7 and 1.4 ms for the
 // 8.4 M LORs x 4 rays of a 64 x 512 scanner's histogram subset at 256 x 256 x
-// 128 (5 M TOF events x 4 rays: 7.3 and 11.3 -> 2.3 and 3.3 ms).
+// 128.
 template <class Fn>
 __device__ __forceinline__ void sidPieces(const DImage& P, const SidRay& r, int lx, int ly,
                                           int lz, int vx, int vy, int vz, int dx, int dy,
                                           int dz, Fn&& fn)
 {
 #pragma clang fp contract(off)
+	// plane numbers are kept as floats (exact: at most 1024 voxels an axis)
 	struct Axis
 	{
-		float start, v, rv, p, d, inv;
-		int dir, n, l, sh, k, vox;
-		bool flat;
-		__device__ float plane(int q) const
+		float start, sv, p, inv;  // plane q: (start + q sv - p) inv
+		float gs, g0;             // planes passed at alpha m: gs m + g0
+		float k, kt, kend;        // next plane, the tile's face, the image's
+		float dirf, off;          // voxel whose far face is plane q: dirf q + off
+		float T;
+		__device__ __forceinline__ float plane(float q) const
 		{
-			const float c = start + (float)(q * dir) * v;
+			const float c = start + q * sv;
 			return (c - p) * inv;
 		}
-		// the plane at the tile's far face, and the voxel whose far face is
-		// plane q
-		__device__ int face() const
+		__device__ __forceinline__ int voxel(float q) const { return (int)(q * dirf + off); }
+		// the first plane after alpha m, from plane k on (at: the alpha of
+		// the tile's face, which is passed if not after m: every round of
+		// the loop leaves a tile, whatever the numbers)
+		__device__ __forceinline__ float after(float m, float at, bool coarse) const
 		{
-			const int t = vox >> l;
-			return (dir > 0 ? min((t + 1) << l, n) : n - (t << l)) + sh;
-		}
-		__device__ int voxelOf(int q) const { return dir > 0 ? q - 1 - sh : n - q + sh; }
-		// the first plane after alpha m, from plane k on (kt: the far face's
-		// plane, at its alpha)
-		__device__ int after(float m, int kt, float at) const
-		{
-			if (flat)
-				return k;
-			int q;
-			if (at <= m)
-				q = kt + 1;
-			else
+			float q = fminf(fmaxf(floorf(fmaf(m, gs, g0)) + 1.f, k), kt + 1.f);
+			const float lo = plane(q - 1.f), hi = plane(q);
+			q += (hi <= m) ? 1.f : ((lo > m && q > k) ? -1.f : 0.f);
+			if (coarse)
 			{
-				const float g = (float)dir * (p + m * d - start) * rv;
-				q = max(k, min((int)floorf(fminf(fmaxf(g, -1.f), 2048.f)) + 1, kt));
-				while (q > k && plane(q - 1) > m)
-					q--;
+				while (q > k && plane(q - 1.f) > m)
+					q -= 1.f;
+				while (q < kend + 16.f && plane(q) <= m)
+					q += 1.f;
 			}
-			while (q < n + 16 && plane(q) <= m)
-				q++;
-			return q;
+			return (at <= m) ? fmaxf(q, kt + 1.f) : q;
 		}
 	};
 	const float FMAX = 3.402823466e+38f;
-	auto axis = [](float len, float v, float p1, float p2, float inv, int dir, int n, int l,
-	               int sh, int vox) {
+	auto axis = [&](float len, float v, float p1, float p2, float inv, int dir, int n, int l,
+	                int sh, int vox) {
 		Axis a;
+		const bool flat = p1 == p2;
+		const float rv = (dir > 0) ? 1.0f / v : -1.0f / v;
 		a.start = (dir > 0) ? -len * 0.5f : len * 0.5f;
-		a.v = v;
-		a.rv = 1.0f / v;
-		a.p = p1;
-		a.d = p2 - p1;
-		a.inv = inv;
-		a.dir = dir;
-		a.n = n;
-		a.l = l;
-		a.sh = sh;
-		a.k = ((dir > 0) ? vox + 1 : n - vox) + sh;
-		a.vox = vox;
-		a.flat = p1 == p2;
+		a.sv = (float)dir * v;
+		a.p = flat ? -FMAX : p1;
+		a.inv = flat ? 1.f : inv;
+		a.k = (float)(((dir > 0) ? vox + 1 : n - vox) + sh);
+		a.gs = (p2 - p1) * rv;
+		a.g0 = flat ? a.k - 1.f : (p1 - a.start) * rv;
+		const int t = vox >> l;
+		a.kt = (float)((dir > 0 ? min((t + 1) << l, n) : n - (t << l)) + sh);
+		a.kend = (float)(n + sh);
+		a.dirf = (float)dir;
+		a.off = (float)(dir > 0 ? -1 - sh : n + sh);
+		a.T = (float)(1 << l);
 		return a;
 	};
+	if ((unsigned)vx >= (unsigned)P.nx || (unsigned)vy >= (unsigned)P.ny ||
+	    (unsigned)vz >= (unsigned)P.nz)
+		return;
 	Axis X = axis(P.lx, P.vx, r.p1.x, r.p2.x, r.invx, r.dirx, P.nx, lx, dx, vx);
 	Axis Y = axis(P.ly, P.vy, r.p1.y, r.p2.y, r.invy, r.diry, P.ny, ly, dy, vy);
 	Axis Z = axis(P.lz, P.vz, r.p1.z, r.p2.z, r.invz, r.dirz, P.nz, lz, dz, vz);
+	const bool coarse =
+	    fmaxf(fmaxf(fabsf(X.gs), fabsf((r.p1.x - X.start) / P.vx)),
+	          fmaxf(fmaxf(fabsf(Y.gs), fabsf((r.p1.y - Y.start) / P.vy)),
+	                fmaxf(fabsf(Z.gs), fabsf((r.p1.z - Z.start) / P.vz)))) > 1e6f;
 	float a0 = r.a_cur;
-	while ((unsigned)X.vox < (unsigned)P.nx && (unsigned)Y.vox < (unsigned)P.ny &&
-	       (unsigned)Z.vox < (unsigned)P.nz)
+	for (;;)
 	{
-		const int fx = X.face(), fy = Y.face(), fz = Z.face();
-		const float ax = X.flat ? FMAX : X.plane(fx), ay = Y.flat ? FMAX : Y.plane(fy),
-		            az = Z.flat ? FMAX : Z.plane(fz);
+		const float ax = X.plane(X.kt), ay = Y.plane(Y.kt), az = Z.plane(Z.kt);
 		const float face = fminf(ax, fminf(ay, az));
 		const bool last = !(face < r.amax);
 		const float m = last ? r.amax : face;
-		const int qx = X.after(m, fx, ax), qy = Y.after(m, fy, ay), qz = Z.after(m, fz, az);
-		fn(a0, X.vox, Y.vox, Z.vox, (qx - X.k) + (qy - Y.k) + (qz - Z.k) + (last ? 1 : 0));
-		if (last)
+		const float qx = X.after(m, ax, coarse), qy = Y.after(m, ay, coarse),
+		            qz = Z.after(m, az, coarse);
+		fn(a0, vx, vy, vz, (int)((qx - X.k) + (qy - Y.k) + (qz - Z.k)) + (last ? 1 : 0));
+		if (last || qx > X.kend || qy > Y.kend || qz > Z.kend)
 			return;
-		X.vox = X.flat ? X.vox : X.voxelOf(qx);
-		Y.vox = Y.flat ? Y.vox : Y.voxelOf(qy);
-		Z.vox = Z.flat ? Z.vox : Z.voxelOf(qz);
+		vx = X.voxel(qx);
+		vy = Y.voxel(qy);
+		vz = Z.voxel(qz);
+		X.kt = (qx > X.kt) ? fminf(X.kt + X.T, X.kend) : X.kt;
+		Y.kt = (qy > Y.kt) ? fminf(Y.kt + Y.T, Y.kend) : Y.kt;
+		Z.kt = (qz > Z.kt) ? fminf(Z.kt + Z.T, Z.kend) : Z.kt;
 		X.k = qx;
 		Y.k = qy;
 		Z.k = qz;

@@ -50,8 +50,9 @@ __device__ __forceinline__ int tileOf(const DTiles& T, int f, int vx, int vy,
 // the LOR resolved once (detector pair or histogram bin, LUT, motion,
 // frame), the multi-ray line and the image offset.  Skipped LORs get frame -1.
 // Distance-driven (DD): the LOR's footprint set-up (ddSetup, ddStore).
+// A plane shift beyond the record's range sets *err (the ray is skipped).
 template <bool DD, bool TOF, bool S64>
-__global__ void __launch_bounds__(256) kRayPrep(KArgs a, float4* __restrict__ tab)
+__global__ void __launch_bounds__(256) kRayPrep(KArgs a, float4* __restrict__ tab, int* err)
 {
 	const int R = a.pr.numRays;
 	const int64_t total = a.L.n * (int64_t)R;
@@ -76,28 +77,38 @@ __global__ void __launch_bounds__(256) kRayPrep(KArgs a, float4* __restrict__ ta
 			continue;
 		}
 		constexpr int V = rayTabVec(S64);
-		const float3 z = make_float3(0.f, 0.f, 0.f);
-		if (l.frame < 0)
+		float3 q1 = make_float3(0.f, 0.f, 0.f), q2 = q1;
+		if (l.frame >= 0)
 		{
-			rayEntry(tab, V, (uint32_t)t, z, z, 0.f, -1);
-			if (!S64)
-				tab[V * (uint64_t)t + 2] = tab[V * (uint64_t)t + 3] = make_float4(0.f, 0.f, 0.f, 0.f);
+			rayLine(a.pr, l, r, q1, q2);
+			q1 = make_float3(q1.x - a.im.ox, q1.y - a.im.oy, q1.z - a.im.oz);
+			q2 = make_float3(q2.x - a.im.ox, q2.y - a.im.oy, q2.z - a.im.oz);
+		}
+		if (S64)
+		{
+			rayEntry(tab, V, (uint32_t)t, q1, q2, l.frame >= 0 ? l.tof : 0.f,
+			         l.frame >= 0 ? l.frame : -1);
 			continue;
 		}
-		float3 q1, q2;
-		rayLine(a.pr, l, r, q1, q2);
-		q1 = make_float3(q1.x - a.im.ox, q1.y - a.im.oy, q1.z - a.im.oz);
-		q2 = make_float3(q2.x - a.im.ox, q2.y - a.im.oy, q2.z - a.im.oz);
-		rayEntry(tab, V, (uint32_t)t, q1, q2, l.tof, l.frame);
-		if (!S64)
+		// the ray's FP32 set-up and its first voxel
+		SidRay sr;
+		int vx = 0, vy = 0, vz = 0, dx = 0, dy = 0, dz = 0;
+		bool ok = l.frame >= 0 && sidSetup<TOF, false>(a.im, q1, q2, a.pr.tof, l.tof, sr) &&
+		          sidFirst<false>(a.im, sr, vx, vy, vz, dx, dy, dz) &&
+		          (unsigned)vx < (unsigned)a.im.nx && (unsigned)vy < (unsigned)a.im.ny &&
+		          (unsigned)vz < (unsigned)a.im.nz;
+		if (ok && (abs(dx) > kMaxShift || abs(dy) > kMaxShift || abs(dz) > kMaxShift))
 		{
-			// the ray's FP32 set-up, for walks re-entered at a tile record
-			SidRay sr;
-			if (sidSetup<TOF, false>(a.im, q1, q2, a.pr.tof, l.tof, sr))
-				sidStore(tab + V * (uint64_t)t + 2, sr);
-			else
-				tab[V * (uint64_t)t + 2] = tab[V * (uint64_t)t + 3] = make_float4(0.f, 0.f, 0.f, 0.f);
+			atomicOr(err, 2);
+			ok = false;
 		}
+		rayEntry(tab, V, (uint32_t)t, q1, q2,
+		         __uint_as_float((uint32_t)vx | ((uint32_t)vy << 10) | ((uint32_t)vz << 20)),
+		         (int32_t)(ok ? rayWord(l.frame, dx, dy, dz) : kNoFrame));
+		if (ok)
+			sidStore(tab + V * (uint64_t)t + 2, sr);
+		else
+			tab[V * (uint64_t)t + 2] = tab[V * (uint64_t)t + 3] = make_float4(0.f, 0.f, 0.f, 0.f);
 	}
 }
 
@@ -113,32 +124,42 @@ __device__ __forceinline__ void binRay(const DImage& im, const DTof& tof, const 
 {
 	constexpr int V = rayTabVec(S64);
 	const float4 A = tab[V * (uint64_t)t], Bq = tab[V * (uint64_t)t + 1];
+	const float3 q1 = make_float3(A.x, A.y, A.z), q2 = make_float3(A.w, Bq.x, Bq.y);
+	SidRay s;
+	if constexpr (!S64)
+	{
+		const float4 s0 = tab[V * (uint64_t)t + 2], s1 = tab[V * (uint64_t)t + 3];
+		const uint32_t w = __float_as_uint(Bq.w), fv = __float_as_uint(Bq.z);
+		const int frame = (int)(w & 0xffffu);
+		if (frame == (int)kNoFrame)
+			return;
+		sidLoad(q1, q2, s0, s1, s);
+		// the entry word's shift bits lie one below the table word's
+		const uint32_t sh = (w >> 1) & 0x07ff8000u;
+		uint32_t first = 0x80000000u;
+		sidPieces(im, s, T.lx, T.ly, T.lz, (int)(fv & 1023u), (int)((fv >> 10) & 1023u),
+		          (int)((fv >> 20) & 1023u), (int)((w >> 16) & 15u) - 8,
+		          (int)((w >> 20) & 15u) - 8, (int)((w >> 24) & 15u) - 8,
+		          [&](float a0, int vx, int vy, int vz, int segs) {
+			          onRecord(tileOf(T, frame, vx, vy, vz), a0,
+			                   (uint32_t)(vx & (T.tx - 1)) | ((uint32_t)(vy & (T.ty - 1)) << 5) |
+			                       ((uint32_t)(vz & (T.tz - 1)) << 10) | sh | first,
+			                   segs);
+			          first = 0u;
+		          });
+		return;
+	}
 	const int frame = __float_as_int(Bq.w);
 	if (frame < 0)
 		return;
-	const float3 q1 = make_float3(A.x, A.y, A.z), q2 = make_float3(A.w, Bq.x, Bq.y);
-	SidRay s;
 	if (!sidSetup<TOF, S64>(im, q1, q2, tof, Bq.z, s))
 		return;
-	int ex, ey, ez, dx, dy, dz;
-	if (!sidFirst<S64>(im, s, ex, ey, ez, dx, dy, dz))
+	int dx, dy, dz;
+	if (!sidPlaneShift<S64>(im, s, dx, dy, dz))
 		return;
 	if (abs(dx) > kMaxShift || abs(dy) > kMaxShift || abs(dz) > kMaxShift)
 	{
 		atomicOr(err, 2);
-		return;
-	}
-	if constexpr (!S64)
-	{
-		bool first = true;
-		sidPieces(im, s, T.lx, T.ly, T.lz, ex, ey, ez, dx, dy, dz,
-		          [&](float a0, int vx, int vy, int vz, int segs) {
-			          onRecord(tileOf(T, frame, vx, vy, vz), a0,
-			                   packEntry(vx & (T.tx - 1), vy & (T.ty - 1), vz & (T.tz - 1), dx,
-			                             dy, dz, first),
-			                   segs);
-			          first = false;
-		          });
 		return;
 	}
 	int last = -1, start = 0, nseg = 0;
@@ -238,11 +259,12 @@ __device__ __forceinline__ void binRayDD(const DImage& im, const DProj& pr, cons
 	}
 }
 
+// (the loop's bound is uniform: a plan of few classes compares few cuts)
 __device__ __forceinline__ int lengthClass(const DPlan& pl, int segs)
 {
 	int c = 0;
-	for (int k = 0; k < kMaxClasses - 1; k++)
-		c += (k < pl.C - 1 && segs >= pl.cut[k]) ? 1 : 0;
+	for (int k = 0; k < pl.C - 1; k++)
+		c += (segs >= pl.cut[k]) ? 1 : 0;
 	return c;
 }
 
@@ -258,7 +280,7 @@ __device__ __forceinline__ int lengthClass(const DPlan& pl, int segs)
 // alpha.
 // LDS: cnt[nB] ints, then (PASS 1) base[nB] 32-bit record indices.
 template <bool DD, bool TOF, bool S64, int PASS>
-__global__ void __launch_bounds__(256) kBin(DImage im, DProj pr, int64_t nRays, DTiles T,
+__global__ void __launch_bounds__(kBinThreads) kBin(DImage im, DProj pr, int64_t nRays, DTiles T,
                                             DPlan pl)
 {
 	extern __shared__ int sm[];
@@ -583,8 +605,8 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 		uint32_t key, pv;
 		float al;
 	};
-	// Siddon: the ray's end points, TOF value and frame (two float4), with
-	// the FP32 set-up two more (sidStore); DD: kDDVec (ddStore)
+	// Siddon: the ray's end points and frame (two float4), with the FP32
+	// set-up two more (sidStore); DD: kDDVec (ddStore)
 	constexpr int NE = DD ? kDDVec : rayTabVec(S64);
 	struct Ray
 	{
@@ -628,7 +650,7 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 			return;
 		{
 			const float4 qa = q.e[0], qb = q.e[1];
-			if (__float_as_int(qb.w) != f)
+			if ((S64 ? __float_as_int(qb.w) : (int)(__float_as_uint(qb.w) & 0xffffu)) != f)
 				return;
 			const float3 q1 = make_float3(qa.x, qa.y, qa.z), q2 = make_float3(qa.w, qb.x, qb.y);
 			// v / R: for R a power of two the product with 1/R is the same
@@ -1071,14 +1093,14 @@ static hipError_t binT(int pass, const KArgs& a, const DTiles& T,
 	const int nB = T.nTiles * pl.C;
 	const int64_t nRays = a.L.n * (int64_t)pl.R;
 	if (pass == 0)
-		kBin<DD, TOF, S64, 0><<<grid, 256, (size_t)nB * sizeof(int), st>>>(a.im, a.pr, nRays,
+		kBin<DD, TOF, S64, 0><<<grid, kBinThreads, (size_t)nB * sizeof(int), st>>>(a.im, a.pr, nRays,
 		                                                                    T, pl);
 	else
-		kBin<DD, TOF, S64, 1><<<grid, 256, binLdsBytes(nB), st>>>(a.im, a.pr, nRays, T, pl);
+		kBin<DD, TOF, S64, 1><<<grid, kBinThreads, binLdsBytes(nB), st>>>(a.im, a.pr, nRays, T, pl);
 	return hipGetLastError();
 }
 
-hipError_t launchRayPrep(const KArgs& a, float4* tab, hipStream_t st)
+hipError_t launchRayPrep(const KArgs& a, float4* tab, int* err, hipStream_t st)
 {
 	const int64_t total = a.L.n * (int64_t)a.pr.numRays;
 	if (total == 0)
@@ -1090,25 +1112,25 @@ hipError_t launchRayPrep(const KArgs& a, float4* tab, hipStream_t st)
 	if (a.pr.type != 1)
 	{
 		if (a.pr.setup64)
-			kRayPrep<false, false, true><<<g, 256, 0, st>>>(a, tab);
+			kRayPrep<false, false, true><<<g, 256, 0, st>>>(a, tab, err);
 		else if (a.pr.useTof)
-			kRayPrep<false, true, false><<<g, 256, 0, st>>>(a, tab);
+			kRayPrep<false, true, false><<<g, 256, 0, st>>>(a, tab, err);
 		else
-			kRayPrep<false, false, false><<<g, 256, 0, st>>>(a, tab);
+			kRayPrep<false, false, false><<<g, 256, 0, st>>>(a, tab, err);
 	}
 	else if (a.pr.useTof)
 	{
 		if (a.pr.setup64)
-			kRayPrep<true, true, true><<<g, 256, 0, st>>>(a, tab);
+			kRayPrep<true, true, true><<<g, 256, 0, st>>>(a, tab, err);
 		else
-			kRayPrep<true, true, false><<<g, 256, 0, st>>>(a, tab);
+			kRayPrep<true, true, false><<<g, 256, 0, st>>>(a, tab, err);
 	}
 	else
 	{
 		if (a.pr.setup64)
-			kRayPrep<true, false, true><<<g, 256, 0, st>>>(a, tab);
+			kRayPrep<true, false, true><<<g, 256, 0, st>>>(a, tab, err);
 		else
-			kRayPrep<true, false, false><<<g, 256, 0, st>>>(a, tab);
+			kRayPrep<true, false, false><<<g, 256, 0, st>>>(a, tab, err);
 	}
 	return hipGetLastError();
 }

@@ -28,6 +28,10 @@ __host__ __device__ constexpr int tileThreads(int shape)
 // kMaxBins / 2.
 constexpr int kMaxBins = 16384;
 constexpr int kMaxClasses = 16;
+// Threads of a binning workgroup, which share its LDS counters (64 KB in the
+// fill pass with 8192 bins: two workgroups per CU, 16 waves of 512 threads).
+// Fill pass of 8.4 M LORs x 4 rays: 256 threads 4.2 ms, 512 2.9, 1024 4.7.
+constexpr int kBinThreads = 512;
 
 // Entry record of a ray in a tile: voxel within the tile (5 bits per axis),
 // the ray's plane shift per axis (sidPlaneShift, 4 bits each, offset 8) and
@@ -118,21 +122,31 @@ struct DPlan
 
 // Ray table of a Siddon plan, rayTabVec(S64) float4 per (LOR, ray) t = lor *
 // R + ray.  The first two: the ray's end points after multi-ray offsets,
-// motion and the image offset (q1, q2, exactly as the walk sets it up), its
-// TOF value and its frame (-1: skipped); the backprojection reads them
-// instead of resolving the LOR.  With the FP32 setup two more hold the
-// ray's set-up (sidStore), from which a walk re-entered at a tile record
-// starts without redoing it.
+// motion and the image offset (q1, q2, exactly as the walk sets it up) and
+// two words.  FP64 set-up: its TOF value and its frame (-1: skipped).  FP32
+// set-up: the walk's first voxel (10 bits per axis) and its frame with the
+// plane shifts (rayWord); two more float4 hold the ray's set-up (sidStore),
+// from which it is cut into its tiles (sidPieces) and walks re-entered at a
+// tile record start without redoing it.
 constexpr int rayTabVec(bool S64)
 {
 	return S64 ? 2 : 4;
 }
 
 __device__ __forceinline__ void rayEntry(float4* tab, int vec, uint32_t t, float3 q1, float3 q2,
-                                         float tof, int32_t frame)
+                                         float w0, int32_t w1)
 {
 	tab[vec * (uint64_t)t] = make_float4(q1.x, q1.y, q1.z, q2.x);
-	tab[vec * (uint64_t)t + 1] = make_float4(q2.y, q2.z, tof, __int_as_float(frame));
+	tab[vec * (uint64_t)t + 1] = make_float4(q2.y, q2.z, w0, __int_as_float(w1));
+}
+
+// Frame (below 65535: a plan has fewer tiles) and plane shifts of an FP32
+// entry; a ray that is skipped, or misses the image, has the frame 0xffff.
+constexpr uint32_t kNoFrame = 0xffffu;
+__device__ __forceinline__ uint32_t rayWord(int frame, int dx, int dy, int dz)
+{
+	return (uint32_t)frame | ((uint32_t)(dx + 8) << 16) | ((uint32_t)(dy + 8) << 20) |
+	       ((uint32_t)(dz + 8) << 24);
 }
 
 // Plan in use.  queue != null: persistent launch, workgroups take chunks
@@ -158,7 +172,8 @@ inline size_t binLdsBytes(int nB)
 	return (size_t)nB * (sizeof(int) + sizeof(uint32_t));
 }
 // The plan's ray table for a.L (before the binning passes).
-hipError_t launchRayPrep(const KArgs& a, float4* tab, hipStream_t st);
+// *err |= 2 for a ray whose plane shift is out of a record's range.
+hipError_t launchRayPrep(const KArgs& a, float4* tab, int* err, hipStream_t st);
 // pass 0: count; pass 1: fill (same grid in both).
 hipError_t launchBin(int pass, const KArgs& a, const DTiles& T, const DPlan& pl,
                      int grid, hipStream_t st);
