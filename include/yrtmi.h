@@ -156,7 +156,7 @@ int yrtmi_ctx_own_stream(yrtmi_ctx* ctx, void** stream);
  * Calls that allocate, copy or synchronise (plan_create, count_segments,
  * histo_subset_nonzero, lor_order, copy, device_alloc/free, lut / histo /
  * motion uploads, and a first per-XCD backprojection that would allocate its
- * partial images) fail with YRTMI_ESTATE while recording. */
+ * partial images or scratch) fail with YRTMI_ESTATE while recording. */
 typedef struct yrtmi_graph yrtmi_graph;
 int yrtmi_graph_begin(yrtmi_ctx* ctx);
 int yrtmi_graph_end(yrtmi_ctx* ctx, yrtmi_graph** out);
@@ -199,10 +199,14 @@ int yrtmi_proj_destroy(yrtmi_proj* p);
  * rays), threads per block, and blocks (0 = sized from the event count). */
 int yrtmi_proj_set_launch(yrtmi_proj* p, int lanes_per_event,
                           int block_size, int grid_blocks);
-/* How backprojections accumulate.  YRTMI_ACCUM_XCD (default): each XCD adds
- * into its own private copy of the target image (chosen by the hardware XCC
- * id), and the copies are folded into the target by one streaming pass after
- * the kernel; the context keeps the copies (n_xcc x image size) between
+/* How backprojections accumulate.  YRTMI_ACCUM_XCD (default): calls of many
+ * rays (32768 to 131072 and more, by projector and image size) are binned by
+ * image tiles on the device, batch by batch, and summed in LDS as a tile
+ * plan's; the context keeps their scratch (at most 1 GiB and, for EM
+ * subsets, a copy of the image) between calls.  In smaller calls each XCD
+ * adds into its own private copy of the target image (chosen by the hardware
+ * XCC id), and the copies are folded into the target by one streaming pass
+ * after the kernel; the context keeps the copies (n_xcc x image size) between
  * calls.  YRTMI_ACCUM_DIRECT: FP32 atomics straight into the target (no
  * extra memory).  Both are the reference's atomicAdd accumulation
  * (SiddonKernels.cuh:426-428) up to summation order. */

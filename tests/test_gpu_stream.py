@@ -1,0 +1,156 @@
+"""Backprojections without a plan on the GPU, of enough rays to be binned by
+tiles on the device: against the same calls with direct accumulation (global
+atomics, never binned).
+
+Bar 1e-5 relative L2, the projector tests' (dyadic voxels: the tile sums are
+exact, the direct ones sum some 10^4 FP32 terms a voxel, whose rounding grows
+as the square root: 100 x 6e-8).  Below and above the
+rule's thresholds; one, two and many batches; every LOR source; a batch with more records
+than there is room for (it takes the direct kernel)."""
+import numpy as np
+import pytest
+import torch
+
+import yrtmi
+from helpers import rel_l2
+from yrtmi import synth
+
+pytestmark = pytest.mark.gpu
+
+SC = ("t", 96.0, 4.0, 4.0, 10.0, 180.0, 128, 24)
+
+
+def setup(im, n, proj="Siddon", rays=1, tof=None, psf=False, fp64=False, frames=0, seed=3,
+          sc=SC, gpu=None, motion=0):
+    sc = yrtmi.Scanner(*sc)
+    rng = np.random.default_rng(seed)
+    ev = synth.random_events(sc, n, rng, tof_fwhm_ps=tof)
+    t = lambda a, d: torch.from_numpy(np.ascontiguousarray(a).astype(d)).to(gpu)
+    ctx = yrtmi.Context(sc)
+    mot = None
+    if motion:
+        ctx.upload_motion(synth.rigid_transforms(rng, motion))
+        mot = t(rng.integers(0, motion + 1, n), np.uint8)  # one index past the last: skipped
+    fr = t(rng.integers(-1, frames, n), np.int32) if frames else None
+    L = yrtmi.LorSet.pairs(t(ev["d1"], np.int32), t(ev["d2"], np.int32),
+                           tof=t(ev["tof"], np.float32) if tof else None, frame=fr,
+                           motion_frame=mot)
+    pp = yrtmi.ProjectorParams(sc, projectorType=proj, numRays=rays, setupFP64=fp64)
+    if tof:
+        pp.addTOF(tof, 5)
+    if psf:
+        k, pp.psf_s_step, pp.psf_k_spacing = synth.gaussian_psf_row(2.0, num_s=2, s_step=60.0)
+        pp.psf_kernels = k * np.array([[1.0], [1.1]], np.float32)
+    return ctx, ctx.projector(pp), L, rng
+
+
+def pair(gpu, im, proj, call):
+    """call(img) with per-XCD accumulation (binned) and with direct atomics,
+    each into an image that already holds something."""
+    out = []
+    for xcd in (True, False):
+        proj.set_accumulation(xcd)
+        img = torch.full(im.shape, 2.0 ** -12, device=gpu)
+        call(img)
+        torch.cuda.synchronize()
+        out.append((img - 2.0 ** -12).cpu().numpy())
+    r = rel_l2(out[0], out[1])
+    print(f"binned vs direct rel L2 {r:.2e}, sum {out[1].sum():.4e}", flush=True)
+    assert np.abs(out[1]).sum() > 0
+    assert r <= 1e-5
+    return out
+
+
+CASES = [
+    # name, image, n, kwargs
+    ("below", (64, 60, 30, 4.0, 4.5, 2.0), 131_071, dict()),
+    ("above", (64, 60, 30, 4.0, 4.5, 2.0), 131_073, dict()),
+    ("above_large_image", (160, 160, 96, 1.5, 1.5, 1.0), 32_769, dict()),
+    ("rays4_tof", (64, 60, 30, 4.0, 4.5, 2.0), 60_001, dict(rays=4, tof=250.0)),
+    ("rays3_frames", (33, 65, 17, 4.0, 4.0, 4.0), 50_000, dict(rays=3, frames=3)),
+    ("motion_tof", (64, 64, 32, 4.0, 4.0, 2.0), 140_000, dict(tof=300.0, motion=4)),
+    ("fp64", (64, 60, 30, 4.0, 4.5, 2.0), 70_000, dict(rays=2, tof=250.0, fp64=True)),
+    ("dd", (64, 60, 30, 4.0, 4.5, 2.0), 70_000, dict(proj="DD")),
+    ("dd_tof_psf", (61, 60, 31, 4.0, 4.5, 2.0), 70_000, dict(proj="DD", tof=300.0, psf=True)),
+    ("two_batches", (64, 64, 32, 4.0, 4.0, 2.0), 700_000, dict(rays=16, tof=250.0)),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_back_and_em(gpu, case):
+    _, imd, n, kw = case
+    im = yrtmi.ImageParams(*imd, nt=max(1, kw.get("frames", 0)))
+    ctx, p, L, rng = setup(im, n, gpu=gpu, **kw)
+    g = torch.Generator(gpu).manual_seed(5)
+    v = torch.rand(n, device=gpu, generator=g) - 0.3
+    v[::17] = 0.0
+    pair(gpu, im, p, lambda u: ctx.back(p, im, u, L, v))
+    x = 0.5 + torch.rand(im.shape, device=gpu, generator=g)
+    c = {k: 0.2 + torch.rand(n, device=gpu, generator=g)
+         for k in ("meas", "sens", "att", "randoms", "scatter")}
+    c["meas"][::5] = 0.0
+    pair(gpu, im, p, lambda u: ctx.em_subset(p, im, x, u, L, global_scale=1.5, **c))
+
+
+@pytest.mark.parametrize("dd", [False, True])
+@pytest.mark.parametrize("att", [False, True])
+def test_sensitivity_of_histogram_subset(gpu, dd, att):
+    im = yrtmi.ImageParams(48, 50, 20, 4.0, 4.0, 4.0)
+    ctx, p, _, _ = setup(im, 10, proj="DD" if dd else "Siddon", rays=1 if dd else 2, gpu=gpu)
+    L = yrtmi.LorSet.histo_subset(ctx, 5, 3)
+    g = torch.Generator(gpu).manual_seed(5)
+    s = torch.rand(L.n, device=gpu, generator=g)
+    mu = 0.1 * torch.rand(im.shape, device=gpu, generator=g)
+    pair(gpu, im, p, lambda u: ctx.sensitivity(p, im, u, L, att_im=im if att else None,
+                                               att_img=mu if att else None, sens=s))
+    bins = torch.arange(0, 200_000, 3, device=gpu, dtype=torch.int32)
+    B = yrtmi.LorSet.bins_(bins)
+    v = torch.rand(B.n, device=gpu, generator=g)
+    pair(gpu, im, p, lambda u: ctx.back(p, im, u, B, v))
+
+
+def test_batch_without_room_takes_the_direct_kernel(gpu):
+    """Crystals 240 voxels high over one column of 64 tiles: some 30 records
+    for each LOR that meets the image, where there is room for 8 per LOR."""
+    im = yrtmi.ImageParams(32, 32, 512, 4.0, 4.0, 0.25)
+    ctx, p, L, _ = setup(im, 70_000, proj="DD", gpu=gpu,
+                         sc=("t", 128.0, 60.0, 4.0, 10.0, 180.0, 128, 2))
+    v = torch.rand(L.n, device=gpu, generator=torch.Generator(gpu).manual_seed(1))
+    plan = ctx.plan(p, im, L, tile_shape=3)
+    assert plan.info()["records"] > 8 * L.n
+    pair(gpu, im, p, lambda u: ctx.back(p, im, u, L, v))
+
+
+def test_recorded_and_on_other_streams(gpu):
+    """Recorded after one eager call and replayed between other calls that
+    use (and grow) the same scratch, and on streams in turn."""
+    im = yrtmi.ImageParams(64, 60, 30, 4.0, 4.5, 2.0)
+    ctx, p, L, _ = setup(im, 70_000, rays=2, tof=250.0, gpu=gpu)
+    big = setup(im, 300_000, rays=2, tof=250.0, gpu=gpu, seed=9)[2]
+    g = torch.Generator(gpu).manual_seed(5)
+    v, w = torch.rand(L.n, device=gpu, generator=g), torch.rand(big.n, device=gpu, generator=g)
+    ref, ref2 = (torch.zeros(im.shape, device=gpu) for _ in range(2))
+    p.set_accumulation(False)
+    ctx.back(p, im, ref, L, v)
+    ctx.back(p, im, ref2, big, w)
+    torch.cuda.synchronize()
+    p.set_accumulation(True)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    u, u2 = (torch.zeros(im.shape, device=gpu) for _ in range(2))
+    torch.cuda.synchronize()
+    ctx.set_stream(streams[0])
+    ctx.back(p, im, u, L, v)
+    with ctx.graph() as gr:
+        ctx.fill(u, 0.0)
+        ctx.back(p, im, u, L, v)
+    for k in range(4):
+        ctx.set_stream(streams[k % 2])
+        gr.launch()
+        ctx.set_stream(streams[(k + 1) % 2])
+        ctx.fill(u2, 0.0)
+        ctx.back(p, im, u2, big, w)  # the first grows the scratch
+        torch.cuda.synchronize()
+        a, b = rel_l2(u.cpu().numpy(), ref.cpu().numpy()), rel_l2(u2.cpu().numpy(),
+                                                                  ref2.cpu().numpy())
+        print(f"replay {k}: {a:.2e}, other call {b:.2e}", flush=True)
+        assert a <= 1e-5 and b <= 1e-5

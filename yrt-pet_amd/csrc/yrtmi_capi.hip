@@ -76,6 +76,15 @@ struct yrtmi_ctx
 	// bricked copy of the image the Siddon EM ratio projects, grown on demand
 	float* brick = nullptr;
 	int64_t brickCap = 0;
+	// scratch of the backprojections binned by tiles without a plan
+	// (streamBack), its last use, and whether a graph refers to it; grown
+	// scratch that a graph refers to stays until the context goes
+	void* ws = nullptr;
+	size_t wsBytes = 0;
+	hipEvent_t wsEvent = nullptr;
+	hipStream_t wsStream = nullptr;
+	bool wsUsed = false, wsCaptured = false;
+	std::vector<void*> wsRetired;
 	hipStream_t owned = nullptr;  // stream created by yrtmi_ctx_own_stream
 	bool capturing = false;       // between yrtmi_graph_begin and _end
 };
@@ -314,12 +323,290 @@ int brickImage(yrtmi_ctx* c, KArgs& a)
 	return YRTMI_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Backprojection through image tiles without a plan: the LORs are taken in
+// batches, each binned by tiles on the device (ray table, count, scan, fill,
+// as a plan's) and backprojected (kTileBack), with no wait by the host, in a
+// scratch buffer of the context.
+//
+// The direct kernels are bound by FP32 global atomics (21 G/s): a
+// backprojection of 1 M TOF LORs x 4 rays into 200 x 200 x 128 took 19.4 ms
+// and takes 1.4, 150 k DD TOF LORs into 95 x 97 x 47 took 5.6 and take 1.0,
+// an EM subset of 2 M corrected LORs into 181 x 173 x 109 took 35.3 and takes
+// 4.0 (of which its forward 1.6).  The binned path's fixed cost (nine
+// launches a batch, the scan, a pass over the touched tiles) is 70 to 100 us;
+// the direct one's is the fold of its partial images, 30 us at 96 x 96 x 48
+// and 90 us at 200 x 200 x 128.  The lines (streamMinRays) lie where the two
+// meet; direct / binned, us:
+//   Siddon, 96 x 96 x 48    65 k rays  back 70-86 / 83-86  EM  88-109 / 121-128
+//   Siddon, 200 x 200 x 128 16 k rays  back 86-126 / 81-106 EM 122-221 / 142-230
+//                           32 k rays  back 110-178 / 88-109 EM 146-274 / 148-232
+//   DD                      32 k LORs  back 404-993 / 388-863 EM 440-1245 / 574-1313
+//                           65 k LORs  back 518-1544 / 419-938 EM 650-1901 / 591-1386
+// ---------------------------------------------------------------------------
+constexpr size_t kStreamBytes = size_t(1) << 30;  // scratch per context
+constexpr int kStreamBinGroups = 1024;
+
+int64_t streamMinRays(const KArgs& a)
+{
+	if (a.pr.type == YRTMI_PROJ_DD)
+		return 65536;
+	return a.im.nvox * a.im.nt >= (int64_t(1) << 21) ? 32768 : 131072;
+}
+
+struct StreamShape
+{
+	DTiles T{};
+	int C = 1;           // length classes
+	int64_t nB = 0;      // bins
+	int words = 0;       // per record
+	int tabVec = 0;      // float4 per ray
+	int64_t recPer = 0;  // room for this many records per ray
+	int R = 1;
+	int persistent = 0;  // tile kernel workgroups
+	bool dd = false;
+	int64_t brick = 0;   // floats of the bricked image (EM, Siddon)
+	size_t fixedBytes() const
+	{
+		return sizeof(StreamState) + (size_t)nB * 20 + (size_t)kStreamBinGroups * nB * 4 +
+		       (size_t)(T.nTiles + 2048) * sizeof(TileChunk) + (size_t)brick * 4 + 16 * 256;
+	}
+	size_t lorBytes() const
+	{
+		return (size_t)R * ((size_t)tabVec * sizeof(float4) + (size_t)recPer * words * 4 + 1) + 4;
+	}
+};
+
+bool streamShape(yrtmi_ctx* c, const KArgs& a, bool em, StreamShape& s)
+{
+	if (a.im.nx > 1024 || a.im.ny > 1024 || a.im.nz > 1024)
+		return false;
+	s.dd = a.pr.type == YRTMI_PROJ_DD;
+	s.R = a.pr.numRays;
+	s.words = recWords(s.dd);
+	s.tabVec = s.dd ? kDDVec : rayTabVec(a.pr.setup64 != 0);
+	int cus = 256;
+	(void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
+	// the flat tiles suit mostly transaxial lines (two workgroups a CU); the
+	// thicker ones take twice the image
+	s.T = tilesOf(3, a.im.nx, a.im.ny, a.im.nz, a.im.nt);
+	s.persistent = 2 * cus;
+	if (s.T.nTiles == 0 || s.T.nTiles > 4096)
+	{
+		s.T = tilesOf(1, a.im.nx, a.im.ny, a.im.nz, a.im.nt);
+		s.persistent = cus;
+	}
+	if (s.T.nTiles == 0 || s.T.nTiles > 8000)  // 64 KB of fill-pass LDS
+		return false;
+	s.C = 1;
+	while (s.C < 8 && s.T.nTiles * s.C * 2 <= 4096)
+		s.C *= 2;
+	s.nB = (int64_t)s.T.nTiles * s.C;
+	// a ray crosses at most one tile face per tile and axis; a footprint's
+	// records are not bounded so (a batch of more takes the direct kernel)
+	s.recPer = s.dd ? std::min<int64_t>(128, 8 * std::max(s.T.ntx, s.T.nty))
+	                : std::min<int64_t>(64, s.T.ntx + s.T.nty + s.T.ntz - 2);
+	s.brick = (em && !s.dd) ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt : 0;
+	return true;
+}
+
+// LORs [b, e) of L.
+DLors sliceLors(const DLors& L, int64_t b, int64_t e)
+{
+	DLors r = L;
+	r.n = e - b;
+	r.first = L.first + b;
+	r.d1 = L.d1 ? L.d1 + b : nullptr;
+	r.d2 = L.d2 ? L.d2 + b : nullptr;
+	r.bins = L.bins ? L.bins + b : nullptr;
+	r.tof = L.tof ? L.tof + b : nullptr;
+	r.frame = L.frame ? L.frame + b : nullptr;
+	r.motion = L.motion ? L.motion + b : nullptr;
+	return r;
+}
+
+// The context's scratch is used in stream order: a call on another stream
+// than the last one's waits for it.
+int wsAcquire(yrtmi_ctx* c)
+{
+	if (!c->capturing && c->wsUsed && c->wsStream != c->stream)
+		HIP_TRY(hipStreamWaitEvent(c->stream, c->wsEvent, 0));
+	return YRTMI_OK;
+}
+
+int wsRelease(yrtmi_ctx* c)
+{
+	if (c->capturing)
+	{
+		c->wsCaptured = true;
+		return YRTMI_OK;
+	}
+	if (c->wsEvent == nullptr)
+		HIP_TRY(hipEventCreateWithFlags(&c->wsEvent, hipEventDisableTiming));
+	HIP_TRY(hipEventRecord(c->wsEvent, c->stream));
+	c->wsStream = c->stream;
+	c->wsUsed = true;
+	return YRTMI_OK;
+}
+
+// LORs per batch that the scratch has room for.
+int64_t streamBatch(const yrtmi_ctx* c, const StreamShape& s, int64_t n)
+{
+	if (c->ws == nullptr || c->wsBytes <= s.fixedBytes())
+		return 0;
+	int64_t b = (int64_t)((c->wsBytes - s.fixedBytes()) / s.lorBytes());
+	// keys and record numbers are 32 bits
+	b = std::min(b, ((int64_t(1) << 31) / std::max<int64_t>(1, s.recPer)) / s.R);
+	return std::min(b, n);
+}
+
+// Whether a backprojection of a.L goes through streamBack, its scratch then
+// made ready.
+bool streamReady(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a, bool em, StreamShape& s)
+{
+	const int64_t n = a.L.n, rays = n * (int64_t)a.pr.numRays, least = streamMinRays(a);
+	if (p->accum != YRTMI_ACCUM_XCD || rays < least || !streamShape(c, a, em, s))
+		return false;
+	const size_t want =
+	    std::max(s.fixedBytes() + (size_t)std::min<int64_t>(n, 1 << 26) * s.lorBytes(), size_t(1));
+	const size_t cap = std::max(std::min(want, kStreamBytes + (size_t)s.brick * 4),
+	                            s.fixedBytes() + (size_t)((least + s.R) / s.R) * s.lorBytes());
+	if (c->wsBytes < cap && !c->capturing)
+	{
+		void* q = nullptr;
+		const size_t bytes = std::max(cap, c->wsBytes + c->wsBytes / 2);
+		if (poolAlloc(c->device, &q, bytes) == hipSuccess)
+		{
+			if (c->wsCaptured)
+				c->wsRetired.push_back(c->ws);
+			else
+				poolFree(c->device, c->ws, c->ws == nullptr || poolQuiesce(c->device));
+			c->ws = q;
+			c->wsBytes = bytes;
+		}
+		else
+			(void)hipGetLastError();
+	}
+	const int64_t b = streamBatch(c, s, n);
+	return b == n || b * s.R >= least;
+}
+
+enum StreamKind
+{
+	STREAM_BACK,  // y += A^T vals
+	STREAM_EM,    // y += A^T (EM ratio of a.x)
+	STREAM_SENS   // y += A^T (sensitivity values)
+};
+
+int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamShape& s,
+               StreamKind kind, float* y, const float* vals)
+{
+	int r = wsAcquire(c);
+	if (r)
+		return r;
+	hipStream_t st = c->stream;
+	const int64_t n = a0.L.n, batch = streamBatch(c, s, n);
+	char* at = (char*)c->ws;
+	auto take = [&](size_t bytes) {
+		char* q = at;
+		at += (bytes + 255) / 256 * 256;
+		return (void*)q;
+	};
+	// the state, counts and cursors are cleared together
+	const size_t clearBytes = sizeof(StreamState) + (size_t)s.nB * 12;
+	StreamState* state = (StreamState*)take(clearBytes);
+	DPlan pl{};
+	pl.R = s.R;
+	pl.C = s.C;
+	lengthCuts(pl, s.dd, s.T);
+	pl.count = (unsigned long long*)(state + 1);
+	pl.cursor = (unsigned int*)(pl.count + s.nB);
+	int64_t* off = (int64_t*)take((size_t)s.nB * 8);
+	pl.tileOff = off;
+	pl.blockCnt = (unsigned int*)take((size_t)kStreamBinGroups * s.nB * 4);
+	pl.err = &state->err;
+	pl.skip = &state->err;
+	float* brick = (float*)take((size_t)s.brick * 4);
+	float* v = (float*)take((size_t)batch * 4);
+	float4* table = (float4*)take((size_t)batch * s.R * s.tabVec * sizeof(float4));
+	const int64_t cap = batch * s.R * s.recPer;
+	TileChunk* chunks = (TileChunk*)take((size_t)(s.T.nTiles + 1024 + cap / 4096 + 2) *
+	                                     sizeof(TileChunk));
+	pl.ray = table;
+	pl.rec = (uint32_t*)take((size_t)cap * s.words * 4);
+	DPlanRead rd{};
+	rd.R = s.R;
+	rd.chunks = chunks;
+	rd.rec = pl.rec;
+	rd.ray = table;
+	rd.queue = state->queue;
+	rd.vexp = reinterpret_cast<const int*>(state->queue + 2);
+	rd.nChunksDev = &state->nChunks;
+	rd.err = &state->err;
+	KArgs a = a0;
+	a.part = nullptr;
+	if (kind == STREAM_SENS)
+	{
+		// frame 0 of the image, without TOF
+		a.pr.useTof = 0;
+		a.im.nt = 1;
+	}
+	if (kind == STREAM_EM && !s.dd)
+	{
+		HIP_TRY(launchToBricks(a.im, a.x, brick, st));
+		a.xb = brick;
+		a.bvox = brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz);
+	}
+	auto shift = [](const float* q, int64_t b) { return q ? q + b : nullptr; };
+	for (int64_t b = 0; b < n; b += batch)
+	{
+		const int64_t e = std::min(n, b + batch);
+		a.L = sliceLors(a0.L, b, e);
+		const int64_t rays = a.L.n * (int64_t)s.R;
+		const int grid =
+		    (int)std::min<int64_t>((rays + kBinThreads - 1) / kBinThreads, kStreamBinGroups);
+		HIP_TRY(launchClearWords((unsigned int*)state, (int64_t)clearBytes / 4, st));
+		HIP_TRY(launchRayPrep(a, table, pl.err, st));
+		HIP_TRY(launchBin(0, a, s.T, pl, grid, st));
+		HIP_TRY(launchStreamScan(pl, off, s.T.nTiles, cap, chunks, state, st));
+		HIP_TRY(launchBin(1, a, s.T, pl, grid, st));
+		const float* bv = v;
+		if (kind == STREAM_BACK)
+			bv = vals + b;
+		else if (kind == STREAM_SENS)
+		{
+			a.vals = shift(a0.vals, b);
+			HIP_TRY(launchSensValue(a, v, st));
+		}
+		else
+		{
+			a.c.meas = shift(a0.c.meas, b);
+			a.c.sens = shift(a0.c.sens, b);
+			a.c.att = shift(a0.c.att, b);
+			a.c.randoms = shift(a0.c.randoms, b);
+			a.c.scatter = shift(a0.c.scatter, b);
+			a.c.precorr = shift(a0.c.precorr, b);
+			a.rays = s.dd ? table : nullptr;
+			HIP_TRY(launchEmRatio(a, p->lpe, v, st));
+		}
+		HIP_TRY(launchTileBack(a, s.T, rd, bv, y, s.persistent, st));
+		a.vals = bv;
+		a.y = y;
+		HIP_TRY(launchBackIf(a, rd.err, st));
+	}
+	return wsRelease(c);
+}
+
 // Set up per-XCD accumulation for a backprojection of n voxels into y, or
 // leave the kernel writing y directly.
 int setupAccum(yrtmi_ctx* c, const yrtmi_proj* p, KArgs& a, int64_t n)
 {
 	a.part = nullptr;
 	if (p->accum != YRTMI_ACCUM_XCD || c->nxcc <= 1)
+		return YRTMI_OK;
+	// recording, no partial images yet, but a call before made the scratch
+	// of streamBack instead of them: straight into y
+	if (c->capturing && c->ws != nullptr && c->partStride < n)
 		return YRTMI_OK;
 	int r = ensurePartials(c, n);
 	if (r)
@@ -400,6 +687,15 @@ int yrtmi_ctx_destroy(yrtmi_ctx* c)
 	(void)hipFree(c->counter);
 	(void)hipFree(c->part);
 	(void)hipFree(c->brick);
+	if (c->ws != nullptr)
+	{
+		const bool idle = poolQuiesce(c->device);
+		poolFree(c->device, c->ws, idle);
+		for (void* p : c->wsRetired)
+			poolFree(c->device, p, idle);
+	}
+	if (c->wsEvent != nullptr)
+		(void)hipEventDestroy(c->wsEvent);
 	if (c->owned != nullptr)
 		(void)hipStreamDestroy(c->owned);
 	poolRelease(c->device);
@@ -478,8 +774,16 @@ int yrtmi_graph_launch(yrtmi_ctx* c, const yrtmi_graph* g)
 	r = notCapturing(c, "graph_launch");
 	if (r)
 		return r;
+	if (!c->wsCaptured)
+	{
+		HIP_TRY(hipGraphLaunch(g->exec, c->stream));
+		return YRTMI_OK;
+	}
+	r = wsAcquire(c);
+	if (r)
+		return r;
 	HIP_TRY(hipGraphLaunch(g->exec, c->stream));
-	return YRTMI_OK;
+	return wsRelease(c);
 }
 
 int yrtmi_graph_destroy(yrtmi_graph* g)
@@ -914,6 +1218,9 @@ int yrtmi_back(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 		return fail(YRTMI_EINVAL, "back: null image or values");
 	a.y = img;
 	a.vals = vals;
+	StreamShape ss;
+	if (streamReady(c, p, a, false, ss))
+		return streamBack(c, p, a, ss, STREAM_BACK, img, vals);
 	const int64_t ny = a.im.nvox * a.im.nt;
 	r = setupAccum(c, p, a, ny);
 	if (r)
@@ -986,6 +1293,9 @@ int yrtmi_em_subset(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 		a.c.denomThr = corr->denom_threshold;
 		a.c.precorr = corr->precorr;
 	}
+	StreamShape ss;
+	if (streamReady(c, p, a, true, ss))
+		return streamBack(c, p, a, ss, STREAM_EM, u, nullptr);
 	const int64_t ny = a.im.nvox * a.im.nt;
 	r = setupAccum(c, p, a, ny);
 	if (r)
@@ -1084,6 +1394,11 @@ int yrtmi_sensitivity(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	a.y = img;
 	a.vals = sens;
 	a.L.tof = nullptr;
+	StreamShape ss;
+	KArgs as = a;
+	as.im.nt = 1;
+	if (streamReady(c, p, as, false, ss))
+		return streamBack(c, p, as, ss, STREAM_SENS, img, nullptr);
 	r = setupAccum(c, p, a, a.im.nvox);
 	if (r)
 		return r;
@@ -1568,17 +1883,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	const int64_t tabBytes = tabVec * (int64_t)sizeof(float4) * l->n * (int64_t)R;
 	if (o.max_bytes > 0 && (int64_t)sizeof(float) * l->n + tabBytes > o.max_bytes)
 		return fail(YRTMI_ENOMEM, "plan: the ray table exceeds the memory budget");
-	DTiles T{};
-	T.shape = o.tile_shape;
-	T.tx = tileDim(T.shape, 0);
-	T.ty = tileDim(T.shape, 1);
-	T.tz = tileDim(T.shape, 2);
-	T.lx = __builtin_ctz((unsigned)T.tx);
-	T.ly = __builtin_ctz((unsigned)T.ty);
-	T.lz = __builtin_ctz((unsigned)T.tz);
-	T.ntx = (int32_t)((im->nx + T.tx - 1) / T.tx);
-	T.nty = (int32_t)((im->ny + T.ty - 1) / T.ty);
-	T.ntz = (int32_t)((im->nz + T.tz - 1) / T.tz);
+	DTiles T = tilesOf(o.tile_shape, im->nx, im->ny, im->nz, im->nt);
 	const int64_t nT = (int64_t)T.ntx * T.nty * T.ntz * im->nt;
 	// the fill pass keeps a counter and a 32-bit base per bin in LDS
 	int maxLds = 65536;
@@ -1595,7 +1900,6 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 		              (long long)nT, (long long)binCap);
 		return fail(YRTMI_EINVAL, msg);
 	}
-	T.nTiles = (int32_t)nT;
 
 	yrtmi_plan* q = new yrtmi_plan();
 	q->device = c->device;
@@ -1645,10 +1949,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	if (l->n == 0)
 		return cleanup(YRTMI_OK);
 	// length classes: up to 8, as long as tiles x classes stays within
-	// 4096 bins (48 KB of fill-pass LDS) and the LDS limit.  Siddon: cut at
-	// fractions of the longest piece a tile can hold (tx + ty + tz segments);
-	// DD: at multiples of the slices of a tile slab (a piece of a footprint
-	// a few voxels wide and high holds a few voxels per slice)
+	// 8192 bins (64 KB of fill-pass LDS) and the LDS limit
 	DPlan pl{};
 	pl.R = R;
 	pl.C = 1;
@@ -1656,24 +1957,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	const int maxC = dd ? kMaxClasses : 8;
 	while (pl.C < maxC && nT * pl.C * 2 <= std::min<int64_t>(binCap, kMaxBins))
 		pl.C *= 2;
-	// (16 classes, DD: about 15 % apart where most pieces lie)
-	if (dd)
-	{
-		const int L = std::max(T.tx, T.ty);
-		static const int f16[15] = {1, 2, 3, 4, 6, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40},
-		                 f8[7] = {1, 2, 4, 8, 12, 16, 24}, f4[3] = {2, 6, 16}, f2[1] = {8};
-		const int* f = pl.C == 16 ? f16 : (pl.C == 8 ? f8 : (pl.C == 4 ? f4 : f2));
-		for (int k = 0; k < pl.C - 1; k++)
-			pl.cut[k] = std::max(1, L * f[k] / 4);
-	}
-	else
-	{
-		const int L = T.tx + T.ty + T.tz;
-		static const int f8[7] = {3, 6, 9, 12, 16, 21, 28}, f4[3] = {6, 12, 21}, f2[1] = {12};
-		const int* f = pl.C == 8 ? f8 : (pl.C == 4 ? f4 : f2);
-		for (int k = 0; k < pl.C - 1; k++)
-			pl.cut[k] = std::max(1, L * f[k] / 40);
-	}
+	lengthCuts(pl, dd, T);
 	const int64_t nB = nT * pl.C;
 	const int64_t rays = l->n * (int64_t)R;
 	const int grid = (int)std::min<int64_t>((rays + kBinThreads - 1) / kBinThreads, 2048);

@@ -188,6 +188,7 @@ struct DLors
 	const uint32_t* d2;
 	const uint32_t* bins;
 	uint32_t S, s, nps;  // subset iterator: S subsets, subset s, phis in it
+	int64_t first;       // subset iterator: its element that is LOR 0
 	const float* tof;
 	const int32_t* frame;
 	const uint8_t* motion;
@@ -320,7 +321,7 @@ __device__ __forceinline__ bool eventPair(const DScanner& S, const DLors& L,
 	else
 	{
 		// BinIteratorRangeHistogram3D::getSafe (BinIterator.cpp:191-198)
-		const uint32_t idx = (uint32_t)e;
+		const uint32_t idx = (uint32_t)(L.first + e);
 		const uint32_t per = L.nps * S.numR;
 		zb = idx / per;
 		const uint32_t rem = idx - zb * per;

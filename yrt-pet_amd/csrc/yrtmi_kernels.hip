@@ -187,6 +187,38 @@ __global__ void __launch_bounds__(256) kEvents(KArgs a)
 	}
 }
 
+// Backprojection of a.vals into a.y with global atomics if *flag is set: a
+// batch that could not be binned by tiles (StreamState::err).
+template <int TYPE, bool TOF, bool S64>
+__global__ void __launch_bounds__(256) kBackIf(KArgs a, const int* __restrict__ flag)
+{
+	if (*flag == 0)
+		return;
+	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+	uint32_t cnt = 0;
+	for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < a.L.n; e += stride)
+	{
+		const Lor l = fetchLor(a.sc, a.L, e, a.im.nt);
+		if (l.frame >= 0 && a.vals[e] != 0.f)
+			backLane<TYPE, TOF, 1, S64, MODE_BACK>(a, l, 0, a.y + (int64_t)l.frame * a.im.nvox,
+			                                       a.vals[e], cnt);
+	}
+}
+
+hipError_t launchBackIf(const KArgs& a, const int* flag, hipStream_t st)
+{
+	const unsigned g = (unsigned)std::min<int64_t>(std::max<int64_t>((a.L.n + 255) / 256, 1), 2048);
+	const bool tof = a.pr.useTof != 0, s64 = a.pr.setup64 != 0;
+	auto go = [&](auto k) { k<<<g, 256, 0, st>>>(a, flag); };
+	if (a.pr.type == 1)
+		tof ? (s64 ? go(kBackIf<1, true, true>) : go(kBackIf<1, true, false>))
+		    : (s64 ? go(kBackIf<1, false, true>) : go(kBackIf<1, false, false>));
+	else
+		tof ? (s64 ? go(kBackIf<0, true, true>) : go(kBackIf<0, true, false>))
+		    : (s64 ? go(kBackIf<0, false, true>) : go(kBackIf<0, false, false>));
+	return hipGetLastError();
+}
+
 // Per-LOR attenuation factor exp(-0.1 * Siddon(mu)) (Corrector.cpp:601-611).
 __global__ void __launch_bounds__(256) kAttFactors(KArgs a)
 {

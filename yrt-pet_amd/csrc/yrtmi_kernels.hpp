@@ -13,6 +13,8 @@ namespace yrtmi
 // the grid from the event count; otherwise the kernel grid-strides.
 hipError_t launchEvents(int mode, const KArgs& a, int lpe, int block,
                         int64_t grid, hipStream_t st);
+// a.y += backprojection of a.vals with global atomics, if *flag (device).
+hipError_t launchBackIf(const KArgs& a, const int* flag, hipStream_t st);
 hipError_t launchAttFactors(const KArgs& a, hipStream_t st);
 hipError_t launchEmUpdate(float* x, const float* u, const float* s,
                           int64_t nvox, int64_t nt, int64_t sFrames, float thr,

@@ -316,6 +316,8 @@ __global__ void __launch_bounds__(kBinThreads) kBin(DImage im, DProj pr, int64_t
 		}
 		return;
 	}
+	if (pl.skip != nullptr && *pl.skip != 0)
+		return;
 	for (int i = threadIdx.x; i < nB; i += blockDim.x)
 	{
 		const int c = (int)myCnt[i];
@@ -860,6 +862,9 @@ __global__ void __launch_bounds__(tileThreads(SHAPE))
 		tileChunk<DD, TOF, S64, SHAPE>(a, T, pl, pl.chunks[blockIdx.x], v, y, acc, psfL);
 		return;
 	}
+	if (pl.err != nullptr && *pl.err != 0)
+		return;
+	const int64_t nChunks = pl.nChunksDev != nullptr ? *pl.nChunksDev : pl.nChunks;
 	// the next chunk's index is passed through the tile's first word (read
 	// between two barriers, before the chunk clears the tile), so the
 	// workgroup's LDS is the tile alone: 32 KB for 16^3, five per CU
@@ -870,7 +875,7 @@ __global__ void __launch_bounds__(tileThreads(SHAPE))
 		__syncthreads();
 		const int64_t c = (int64_t)acc[0];
 		__syncthreads();
-		if (c >= pl.nChunks)
+		if (c >= nChunks)
 			break;
 		tileChunk<DD, TOF, S64, SHAPE>(a, T, pl, pl.chunks[c], v, y, acc, psfL);
 	}
@@ -1279,10 +1284,119 @@ __global__ void __launch_bounds__(256) kVExpScale(const float* __restrict__ v, i
 		*e = t - 126;
 }
 
+__global__ void __launch_bounds__(256) kClearWords(unsigned int* __restrict__ p, int64_t n)
+{
+	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+	for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+		p[i] = 0u;
+}
+
+hipError_t launchClearWords(unsigned int* p, int64_t words, hipStream_t st)
+{
+	const unsigned g = (unsigned)std::min<int64_t>(std::max<int64_t>((words + 255) / 256, 1), 256);
+	kClearWords<<<g, 256, 0, st>>>(p, words);
+	return hipGetLastError();
+}
+
+// Exclusive prefix of v over the workgroup's 1024 threads; *total, its sum.
+__device__ __forceinline__ unsigned long long scan1024(unsigned long long v,
+                                                       unsigned long long* lds,
+                                                       unsigned long long* total)
+{
+	const int lane = (int)(threadIdx.x & 63u), w = (int)(threadIdx.x >> 6);
+	unsigned long long incl = v;
+#pragma unroll
+	for (int d = 1; d < 64; d <<= 1)
+	{
+		const unsigned long long t = __shfl_up(incl, (unsigned int)d, 64);
+		if (lane >= d)
+			incl += t;
+	}
+	__syncthreads();
+	if (lane == 63)
+		lds[w] = incl;
+	__syncthreads();
+	unsigned long long before = 0, sum = 0;
+#pragma unroll
+	for (int k = 0; k < 16; k++)
+	{
+		before += (k < w) ? lds[k] : 0ull;
+		sum += lds[k];
+	}
+	*total = sum;
+	return before + incl - v;
+}
+
+__global__ void __launch_bounds__(1024)
+    kStreamScan(DPlan pl, int64_t* __restrict__ tileOff, int nTiles, int64_t cap,
+                TileChunk* __restrict__ chunks, StreamState* s)
+{
+	__shared__ unsigned long long lds[16];
+	const int per = (nTiles + 1023) / 1024;
+	const int t0 = min((int)threadIdx.x * per, nTiles), t1 = min(t0 + per, nTiles);
+	auto tileCount = [&](int t) {
+		unsigned long long n = 0;
+		for (int k = 0; k < pl.C; k++)
+			n += pl.count[t * pl.C + k];
+		return n;
+	};
+	unsigned long long recs = 0;
+	for (int t = t0; t < t1; t++)
+		recs += tileCount(t);
+	unsigned long long total, nFull, nPart;
+	unsigned long long at = scan1024(recs, lds, &total);
+	if (total > (unsigned long long)cap || s->err != 0)
+	{
+		if (threadIdx.x == 0)
+		{
+			s->nChunks = 0;
+			if (total > (unsigned long long)cap)
+				s->err |= 4;
+		}
+		return;
+	}
+	const unsigned long long CH = (unsigned long long)chunkRecords((int64_t)total);
+	unsigned long long full = 0, part = 0;
+	for (int t = t0; t < t1; t++)
+	{
+		const unsigned long long n = tileCount(t);
+		full += n / CH;
+		part += (n % CH != 0) ? 1 : 0;
+	}
+	unsigned long long fi = scan1024(full, lds, &nFull);
+	unsigned long long pi = scan1024(part, lds, &nPart) + nFull;
+	for (int t = t0; t < t1; t++)
+	{
+		const unsigned long long begin = at;
+		for (int k = 0; k < pl.C; k++)
+		{
+			tileOff[t * pl.C + k] = (int64_t)at;
+			at += pl.count[t * pl.C + k];
+		}
+		for (unsigned long long b = begin; b < at; b += CH)
+		{
+			TileChunk c;
+			c.begin = (int64_t)b;
+			c.tile = t;
+			c.count = (int32_t)(at - b < CH ? at - b : CH);
+			chunks[c.count == (int32_t)CH ? fi++ : pi++] = c;
+		}
+	}
+	if (threadIdx.x == 0)
+		s->nChunks = (int64_t)(nFull + nPart);
+}
+
+hipError_t launchStreamScan(const DPlan& pl, int64_t* tileOff, int nTiles, int64_t cap,
+                            TileChunk* chunks, StreamState* s, hipStream_t st)
+{
+	kStreamScan<<<1, 1024, 0, st>>>(pl, tileOff, nTiles, cap, chunks, s);
+	return hipGetLastError();
+}
+
 hipError_t launchTileBack(const KArgs& a, const DTiles& T, const DPlanRead& pl,
                           const float* v, float* y, int persistent, hipStream_t st)
 {
-	if (pl.nChunks <= 0)
+	if (pl.nChunks <= 0 && pl.nChunksDev == nullptr)
 		return hipSuccess;
 	if (pl.vexp != nullptr)
 	{
@@ -1299,7 +1413,9 @@ hipError_t launchTileBack(const KArgs& a, const DTiles& T, const DPlanRead& pl,
 	}
 	DPlanRead q = pl;
 	unsigned grid;
-	if (persistent > 0 && pl.queue != nullptr)
+	if (pl.nChunksDev != nullptr)
+		grid = (unsigned)persistent;
+	else if (persistent > 0 && pl.queue != nullptr)
 		grid = (unsigned)std::min<int64_t>(persistent, pl.nChunks);
 	else
 	{

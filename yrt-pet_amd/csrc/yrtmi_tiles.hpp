@@ -118,7 +118,44 @@ struct DPlan
 	uint32_t* rec;
 	const float4* ray;          // ray table (rayEntry + sidStore / ddStore, kRayPrep)
 	int* err;                   // set when a tile range would overflow
+	const int* skip;            // (nullable) the fill pass does nothing if set
 };
+
+// Cuts of a plan's length classes (DPlan::cut) for its number of classes.
+// Siddon: at fractions of the longest piece a tile can hold (tx + ty + tz
+// segments); DD: at multiples of the slices of a tile slab (a piece of a
+// footprint a few voxels wide and high holds a few voxels per slice; 16
+// classes are about 15 % apart where most pieces lie).
+inline void lengthCuts(DPlan& pl, bool dd, const DTiles& T)
+{
+	static const int d16[15] = {1, 2, 3, 4, 6, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40},
+	                 d8[7] = {1, 2, 4, 8, 12, 16, 24}, d4[3] = {2, 6, 16}, d2[1] = {8};
+	static const int s8[7] = {3, 6, 9, 12, 16, 21, 28}, s4[3] = {6, 12, 21}, s2[1] = {12};
+	const int* f = dd ? (pl.C == 16 ? d16 : (pl.C == 8 ? d8 : (pl.C == 4 ? d4 : d2)))
+	                  : (pl.C == 8 ? s8 : (pl.C == 4 ? s4 : s2));
+	const int L = dd ? std::max(T.tx, T.ty) : T.tx + T.ty + T.tz;
+	for (int k = 0; k < pl.C - 1; k++)
+		pl.cut[k] = std::max(1, L * f[k] / (dd ? 4 : 40));
+}
+
+// Tiles of shape `shape` of an image of nt frames (nTiles 0: 2^31 or more).
+inline DTiles tilesOf(int shape, int64_t nx, int64_t ny, int64_t nz, int64_t nt)
+{
+	DTiles T{};
+	T.shape = shape;
+	T.tx = tileDim(shape, 0);
+	T.ty = tileDim(shape, 1);
+	T.tz = tileDim(shape, 2);
+	T.lx = __builtin_ctz((unsigned)T.tx);
+	T.ly = __builtin_ctz((unsigned)T.ty);
+	T.lz = __builtin_ctz((unsigned)T.tz);
+	T.ntx = (int32_t)((nx + T.tx - 1) / T.tx);
+	T.nty = (int32_t)((ny + T.ty - 1) / T.ty);
+	T.ntz = (int32_t)((nz + T.tz - 1) / T.tz);
+	const int64_t n = (int64_t)T.ntx * T.nty * T.ntz * nt;
+	T.nTiles = n < (int64_t(1) << 31) ? (int32_t)n : 0;
+	return T;
+}
 
 // Ray table of a Siddon plan, rayTabVec(S64) float4 per (LOR, ray) t = lor *
 // R + ray.  The first two: the ray's end points after multi-ray offsets,
@@ -164,7 +201,28 @@ struct DPlanRead
 	// before each launch): sets the fixed-point scale of the tile
 	// accumulation
 	const int* vexp;
+	// plans made and used on the device (launchStreamScan): the chunk count,
+	// and an error word that, when set, leaves the image untouched
+	const int64_t* nChunksDev;
+	const int* err;
 };
+
+// State of a plan made on the device: cleared before each batch, together
+// with the bins' counts and cursors behind it.
+struct StreamState
+{
+	int64_t nChunks;
+	int err;  // 1 / 2: as DPlan::err; 4: more records than there is room for
+	int pad;
+	unsigned int queue[260];  // as a plan's queue words
+};
+// Clears `words` 32-bit words.
+hipError_t launchClearWords(unsigned int* p, int64_t words, hipStream_t st);
+// From pl.count: pl.tileOff, the chunk table (chunkRecords of the total,
+// full chunks first) and s->nChunks; s->err |= 4 and no chunks when there
+// are more than `cap` records or an error before.  One workgroup.
+hipError_t launchStreamScan(const DPlan& pl, int64_t* tileOff, int nTiles, int64_t cap,
+                            TileChunk* chunks, StreamState* s, hipStream_t st);
 
 // LDS of the fill pass: an int counter and a 32-bit base per bin.
 inline size_t binLdsBytes(int nB)
