@@ -1493,10 +1493,7 @@ int yrtmi_psf_apply(yrtmi_ctx* c, const yrtmi_image* im, const float* in, float*
 			taps[a].k[i] = transpose ? ks[a][nk[a] - 1 - i] : ks[a][i];
 	}
 	const int nx = (int)im->nx, ny = (int)im->ny, nz = (int)im->nz;
-	// x: in -> out, y: out -> tmp, z: tmp -> out
-	HIP_TRY(launchPsfAxis(0, in, out, taps[0], nx, ny, nz, (int)total, c->stream));
-	HIP_TRY(launchPsfAxis(1, out, tmp, taps[1], nx, ny, nz, (int)total, c->stream));
-	HIP_TRY(launchPsfAxis(2, tmp, out, taps[2], nx, ny, nz, (int)total, c->stream));
+	HIP_TRY(launchPsf(in, tmp, out, taps, nx, ny, nz, im->nt, c->stream));
 	return YRTMI_OK;
 }
 

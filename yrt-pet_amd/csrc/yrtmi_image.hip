@@ -1,62 +1,200 @@
 // Image-space kernels for gfx950: the separable image-space PSF
 // (OperatorPsf::convolve, OperatorPsf.cpp:290-375; its device form
-// convolve3DSeparable_kernel, ImageSpaceKernels.cu:296-341).
-//
-// One launch per axis over every voxel of every frame, x fastest in the
-// thread index, so that the loads of each tap are coalesced whatever the
-// axis; the taps are kernel arguments (uniform: scalar loads).  The sum runs
-// over kk = -h..h ascending with a separate multiply and add, the order of
-// the reference's CPU loop, so the result is bitwise the same.  HBM-bound:
-// 8 B per voxel per axis (the taps' neighbours hit L2).
+// convolve3DSeparable_kernel, ImageSpaceKernels.cu:296-341), and the
+// time-averaged moved image.
 #include "yrtmi_kernels.hpp"
 
 namespace yrtmi
 {
 
-template <int AXIS>
-__global__ void __launch_bounds__(256) kPsfAxis(const float* __restrict__ in,
-                                                float* __restrict__ out, PsfTaps t,
-                                                int nx, int ny, int nz, int total)
+// One output of an axis is sum over i = 0 .. n - 1, ascending, of k[i] *
+// in[c + h - i] (circular), each product and sum rounded separately: the
+// order of the reference's CPU loop, so the result is bitwise the same.  A
+// thread forms M consecutive outputs of a line in registers; per tap it needs
+// one new element of the line (get(j): element c + j of the first output's),
+// so a voxel costs (M + n - 1) / M reads an axis and two VALU a tap, the taps
+// being kernel arguments (uniform: scalar loads).
+template <int M, class Get>
+__device__ __forceinline__ void convolveLine(const PsfTaps& t, Get&& get, float (&acc)[M])
 {
 #pragma clang fp contract(off)
-	const int h = t.n / 2;
-	const int stride = (int)(gridDim.x * blockDim.x);
-	for (int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); i < total; i += stride)
+	// four taps a round: w[j] = element h - i - 3 + j, moved on by four
+	float w[M + 3];
+	int e = t.n / 2;  // h - i
+#pragma unroll
+	for (int j = 0; j < M; j++)
 	{
-		const int x = i % nx;
-		const int r = i / nx;
-		const int y = r % ny;
-		const int z = (r / ny) % nz;
-		// the voxel's line along AXIS: its first element and stride, the
-		// coordinate along it and its length
-		const int c = AXIS == 0 ? x : (AXIS == 1 ? y : z);
-		const int n = AXIS == 0 ? nx : (AXIS == 1 ? ny : nz);
-		const int st = AXIS == 0 ? 1 : (AXIS == 1 ? nx : nx * ny);
-		const int base = i - c * st;
-		float sum = 0.f;
-		for (int kk = -h; kk <= h; kk++)
+		acc[j] = 0.f;
+		w[j + 3] = get(e + j);
+	}
+	int i = 0;
+	for (; i + 4 <= t.n; i += 4, e -= 4)
+	{
+#pragma unroll
+		for (int j = 0; j < 3; j++)
+			w[j] = get(e - 3 + j);
+#pragma unroll
+		for (int u = 0; u < 4; u++)
 		{
-			// util::circular (Tools.cpp:160-167): one wrap (h < n)
-			int q = c - kk;
-			q = q < 0 ? q + n : (q >= n ? q - n : q);
-			sum = sum + t.k[kk + h] * in[base + q * st];
+			const float k = t.k[i + u];
+#pragma unroll
+			for (int j = 0; j < M; j++)
+				acc[j] = acc[j] + k * w[j + 3 - u];
 		}
-		out[i] = sum;
+#pragma unroll
+		for (int j = M + 2; j >= 4; j--)
+			w[j] = w[j - 4];
+		// (read only where a tap follows)
+		w[3] = (i + 4 < t.n) ? get(e - 4) : 0.f;
+	}
+	for (; i < t.n; i++, e--)
+	{
+		const float k = t.k[i];
+#pragma unroll
+		for (int j = 0; j < M; j++)
+			acc[j] = acc[j] + k * w[j + 3];
+#pragma unroll
+		for (int j = M + 2; j >= 4; j--)
+			w[j] = w[j - 1];
+		w[3] = (i + 1 < t.n) ? get(e - 1) : 0.f;
 	}
 }
 
-hipError_t launchPsfAxis(int axis, const float* in, float* out, const PsfTaps& t, int nx,
-                         int ny, int nz, int total, hipStream_t st)
+// x, then y: one workgroup per kPsfTX x TY voxels of a plane (TY 32, or 16
+// where kernels of up to 63 taps would take more than 64 KB of LDS), the plane's
+// patch with its halo read into LDS once, convolved along x into a second
+// LDS array and from there along y.  (Rows are a multiple of 8 plus one word
+// apart in both, so the 8 threads of each of 8 rows meet 64 different banks.)
+// One pass over memory for two axes; with kPsfZ a PSF of 9 taps of 4 frames
+// of 200 x 200 x 128 takes 105 us where three passes, a global load per tap,
+// took 460; a copy of the image takes 32.
+constexpr int kPsfTX = 64, kPsfM = 8;
+
+__host__ __device__ constexpr int psfPitch(int hx) { return (kPsfTX + 2 * hx + 7) / 8 * 8 + 1; }
+
+__global__ void __launch_bounds__(256) kPsfXY(const float* __restrict__ in,
+                                              float* __restrict__ out, PsfTaps tx, PsfTaps ty,
+                                              int nx, int ny, int TY)
 {
-	if (total <= 0)
-		return hipSuccess;
-	const unsigned g = (unsigned)std::min(std::max((total + 255) / 256, 1), 65536);
-	if (axis == 0)
-		kPsfAxis<0><<<g, 256, 0, st>>>(in, out, t, nx, ny, nz, total);
-	else if (axis == 1)
-		kPsfAxis<1><<<g, 256, 0, st>>>(in, out, t, nx, ny, nz, total);
-	else
-		kPsfAxis<2><<<g, 256, 0, st>>>(in, out, t, nx, ny, nz, total);
+	extern __shared__ float sm[];
+	const int hx = tx.n / 2, hy = ty.n / 2;
+	const int pitch = psfPitch(hx), rows = TY + 2 * hy;
+	float* patch = sm;
+	float* mid = sm + pitch * rows;  // rows of kPsfTX, kPsfTX + 1 apart
+	const int x0 = (int)blockIdx.x * kPsfTX, y0 = (int)blockIdx.y * TY;
+	const int64_t plane = (int64_t)blockIdx.z * nx * ny;
+	// util::circular (Tools.cpp:160-167): one wrap (h < n); elements that no
+	// output inside the image needs are read somewhere inside it
+	auto wrap = [](int q, int n) {
+		q = q < 0 ? q + n : (q >= n ? q - n : q);
+		return q < n ? q : 0;
+	};
+	const int lane = (int)(threadIdx.x & 63u),
+	          wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+	// (a row of at most 64 + 62 elements: two a lane)
+	const int xa = wrap(x0 - hx + lane, nx), xb = wrap(x0 - hx + 64 + lane, nx);
+	const bool second = lane < 2 * hx;
+	// the loads of four rows in flight together
+	for (int r0 = wv; r0 < rows; r0 += 16)
+	{
+		float va[4], vb[4];
+#pragma unroll
+		for (int j = 0; j < 4; j++)
+		{
+			const int r = min(r0 + 4 * j, rows - 1);
+			const float* line = in + plane + (int64_t)wrap(y0 - hy + r, ny) * nx;
+			va[j] = line[xa];
+			vb[j] = second ? line[xb] : 0.f;
+		}
+#pragma unroll
+		for (int j = 0; j < 4; j++)
+		{
+			const int r = r0 + 4 * j;
+			if (r < rows)
+			{
+				patch[r * pitch + lane] = va[j];
+				if (second)
+					patch[r * pitch + 64 + lane] = vb[j];
+			}
+		}
+	}
+	__syncthreads();
+	const int c8 = (int)(threadIdx.x & 7u) * kPsfM;
+	for (int r = (int)(threadIdx.x >> 3); r < rows; r += 32)
+	{
+		const float* p = patch + r * pitch + hx + c8;
+		float acc[kPsfM];
+		convolveLine<kPsfM>(tx, [&](int j) { return p[j]; }, acc);
+#pragma unroll
+		for (int j = 0; j < kPsfM; j++)
+			mid[r * (kPsfTX + 1) + c8 + j] = acc[j];
+	}
+	__syncthreads();
+	const int x = x0 + lane;
+	for (int g = wv; g < TY / kPsfM; g += 4)
+	{
+		const float* p = mid + (hy + g * kPsfM) * (kPsfTX + 1) + lane;
+		float acc[kPsfM];
+		convolveLine<kPsfM>(ty, [&](int j) { return p[j * (kPsfTX + 1)]; }, acc);
+#pragma unroll
+		for (int j = 0; j < kPsfM; j++)
+		{
+			const int y = y0 + g * kPsfM + j;
+			if (x < nx && y < ny)
+				out[plane + (int64_t)y * nx + x] = acc[j];
+		}
+	}
+}
+
+// z: one thread per column of kPsfMz voxels, x fastest across the threads;
+// the columns' overlap is read from cache.
+constexpr int kPsfMz = 16;
+
+__global__ void __launch_bounds__(256) kPsfZ(const float* __restrict__ in,
+                                             float* __restrict__ out, PsfTaps t, int nxy, int nz)
+{
+	const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+	if (i >= nxy)
+		return;
+	const int z0 = (int)blockIdx.y * kPsfMz;
+	const float* p = in + (int64_t)blockIdx.z * nxy * nz + i;
+	float acc[kPsfMz];
+	convolveLine<kPsfMz>(
+	    t,
+	    [&](int j) {
+		    int q = z0 + j;
+		    q = q < 0 ? q + nz : (q >= nz ? q - nz : q);
+		    return p[(int64_t)(q < nz ? q : 0) * nxy];
+	    },
+	    acc);
+	float* o = out + (int64_t)blockIdx.z * nxy * nz + i;
+#pragma unroll
+	for (int j = 0; j < kPsfMz; j++)
+		if (z0 + j < nz)
+			o[(int64_t)(z0 + j) * nxy] = acc[j];
+}
+
+hipError_t launchPsf(const float* in, float* tmp, float* out, const PsfTaps* t, int nx, int ny,
+                     int nz, int64_t frames, hipStream_t st)
+{
+	const int hx = t[0].n / 2, hy = t[1].n / 2;
+	auto ldsOf = [&](int TY) {
+		return sizeof(float) * (size_t)(psfPitch(hx) + kPsfTX + 1) * (size_t)(TY + 2 * hy);
+	};
+	const int TY = ldsOf(32) <= 65536 ? 32 : 16;
+	const size_t lds = ldsOf(TY);
+	const unsigned gx = (unsigned)((nx + kPsfTX - 1) / kPsfTX),
+	               gy = (unsigned)((ny + TY - 1) / TY);
+	const int nxy = nx * ny;
+	const unsigned gc = (unsigned)((nxy + 255) / 256), gz = (unsigned)((nz + kPsfMz - 1) / kPsfMz);
+	// (a grid has at most 65535 planes and frames)
+	const int64_t planes = frames * nz;
+	for (int64_t p = 0; p < planes; p += 65535)
+		kPsfXY<<<dim3(gx, gy, (unsigned)std::min<int64_t>(65535, planes - p)), 256, lds, st>>>(
+		    in + p * nxy, tmp + p * nxy, t[0], t[1], nx, ny, TY);
+	for (int64_t f = 0; f < frames; f += 65535)
+		kPsfZ<<<dim3(gc, gz, (unsigned)std::min<int64_t>(65535, frames - f)), 256, 0, st>>>(
+		    tmp + f * nz * nxy, out + f * nz * nxy, t[2], nxy, nz);
 	return hipGetLastError();
 }
 

@@ -37,17 +37,17 @@ hipError_t launchPairBins(const uint32_t* d1, const uint32_t* d2, int64_t n,
                           hipStream_t st);
 hipError_t launchFillI32(int32_t* x, int64_t n, int32_t v, hipStream_t st);
 
-// Image-space PSF: one axis (0 x, 1 y, 2 z) of the separable circular
-// convolution of every frame (nx * ny * nz * frames = total < 2^31 voxels),
-// taps passed by value.
+// Image-space PSF: the separable circular convolution of `frames` frames of
+// nx * ny * nz voxels with taps t[0] along x, t[1] along y (in -> tmp), t[2]
+// along z (tmp -> out), taps passed by value.
 constexpr int kMaxPsfTaps = 63;
 struct PsfTaps
 {
 	float k[kMaxPsfTaps];
 	int n;  // odd, <= kMaxPsfTaps
 };
-hipError_t launchPsfAxis(int axis, const float* in, float* out, const PsfTaps& t, int nx,
-                         int ny, int nz, int total, hipStream_t st);
+hipError_t launchPsf(const float* in, float* tmp, float* out, const PsfTaps* t, int nx, int ny,
+                     int nz, int64_t frames, hipStream_t st);
 
 // Time-averaged moved image: out[v] += sum over frames of weight *
 // trilinear(in, inverse transform * centre of v), for one frame of
