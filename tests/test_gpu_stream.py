@@ -154,3 +154,35 @@ def test_recorded_and_on_other_streams(gpu):
                                                                   ref2.cpu().numpy())
         print(f"replay {k}: {a:.2e}, other call {b:.2e}", flush=True)
         assert a <= 1e-5 and b <= 1e-5
+
+
+@pytest.mark.parametrize("kw", [dict(rays=2, tof=250.0), dict(rays=3, frames=2), dict(rays=5),
+                                dict(rays=2, tof=300.0, fp64=True)], ids=str)
+def test_bricked_forward_is_the_forward(gpu, kw):
+    """A forward of many rays of a large image gathers from its bricked copy;
+    calls of a few of its LORs do not: the same sums, bit for bit, also
+    recorded and replayed, and the attenuation of a sensitivity image too."""
+    nt = max(1, kw.get("frames", 0))
+    im = yrtmi.ImageParams(161, 127, 103, 1.5, 1.75, 1.0, nt=nt)
+    n = (im.nvox * nt // 4) // kw["rays"] + 1000
+    ctx, p, L, _ = setup(im, n, gpu=gpu, **kw)
+    x = torch.rand(im.shape, device=gpu, generator=torch.Generator(gpu).manual_seed(2))
+    y, z = torch.zeros(n, device=gpu), torch.zeros(n, device=gpu)
+    ctx.forward(p, im, x, L, y)
+    step = n // 5
+    for a in range(0, n, step):
+        b = min(n, a + step)
+        ctx.forward(p, im, x, L.slice(a, b), z[a:b])
+    torch.cuda.synchronize()
+    assert float(y.abs().sum()) > 0 and torch.equal(y, z)
+    s = torch.cuda.Stream()
+    ctx.set_stream(s)
+    with ctx.graph() as g:
+        ctx.forward(p, im, x, L, z)
+    for _ in range(3):
+        z.zero_()
+        torch.cuda.synchronize()
+        g.launch()
+        ctx.forward(p, im, x, L, y)
+        torch.cuda.synchronize()
+        assert torch.equal(y, z)

@@ -225,14 +225,14 @@ struct KArgs
 	float* part;
 	int64_t partStride;
 	int32_t nxcc;
-	// Ray table of a tile plan for these LORs (two float4 per LOR and ray:
-	// end points after offsets, TOF value, frame), or null: the forward of
-	// the EM ratio then reads it instead of resolving each LOR.
+	// Ray table of a DD tile plan for these LORs (ddStore), or null: the
+	// forward of the EM ratio then reads it instead of resolving each LOR.
 	const float4* rays;
 	// The Siddon EM ratio's forward reads the bricked copy of x (xb, bvox
-	// floats per frame, brickIndex), made by launchToBricks.
+	// floats per frame, brickIndex), made by launchToBricks, or x if null.
 	const float* xb;
 	int64_t bvox;
+	int32_t plain;  // the EM ratio kernels write the projection itself
 };
 
 // Hardware id of the XCD (accelerator complex die) running this wave.

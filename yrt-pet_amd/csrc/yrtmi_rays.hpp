@@ -900,16 +900,22 @@ __device__ __forceinline__ float siddonRay(const DImage& P,
 		return 0.f;
 	if constexpr (MODE == MODE_FWD)
 	{
-		// one FMA per segment in the walk's order, the voxel's value
-		// fetched one segment ahead (its gather overlaps a whole step)
-		float acc = 0.f, xv = 0.f;
+		// one FMA per segment in the walk's order, a segment behind the walk,
+		// and the voxel's value fetched a segment ahead: its gather has two
+		// steps to arrive (8.4 M attenuation rays at 256 x 256 x 128 3.5 ->
+		// 3.1 ms, 1 M unordered TOF LORs x 4 rays at 200 x 200 x 128 0.85 ->
+		// 0.76; a third step spills: slower)
+		float acc = 0.f, xv = 0.f, w1 = 0.f, x1 = 0.f;
 		sidWalk<TOF, S64, BRICK>(
 		    P, r, tof, imageBox(P), true, 0, 0, 0,
 		    [&](int, int, int, uint32_t, float, float w, uint32_t nidx) {
-			    acc = fmaf(w, xv, acc);
+			    acc = fmaf(w1, x1, acc);
+			    w1 = w;
+			    x1 = xv;
 			    xv = img[nidx];
 		    },
 		    [&](uint32_t idx) { xv = img[idx]; });
+		acc = fmaf(w1, x1, acc);
 		return acc * r.ws;
 	}
 	const float vs = val * r.ws;

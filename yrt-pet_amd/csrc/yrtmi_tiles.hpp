@@ -243,11 +243,18 @@ hipError_t launchChunkSort(bool dd, const DPlan& pl, const TileChunk* chunks, in
 // workgroup per chunk, or `persistent` workgroups on the chunk queue.
 hipError_t launchTileBack(const KArgs& a, const DTiles& T, const DPlanRead& pl,
                           const float* v, float* y, int persistent, hipStream_t st);
+// Whether Siddon forward projections of an image gather from its bricked
+// copy: of 2 M voxels (8 MB) and more, which an XCD's 4 MB L2 does not hold.
+// A smaller image is in L2 anyway, and the bricked walk's extra instructions
+// show: 1 M TOF rays of 96 x 96 x 48 111 us from rows and 140 bricked, of 200
+// x 200 x 128 190 and 163.
+inline bool useBricks(int64_t voxels) { return voxels >= (int64_t(1) << 21); }
 // xb (nt frames of brickFrameVoxels floats) = bricked copy of x (nt frames
 // of the image's voxels), padding voxels 0.
 hipError_t launchToBricks(const DImage& im, const float* x, float* xb, hipStream_t st);
-// v[e] = EM ratio of LOR e (0 where skipped), Siddon or DD (a.pr.type);
-// Siddon reads a.xb (launchToBricks of a.x).
+// v[e] = EM ratio of LOR e (0 where skipped), or with a.plain its projection,
+// Siddon or DD (a.pr.type); Siddon reads a.xb (launchToBricks of a.x) where
+// it is given, else a.x.
 hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st);
 // v[e] = sensitivity value of LOR e (factor x attenuation).
 hipError_t launchSensValue(const KArgs& a, float* v, hipStream_t st);
