@@ -1184,7 +1184,7 @@ int yrtmi_proj_create(yrtmi_ctx* c, const yrtmi_projector_desc* d,
 		q.psf.kSpacing = d->psf_k_spacing;
 		// getHalfWidth_mm (ProjectionPsfManager.cpp:52-56)
 		q.psf.halfWidth = (float)((d->psf_ksize + 1) / 2) * d->psf_k_spacing;
-		const int64_t lds = nkp * (int64_t)sizeof(float) + (int64_t)d->psf_num_s * KC * 8;
+		const int64_t lds = (int64_t)d->psf_num_s * psfSegments((int)K) * (int64_t)sizeof(float4);
 		q.psf.ldsBytes = lds <= kPsfLdsMax ? (int32_t)lds : 0;
 	}
 	p->lpe = (q.numRays >= 4) ? 4 : (q.numRays >= 2 ? 2 : 1);

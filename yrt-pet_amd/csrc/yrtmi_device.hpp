@@ -144,16 +144,20 @@ struct DPsf
 	int32_t numS, K;
 	float sStep, kSpacing, halfWidth;
 	float rks;  // RN(1 / kSpacing)
-	// bytes of one direction's tables (the prefix sums, then the padded
-	// taps) when the DD kernels stage them in LDS, else 0 (too large: they
-	// read them from global memory)
+	// bytes of one direction's segment table (psfSegments float4 per row)
+	// when the DD kernels stage it in LDS, else 0 (too large: they read the
+	// tables above from global memory)
 	int32_t ldsBytes;
 };
+
+// Segments of a row's interpolant: from each tap, -1 and K - 1 included, to
+// the next.
+__host__ __device__ constexpr int psfSegments(int K) { return K + 1; }
 
 // Row stride of DPsf::k and DPsf::kflip.
 __host__ __device__ constexpr int psfRowTaps(int K) { return K + 4; }
 // LDS tables of at most this many bytes are staged.
-constexpr int kPsfLdsMax = 16384;
+constexpr int kPsfLdsMax = 21504;
 
 struct DProj
 {
@@ -510,6 +514,42 @@ __device__ __forceinline__ float psfWeight(const DPsf& P, const float* kp, const
 			out += (float)(cb - ca);
 	}
 	return out;
+}
+
+// psfWeight from the row's segment table: segment s (from tap s - 1) holds
+// {the integral up to it (FP64, two words), ks tap(s - 1), ks (tap(s) -
+// tap(s - 1)) / 2}, so the integral up to x = (s - 1 - half + f) ks is c + f
+// (a + f h): one 16-byte read an end, and 30 VALU an integral where the
+// trapezoids at both ends and the clamps of six reads took ~50.  x / ks is the
+// correctly rounded quotient, as in psfWeight; whole segments are summed in
+// FP64, the parts of the end segments in FP32.
+__device__ __forceinline__ void psfSegment(const float* kp, const double* cum, float ks, int s,
+                                           float4* out)
+{
+	const double c = cum[s];
+	const float a = kp[s + 1], b = kp[s + 2];
+	const unsigned long long u = __builtin_bit_cast(unsigned long long, c);
+	*out = make_float4(__uint_as_float((uint32_t)u), __uint_as_float((uint32_t)(u >> 32)), ks * a,
+	                   0.5f * ks * (b - a));
+}
+
+__device__ __forceinline__ float psfWeightTab(const DPsf& P, const float4* tab, float x0, float x1)
+{
+#pragma clang fp contract(off)
+	const int half = (P.K - 1) / 2;
+	const float lim = (float)(half + 1);
+	auto end = [&](float x, double& c) {
+		const float q = fminf(fmaxf(divByRecip(x, P.kSpacing, P.rks), -lim), lim);
+		const float s = fminf(floorf(q), (float)half);
+		const float f = q - s;
+		const float4 e = tab[(int)s + half + 1];
+		c = __builtin_bit_cast(double, ((unsigned long long)__float_as_uint(e.y) << 32) |
+		                                   (unsigned long long)__float_as_uint(e.x));
+		return f * fmaf(f, e.w, e.z);
+	};
+	double c0, c1;
+	const float p0 = end(x0, c0), p1 = end(x1, c1);
+	return x0 < x1 ? (float)(c1 - c0) + (p1 - p0) : 0.f;
 }
 
 }  // namespace yrtmi

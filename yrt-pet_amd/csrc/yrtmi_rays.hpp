@@ -942,6 +942,7 @@ struct DDRay
 	int psfRow;         // row of the PSF table for this LOR
 	const float* pk;    // PSF taps, padded (flipped for backprojection)
 	const double* pcum; // the row's trapezoid prefix sums (flipped likewise)
+	const float4* ptab; // the row's segments in LDS (TAB sweeps only)
 	float ext, d_norm, d1_i, d2_i;
 	// reciprocals of the slice-invariant denominators of ddSlice: the
 	// footprint edges' (a_xy_lo, a_xy_hi, a_z_lo, a_z_hi) and the TOF slab's
@@ -1413,7 +1414,8 @@ constexpr int DD_ZW = 4;
 // PRE: xv = img[io], the loads of a minor-axis voxel's z planes issued
 // before its weight is computed (the PSF integral then covers their
 // latency); else xv = 0.
-template <bool TOF, bool PRE, class Fn>
+// TAB: the PSF integrals from the row's segments in LDS (R.ptab).
+template <bool TOF, bool PRE, bool TAB, class Fn>
 __device__ __forceinline__ void ddVisitX(const DImage& P, const DDRay& R, const DProj& pr,
                                          int xlo, int xhi, int ylo, int yhi, int zlo, int zhi,
                                          const float* __restrict__ img, Fn&& fn)
@@ -1462,9 +1464,12 @@ __device__ __forceinline__ void ddVisitX(const DImage& P, const DDRay& R, const 
 			for (int j = 0; j < DD_ZW; j++)
 				xv[j] = (PRE && nzv <= DD_ZW && ((zmask >> j) & 1u)) ? img[(zi0 + j) * P.nxy + ib]
 				                                                      : 0.f;
-			const float wxy =
-			    R.usePsf ? psfWeight(pr.psf, R.pk, R.pcum, p0 - q.r1ov, p1 - q.r0ov)
-			             : (fminf(p1, q.r1ov) - fmaxf(p0, q.r0ov));
+			float wxy;
+			if constexpr (TAB)
+				wxy = psfWeightTab(pr.psf, R.ptab, p0 - q.r1ov, p1 - q.r0ov);
+			else
+				wxy = R.usePsf ? psfWeight(pr.psf, R.pk, R.pcum, p0 - q.r1ov, p1 - q.r0ov)
+				               : (fminf(p1, q.r1ov) - fmaxf(p0, q.r0ov));
 			const float wxy_s = ddDivW(wxy, q.widthFrac_yx, ry, oky);
 			if (nzv <= DD_ZW)
 			{
@@ -1503,12 +1508,12 @@ __device__ __forceinline__ void ddVisitX(const DImage& P, const DDRay& R, const 
 }
 
 // ddVisitX without the image loads: fn(io, xyi, yxi, zi, w).
-template <bool TOF, class Fn>
+template <bool TOF, bool TAB = false, class Fn>
 __device__ __forceinline__ void ddVisit(const DImage& P, const DDRay& R, const DProj& pr,
                                         int xlo, int xhi, int ylo, int yhi, int zlo, int zhi,
                                         Fn&& fn)
 {
-	ddVisitX<TOF, false>(P, R, pr, xlo, xhi, ylo, yhi, zlo, zhi, nullptr,
+	ddVisitX<TOF, false, TAB>(P, R, pr, xlo, xhi, ylo, yhi, zlo, zhi, nullptr,
 	                     [&](int io, int xyi, int yxi, int zi, float w, float) {
 		                     fn(io, xyi, yxi, zi, w);
 	                     });
@@ -1516,12 +1521,12 @@ __device__ __forceinline__ void ddVisit(const DImage& P, const DDRay& R, const D
 
 // Forward sweep of a set-up DD LOR over the whole image: the sum of w * x
 // in the sweep's voxel order.
-template <bool TOF>
+template <bool TOF, bool TAB = false>
 __device__ __forceinline__ float ddSweepFwd(const DImage& P, const float* __restrict__ img,
                                             const DDRay& R, const DProj& pr)
 {
 	float acc = 0.f;
-	ddVisitX<TOF, true>(P, R, pr, 0, 1 << 30, 0, 1 << 30, 0, 1 << 30, img,
+	ddVisitX<TOF, true, TAB>(P, R, pr, 0, 1 << 30, 0, 1 << 30, 0, 1 << 30, img,
 	                    [&](int, int, int, int, float w, float xv) { acc = fmaf(w, xv, acc); });
 	return acc;
 }

@@ -494,33 +494,31 @@ hipError_t launchChunkSort(bool dd, const DPlan& pl, const TileChunk* chunks, in
 // DD records (DD = true) hold the LOR alone: its table entry (ddEntry) is set
 // up (ddSetup) and its footprint swept over the slices, minor-axis voxels and
 // z planes of the tile (ddVisit), the voxel weights exactly those of the
-// direct sweep.  A voxel again takes one contribution per record.
-// The projector's PSF tables of one direction (flip: the backprojection's),
-// the prefix sums then the padded taps, copied into the workgroup's dynamic
-// LDS (DPsf::ldsBytes, given by the DD kernels' launches) by all its
-// threads; the caller waits at a barrier before reading them.  Returns the
-// LDS prefix sums, or null when the tables stay in global memory.
-__device__ __forceinline__ const double* psfStage(const DPsf& P, bool flip, double* l)
+// direct sweep.  A footprint's weights have no bound of a few instructions, so
+// DD tiles are summed in FP64 (ds_add_f64: any term, no scale, sums good to
+// 2^-53, rounded once at the flush): the per-term range test and its global
+// atomic, in fixed point, cost more than the slower LDS add (4 M bins of 16
+// frames at 128 x 128 x 96, projection PSF: 28.2 -> 14.1 ms, with the PSF
+// segment table 34.5 before).  Siddon, with more adds an instruction, loses
+// by it: 6.0 -> 7.5 ms for 10 M TOF LORs x 4 rays.
+// The projector's PSF segment tables of one direction (flip: the
+// backprojection's), made in the workgroup's dynamic LDS (DPsf::ldsBytes,
+// given by the DD kernels' launches) by all its threads; the caller waits at
+// a barrier before reading them.  Returns the LDS tables, or null when the
+// projector's stay in global memory.
+__device__ __forceinline__ const float4* psfStage(const DPsf& P, bool flip, float4* l)
 {
 	if (P.ldsBytes == 0)
 		return nullptr;
-	const int nc = P.numS * (P.K + 2), nk = P.numS * psfRowTaps(P.K);
+	const int ns = psfSegments(P.K);
 	const double* c = flip ? P.cumFlip : P.cum;
 	const float* k = flip ? P.kflip : P.k;
-	for (int i = threadIdx.x; i < nc; i += blockDim.x)
-		l[i] = c[i];
-	float* lk = reinterpret_cast<float*>(l + nc);
-	for (int i = threadIdx.x; i < nk; i += blockDim.x)
-		lk[i] = k[i];
+	for (int i = threadIdx.x; i < P.numS * ns; i += blockDim.x)
+	{
+		const int row = i / ns;
+		psfSegment(k + row * psfRowTaps(P.K), c + row * (P.K + 2), P.kSpacing, i - row * ns, l + i);
+	}
 	return l;
-}
-
-// A DD ray's PSF rows pointed at the staged tables.
-__device__ __forceinline__ void psfRowsLds(const DPsf& P, const double* lc, DDRay& D)
-{
-	const float* lk = reinterpret_cast<const float*>(lc + P.numS * (P.K + 2));
-	D.pcum = lc + D.psfRow * (P.K + 2);
-	D.pk = lk + D.psfRow * psfRowTaps(P.K);
 }
 
 template <bool DD, bool TOF, bool S64, int SHAPE>
@@ -528,7 +526,7 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
                                           const DPlanRead& pl, const TileChunk ch,
                                           const float* __restrict__ v,
                                           float* __restrict__ y, unsigned long long* acc64,
-                                          const double* psfL)
+                                          const float4* psfL)
 {
 	float* acc = reinterpret_cast<float*>(acc64);
 	constexpr int TX = tileDim(SHAPE, 0), TY = tileDim(SHAPE, 1), TZ = tileDim(SHAPE, 2);
@@ -560,17 +558,13 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 	// fixed-point scale of this chunk (uniform)
 	int fixed = 0, k = 0;
 	float climit = 0.f, wbound = 0.f;
-	if constexpr (SHAPE != 2)
+	if constexpr (SHAPE != 2 && !DD)
 	{
 		if (pl.vexp != nullptr)
 		{
-			// largest voxel weight: a Siddon segment is at most the voxel
-			// diagonal; a DD weight is at most the slice width over the cosine
-			// of the LOR to the major axis (taken as up to 1/4 here: a larger
-			// weight only takes the global-atomic path)
-			float wmax = DD ? 4.f * fmaxf(a.im.vx, a.im.vy)
-			                : 1.01f * sqrtf(a.im.vx * a.im.vx + a.im.vy * a.im.vy +
-			                                a.im.vz * a.im.vz);
+			// largest voxel weight: a segment is at most the voxel diagonal
+			float wmax = 1.01f * sqrtf(a.im.vx * a.im.vx + a.im.vy * a.im.vy +
+			                           a.im.vz * a.im.vz);
 			if (TOF)
 				wmax *= 1.01f * a.pr.tof.norm;
 			int ew = 0;
@@ -749,8 +743,9 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 				if (xyi >= (D.flag_y ? B.y1 : B.x1))
 					continue;
 				const int ylo = D.flag_y ? B.x0 : B.y0, yhi = (D.flag_y ? B.x1 : B.y1) - 1;
-				auto sweep = [&](const DDRay& Q) {
-					ddVisit<TOF>(a.im, Q, a.pr, xyi, xyi, ylo, yhi, B.z0, B.z1 - 1,
+				auto sweep = [&](const DDRay& Q, auto tab) {
+					ddVisit<TOF, decltype(tab)::value>(
+					             a.im, Q, a.pr, xyi, xyi, ylo, yhi, B.z0, B.z1 - 1,
 					             [&](int, int xs, int yxi, int zi, float w) {
 						             const int gx = Q.flag_y ? yxi : xs,
 						                       gy = Q.flag_y ? xs : yxi;
@@ -758,14 +753,14 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 						                 gx, gy, zi, val * w);
 					             });
 				};
-				// (two copies of the sweep: one reads the PSF rows from LDS)
+				// (two copies of the sweep: one reads the PSF segments from LDS)
 				if (psfL != nullptr)
 				{
-					psfRowsLds(a.pr.psf, psfL, D);
-					sweep(D);
+					D.ptab = psfL + D.psfRow * psfSegments(a.pr.psf.K);
+					sweep(D, std::true_type{});
 				}
 				else
-					sweep(D);
+					sweep(D, std::false_type{});
 			}
 		}
 	};
@@ -801,7 +796,18 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 	const double scale = ldexp(1.0, k);
 	constexpr double kBias = 6755399441055744.0;  // 1.5 * 2^52
 	constexpr unsigned long long kBiasBits = 0x4338000000000000ull;
-	if (fixed)
+	if constexpr (DD && SHAPE != 2)
+	{
+		// DD: FP64 sums
+		wordBytes(8);
+		auto addD = [&](uint32_t idx, int, int, int, float c) {
+			__hip_atomic_fetch_add(
+			    reinterpret_cast<double*>(reinterpret_cast<char*>(acc64) + idx), (double)c,
+			    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+		};
+		pipeline(addD, addD, std::integral_constant<bool, false>{});
+	}
+	else if (fixed)
 	{
 		wordBytes(8);
 		auto addFixed = [&](uint32_t idx, float c) {
@@ -817,7 +823,7 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 				    unsafeAtomicAdd(yf + (int64_t)gz * a.im.nxy + (int64_t)gy * a.im.nx + gx, c);
 		    },
 		    [&](uint32_t idx, int, int, int, float c) { addFixed(idx, c); },
-		    std::integral_constant<bool, !DD>{});
+		    std::true_type{});
 	}
 	else
 	{
@@ -832,7 +838,11 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 	{
 		const int lx = i % TX, ly = (i / TX) % TY, lz = i / (TX * TY);
 		const int gx = B.x0 + lx, gy = B.y0 + ly, gz = B.z0 + lz;
-		const float s = fixed ? ldexpf((float)(long long)acc64[i], -k) : acc[i];
+		float s;
+		if constexpr (DD && SHAPE != 2)
+			s = (float)__longlong_as_double((long long)acc64[i]);
+		else
+			s = fixed ? ldexpf((float)(long long)acc64[i], -k) : acc[i];
 		if (s != 0.f && gx < B.x1 && gy < B.y1 && gz < B.z1)
 			unsafeAtomicAdd(yf + (int64_t)gz * a.im.nxy + (int64_t)gy * a.im.nx + gx, s);
 	}
@@ -850,8 +860,8 @@ __global__ void __launch_bounds__(tileThreads(SHAPE))
 	// NV 64-bit words (fixed point), or NV floats for the 32^3 shape
 	constexpr int NV = tileDim(SHAPE, 0) * tileDim(SHAPE, 1) * tileDim(SHAPE, 2);
 	__shared__ unsigned long long acc[SHAPE == 2 ? NV / 2 : NV];
-	extern __shared__ double psfLds[];
-	const double* psfL = nullptr;
+	extern __shared__ float4 psfLds[];
+	const float4* psfL = nullptr;
 	if constexpr (DD)
 	{
 		psfL = psfStage(a.pr.psf, true, psfLds);
@@ -985,8 +995,8 @@ kEmRatio(KArgs a, float* __restrict__ v)
 template <bool TOF, bool S64, bool TAB>
 __global__ void __launch_bounds__(256) kEmRatioDD(KArgs a, float* __restrict__ v)
 {
-	extern __shared__ double psfLds[];
-	const double* psfL = psfStage(a.pr.psf, false, psfLds);
+	extern __shared__ float4 psfLds[];
+	const float4* psfL = psfStage(a.pr.psf, false, psfLds);
 	__syncthreads();
 	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
 	for (int64_t e = xcdRange(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; e < a.L.n;
@@ -1028,12 +1038,12 @@ __global__ void __launch_bounds__(256) kEmRatioDD(KArgs a, float* __restrict__ v
 				ddSetup<TOF, S64>(a.im, d1, d2, l.n1, l.n2, a.pr, l.tof, false, D);
 			}
 			const float* img = a.x + (int64_t)frame * a.im.nvox;
-			// (two copies of the sweep: one reads the PSF rows from LDS)
+			// (two copies of the sweep: one reads the PSF segments from LDS)
 			float s;
 			if (psfL != nullptr)
 			{
-				psfRowsLds(a.pr.psf, psfL, D);
-				s = ddSweepFwd<TOF>(a.im, img, D, a.pr);
+				D.ptab = psfL + D.psfRow * psfSegments(a.pr.psf.K);
+				s = ddSweepFwd<TOF, true>(a.im, img, D, a.pr);
 			}
 			else
 				s = ddSweepFwd<TOF>(a.im, img, D, a.pr);
@@ -1379,7 +1389,7 @@ hipError_t launchTileBack(const KArgs& a, const DTiles& T, const DPlanRead& pl,
 {
 	if (pl.nChunks <= 0 && pl.nChunksDev == nullptr)
 		return hipSuccess;
-	if (pl.vexp != nullptr)
+	if (pl.vexp != nullptr && a.pr.type != 1 && T.shape != 2)
 	{
 		// the scale word is followed by the finished-workgroups counter and
 		// the 256-bin exponent histogram

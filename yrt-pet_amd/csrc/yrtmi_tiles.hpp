@@ -10,7 +10,7 @@ namespace yrtmi
 {
 
 // Image tiles held in LDS by one workgroup, by shape (64-bit fixed-point
-// voxels, FP32 for shape 2):
+// voxels, DD FP64, FP32 for shape 2):
 //   0: 16 x 16 x 16 (32 KB, 256 threads)   1: 32 x 32 x 16 (128 KB, 512)
 //   2: 32 x 32 x 32 (128 KB FP32, 1024)    3: 32 x 32 x 8 (64 KB, 512)
 constexpr int kNumTileShapes = 4;
