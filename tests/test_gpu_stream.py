@@ -186,3 +186,31 @@ def test_bricked_forward_is_the_forward(gpu, kw):
         ctx.forward(p, im, x, L, y)
         torch.cuda.synchronize()
         assert torch.equal(y, z)
+
+
+@pytest.mark.parametrize("kw", [dict(proj="DD", psf=True), dict(proj="DD", tof=300.0, frames=2),
+                                dict(proj="DD", fp64=True)], ids=str)
+def test_bricked_dd_ratio_is_the_ratio(gpu, kw):
+    """EM ratios of a large image, from its bricked copy, against those of a
+    recording made before there is a buffer for it (from rows): the same sums,
+    bit for bit; and from two streams in turn."""
+    nt = max(1, kw.get("frames", 0))
+    im = yrtmi.ImageParams(161, 127, 103, 1.5, 1.75, 1.0, nt=nt)
+    ctx, p, L, _ = setup(im, 30_000, gpu=gpu, **kw)
+    x = 0.5 + torch.rand(im.shape, device=gpu, generator=torch.Generator(gpu).manual_seed(2))
+    x2 = 2.0 * x
+    y, z, w = (torch.zeros(L.n, device=gpu) for _ in range(3))
+    s, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    ctx.set_stream(s)
+    with ctx.graph() as g:
+        ctx.em_ratio(p, im, x, L, y)
+    g.launch()
+    for k in range(3):
+        ctx.set_stream(s2)
+        ctx.em_ratio(p, im, x2, L, w)
+        ctx.set_stream(s)
+        ctx.em_ratio(p, im, x, L, z)
+        torch.cuda.synchronize()
+        assert float(y.abs().sum()) > 0 and torch.equal(y, z)
+        assert torch.allclose(w, 0.5 * y, rtol=1e-6, atol=0)

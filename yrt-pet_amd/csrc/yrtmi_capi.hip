@@ -86,9 +86,7 @@ struct yrtmi_ctx
 	float* part = nullptr;
 	int64_t partStride = 0;
 	int nxcc = 1;
-	// bricked copy of the image the Siddon EM ratio projects, grown on demand
-	float* brick = nullptr;
-	int64_t brickCap = 0;
+	Scratch em;   // the bricked image that EM ratios project
 	Scratch ws;   // of the backprojections binned by tiles without a plan (streamBack)
 	Scratch fwd;  // the bricked image of forward and sensitivity projections
 	hipStream_t owned = nullptr;  // stream created by yrtmi_ctx_own_stream
@@ -293,42 +291,6 @@ int ensurePartials(yrtmi_ctx* c, int64_t n)
 	return YRTMI_OK;
 }
 
-// The buffer of the bricked image the Siddon EM ratio's forward reads, at
-// least `need` floats (grown outside graph recording only; tile plans size
-// it for their image, so planned EM calls never allocate).
-int ensureBrick(yrtmi_ctx* c, int64_t need)
-{
-	if (c->brick == nullptr || c->brickCap < need)
-	{
-		int r = notCapturing(c, "bricked image (run one EM ratio of this size before recording)");
-		if (r)
-			return r;
-		HIP_TRY(hipStreamSynchronize(c->stream));
-		HIP_TRY(hipFree(c->brick));
-		c->brick = nullptr;
-		c->brickCap = 0;
-		HIP_TRY(poolMalloc(c->device, &c->brick, sizeof(float) * need));
-		c->brickCap = need;
-	}
-	return YRTMI_OK;
-}
-
-// The bricked copy of a.x for the Siddon EM ratio's forward; DD, and Siddon on
-// small images, read a.x itself.
-int brickImage(yrtmi_ctx* c, KArgs& a)
-{
-	if (a.pr.type == 1 || !useBricks(a.im.nvox * a.im.nt))
-		return YRTMI_OK;
-	const int64_t bvox = brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz);
-	const int r = ensureBrick(c, bvox * a.im.nt);
-	if (r)
-		return r;
-	HIP_TRY(launchToBricks(a.im, a.x, c->brick, c->stream));
-	a.xb = c->brick;
-	a.bvox = bvox;
-	return YRTMI_OK;
-}
-
 // Before and after a call's use of the scratch.
 int acquire(yrtmi_ctx* c, Scratch& w)
 {
@@ -374,6 +336,35 @@ bool reserve(yrtmi_ctx* c, Scratch& w, size_t bytes)
 	w.p = q;
 	w.bytes = bytes;
 	return true;
+}
+
+// The bricked copy of a.x for the EM ratio's forward; small images are read
+// as they are, and so is a DD call's while recording without the buffer
+// (Siddon refuses that).  The caller releases it after its launch
+// (brickDone).  Tile plans reserve it for their image, so planned EM calls
+// never allocate.
+int brickImage(yrtmi_ctx* c, KArgs& a)
+{
+	if (!useBricks(a.im.nvox * a.im.nt))
+		return YRTMI_OK;
+	const int64_t bvox = brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz);
+	if (!reserve(c, c->em, sizeof(float) * (size_t)(bvox * a.im.nt)))
+		return a.pr.type == YRTMI_PROJ_DD
+		           ? YRTMI_OK
+		           : notCapturing(c,
+		                          "bricked image (run one EM ratio of this size before recording)");
+	const int r = acquire(c, c->em);
+	if (r)
+		return r;
+	HIP_TRY(launchToBricks(a.im, a.x, (float*)c->em.p, c->stream));
+	a.xb = (const float*)c->em.p;
+	a.bvox = bvox;
+	return YRTMI_OK;
+}
+
+int brickDone(yrtmi_ctx* c, const KArgs& a)
+{
+	return a.xb != nullptr ? release(c, c->em) : YRTMI_OK;
 }
 
 constexpr int64_t kBrickRays = 4;  // voxels a ray above which it is not
@@ -448,7 +439,7 @@ struct StreamShape
 	int R = 1;
 	int persistent = 0;  // tile kernel workgroups
 	bool dd = false;
-	int64_t brick = 0;   // floats of the bricked image (EM, Siddon)
+	int64_t brick = 0;   // floats of the bricked image (EM)
 	size_t fixedBytes() const
 	{
 		return sizeof(StreamState) + (size_t)nB * 20 + (size_t)kStreamBinGroups * nB * 4 +
@@ -489,7 +480,7 @@ bool streamShape(yrtmi_ctx* c, const KArgs& a, bool em, StreamShape& s)
 	// records are not bounded so (a batch of more takes the direct kernel)
 	s.recPer = s.dd ? std::min<int64_t>(128, 8 * std::max(s.T.ntx, s.T.nty))
 	                : std::min<int64_t>(64, s.T.ntx + s.T.nty + s.T.ntz - 2);
-	s.brick = (em && !s.dd && useBricks(a.im.nvox * a.im.nt)) ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt : 0;
+	s.brick = (em && useBricks(a.im.nvox * a.im.nt)) ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt : 0;
 	return true;
 }
 
@@ -747,8 +738,7 @@ int yrtmi_ctx_destroy(yrtmi_ctx* c)
 	(void)hipFree(c->gatherErr);
 	(void)hipFree(c->counter);
 	(void)hipFree(c->part);
-	(void)hipFree(c->brick);
-	for (Scratch* w : {&c->ws, &c->fwd})
+	for (Scratch* w : {&c->em, &c->ws, &c->fwd})
 	{
 		if (w->p != nullptr)
 		{
@@ -838,11 +828,11 @@ int yrtmi_graph_launch(yrtmi_ctx* c, const yrtmi_graph* g)
 	r = notCapturing(c, "graph_launch");
 	if (r)
 		return r;
-	for (Scratch* w : {&c->ws, &c->fwd})
+	for (Scratch* w : {&c->em, &c->ws, &c->fwd})
 		if (w->captured && (r = acquire(c, *w)) != YRTMI_OK)
 			return r;
 	HIP_TRY(hipGraphLaunch(g->exec, c->stream));
-	for (Scratch* w : {&c->ws, &c->fwd})
+	for (Scratch* w : {&c->em, &c->ws, &c->fwd})
 		if (w->captured && (r = release(c, *w)) != YRTMI_OK)
 			return r;
 	return YRTMI_OK;
@@ -1923,12 +1913,13 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	const bool dd = p->d.type == YRTMI_PROJ_DD;
 	if (im->nx > 1024 || im->ny > 1024 || im->nz > 1024)
 		return fail(YRTMI_EINVAL, "plan: image dimensions above 1024");
-	if (!dd && useBricks(a.im.nvox * a.im.nt))
+	if (useBricks(a.im.nvox * a.im.nt))
 	{
 		// the bricked image of the planned EM ratio, sized here
-		r = ensureBrick(c, brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt);
-		if (r)
-			return r;
+		if (!reserve(c, c->em,
+		             sizeof(float) *
+		                 (size_t)(brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt)))
+			return fail(YRTMI_ENOMEM, "plan: bricked image");
 	}
 	const int R = p->d.numRays;
 	if ((l->n * (int64_t)R) >= (int64_t(1) << 32))
@@ -2239,7 +2230,7 @@ int yrtmi_em_ratio(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	if (r)
 		return r;
 	HIP_TRY(launchEmRatio(a, p->lpe, v, c->stream));
-	return YRTMI_OK;
+	return brickDone(c, a);
 }
 
 int yrtmi_em_ratio_planned(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
@@ -2264,7 +2255,7 @@ int yrtmi_em_ratio_planned(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image*
 	if (r)
 		return r;
 	HIP_TRY(launchEmRatio(a, p->lpe, v, c->stream));
-	return YRTMI_OK;
+	return brickDone(c, a);
 }
 
 int yrtmi_em_subset_planned(yrtmi_ctx* c, const yrtmi_proj* p,
@@ -2290,6 +2281,9 @@ int yrtmi_em_subset_planned(yrtmi_ctx* c, const yrtmi_proj* p,
 	if (r)
 		return r;
 	HIP_TRY(launchEmRatio(a, p->lpe, q->v, c->stream));
+	r = brickDone(c, a);
+	if (r)
+		return r;
 	HIP_TRY(launchTileBack(a, q->T, planRead(q), q->v, u, q->persistent, c->stream));
 	return YRTMI_OK;
 }
@@ -2688,6 +2682,9 @@ int yrtmi_autotune(yrtmi_ctx* c, yrtmi_proj* p, const yrtmi_image* im,
 		}
 	}
 	p->lpe = best->lanes_per_event;
+	r = brickDone(c, a);
+	if (r)
+		return done(r);
 	// v now holds the EM ratios of x: backproject them through each shape
 	best->back_ms = 1e30f;
 	for (int shape = 0; shape < kNumTileShapes; shape++)

@@ -1415,7 +1415,8 @@ constexpr int DD_ZW = 4;
 // before its weight is computed (the PSF integral then covers their
 // latency); else xv = 0.
 // TAB: the PSF integrals from the row's segments in LDS (R.ptab).
-template <bool TOF, bool PRE, bool TAB, class Fn>
+// BRICK (with PRE): img is the frame's bricked copy (brickIndex).
+template <bool TOF, bool PRE, bool TAB, bool BRICK, class Fn>
 __device__ __forceinline__ void ddVisitX(const DImage& P, const DDRay& R, const DProj& pr,
                                          int xlo, int xhi, int ylo, int yhi, int zlo, int zhi,
                                          const float* __restrict__ img, Fn&& fn)
@@ -1437,6 +1438,13 @@ __device__ __forceinline__ void ddVisitX(const DImage& P, const DDRay& R, const 
 		// footprint overlaps
 		float wz[DD_ZW];
 		uint32_t zmask = 0u;
+		// offset of each plane in the frame or its bricked copy
+		auto zOffset = [&](int zi) {
+			if constexpr (BRICK)
+				return (zi >> 1) * (brickNx(P.nx) * brickNy(P.ny) * 32) + ((zi & 1) << 4);
+			else
+				return zi * P.nxy;
+		};
 		if (nzv <= DD_ZW)
 		{
 #pragma unroll
@@ -1459,10 +1467,16 @@ __device__ __forceinline__ void ddVisitX(const DImage& P, const DDRay& R, const 
 			if (!(q.r1 >= p0 && q.r0 < p1))
 				continue;
 			const int ib = xyi * R.strideXY + yxi * R.strideYX;
+			int im = ib;
+			if constexpr (BRICK)
+			{
+				const int x = R.flag_y ? yxi : xyi, y = R.flag_y ? xyi : yxi;
+				im = ((y >> 2) * brickNx(P.nx) + (x >> 2)) * 32 + ((y & 3) << 2) + (x & 3);
+			}
 			float xv[DD_ZW];
 #pragma unroll
 			for (int j = 0; j < DD_ZW; j++)
-				xv[j] = (PRE && nzv <= DD_ZW && ((zmask >> j) & 1u)) ? img[(zi0 + j) * P.nxy + ib]
+				xv[j] = (PRE && nzv <= DD_ZW && ((zmask >> j) & 1u)) ? img[zOffset(zi0 + j) + im]
 				                                                      : 0.f;
 			float wxy;
 			if constexpr (TAB)
@@ -1500,7 +1514,7 @@ __device__ __forceinline__ void ddVisitX(const DImage& P, const DDRay& R, const 
 					if (TOF)
 						w *= q.tw;
 					const int io = zi * P.nxy + ib;
-					fn(io, xyi, yxi, zi, w, PRE ? img[io] : 0.f);
+					fn(io, xyi, yxi, zi, w, PRE ? img[zOffset(zi) + im] : 0.f);
 				}
 			}
 		}
@@ -1513,7 +1527,7 @@ __device__ __forceinline__ void ddVisit(const DImage& P, const DDRay& R, const D
                                         int xlo, int xhi, int ylo, int yhi, int zlo, int zhi,
                                         Fn&& fn)
 {
-	ddVisitX<TOF, false, TAB>(P, R, pr, xlo, xhi, ylo, yhi, zlo, zhi, nullptr,
+	ddVisitX<TOF, false, TAB, false>(P, R, pr, xlo, xhi, ylo, yhi, zlo, zhi, nullptr,
 	                     [&](int io, int xyi, int yxi, int zi, float w, float) {
 		                     fn(io, xyi, yxi, zi, w);
 	                     });
@@ -1521,12 +1535,12 @@ __device__ __forceinline__ void ddVisit(const DImage& P, const DDRay& R, const D
 
 // Forward sweep of a set-up DD LOR over the whole image: the sum of w * x
 // in the sweep's voxel order.
-template <bool TOF, bool TAB = false>
+template <bool TOF, bool TAB = false, bool BRICK = false>
 __device__ __forceinline__ float ddSweepFwd(const DImage& P, const float* __restrict__ img,
                                             const DDRay& R, const DProj& pr)
 {
 	float acc = 0.f;
-	ddVisitX<TOF, true, TAB>(P, R, pr, 0, 1 << 30, 0, 1 << 30, 0, 1 << 30, img,
+	ddVisitX<TOF, true, TAB, BRICK>(P, R, pr, 0, 1 << 30, 0, 1 << 30, 0, 1 << 30, img,
 	                    [&](int, int, int, int, float w, float xv) { acc = fmaf(w, xv, acc); });
 	return acc;
 }

@@ -991,8 +991,11 @@ kEmRatio(KArgs a, float* __restrict__ v)
 }
 
 // DD: one lane per LOR, its set-up read from the plan's table (TAB) or made
-// from the resolved LOR.
-template <bool TOF, bool S64, bool TAB>
+// from the resolved LOR.  BRICK: gathers from the bricked copy of x, as the
+// Siddon forward: a brick serves 4 slices of the sweep whichever the major
+// axis, where rows along x serve one of y (4 M bins of 16 frames at 128 x 128 x 96:
+// 15.8 -> 12.1 ms).
+template <bool TOF, bool S64, bool TAB, bool BRICK>
 __global__ void __launch_bounds__(256) kEmRatioDD(KArgs a, float* __restrict__ v)
 {
 	extern __shared__ float4 psfLds[];
@@ -1037,16 +1040,17 @@ __global__ void __launch_bounds__(256) kEmRatioDD(KArgs a, float* __restrict__ v
 				const float3 d2 = make_float3(l.p2.x - a.im.ox, l.p2.y - a.im.oy, l.p2.z - a.im.oz);
 				ddSetup<TOF, S64>(a.im, d1, d2, l.n1, l.n2, a.pr, l.tof, false, D);
 			}
-			const float* img = a.x + (int64_t)frame * a.im.nvox;
+			const float* img = BRICK ? a.xb + (int64_t)frame * a.bvox
+			                         : a.x + (int64_t)frame * a.im.nvox;
 			// (two copies of the sweep: one reads the PSF segments from LDS)
 			float s;
 			if (psfL != nullptr)
 			{
 				D.ptab = psfL + D.psfRow * psfSegments(a.pr.psf.K);
-				s = ddSweepFwd<TOF, true>(a.im, img, D, a.pr);
+				s = ddSweepFwd<TOF, true, BRICK>(a.im, img, D, a.pr);
 			}
 			else
-				s = ddSweepFwd<TOF>(a.im, img, D, a.pr);
+				s = ddSweepFwd<TOF, false, BRICK>(a.im, img, D, a.pr);
 			out = emRatioOut(a, e, s, m, sf, af);
 		}
 		v[e] = out;
@@ -1448,10 +1452,13 @@ static hipError_t ratioT(const KArgs& a, int lpe, dim3 g, float* v, hipStream_t 
 {
 	if (a.pr.type == 1)
 	{
-		if (a.rays != nullptr)
-			kEmRatioDD<TOF, S64, true><<<g, 256, a.pr.psf.ldsBytes, st>>>(a, v);
+		auto go = [&](auto k) { k<<<g, 256, a.pr.psf.ldsBytes, st>>>(a, v); };
+		if (a.xb != nullptr)
+			a.rays != nullptr ? go(kEmRatioDD<TOF, S64, true, true>)
+			                  : go(kEmRatioDD<TOF, S64, false, true>);
 		else
-			kEmRatioDD<TOF, S64, false><<<g, 256, a.pr.psf.ldsBytes, st>>>(a, v);
+			a.rays != nullptr ? go(kEmRatioDD<TOF, S64, true, false>)
+			                  : go(kEmRatioDD<TOF, S64, false, false>);
 		return hipGetLastError();
 	}
 	return a.xb != nullptr ? ratioLpe<TOF, S64, true>(a, lpe, g, v, st)
@@ -1488,8 +1495,7 @@ hipError_t launchToBricks(const DImage& im, const float* x, float* xb, hipStream
 
 hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st)
 {
-	if (a.pr.type != 1 && a.xb != nullptr &&
-	    a.bvox != brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz))
+	if (a.xb != nullptr && a.bvox != brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz))
 		return hipErrorInvalidValue;
 	if (a.pr.type == 1)
 		lpe = 1;
