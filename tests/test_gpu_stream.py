@@ -214,3 +214,31 @@ def test_bricked_dd_ratio_is_the_ratio(gpu, kw):
         torch.cuda.synchronize()
         assert float(y.abs().sum()) > 0 and torch.equal(y, z)
         assert torch.allclose(w, 0.5 * y, rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("dims", [(3, 2, 40, 60.0, 60.0, 2.0), (33, 65, 17, 4.0, 4.0, 4.0),
+                                  (161, 127, 103, 1.5, 1.75, 1.0)], ids=str)
+@pytest.mark.parametrize("kw", [dict(), dict(tof=300.0, psf=True), dict(frames=2, fp64=True)],
+                         ids=str)
+def test_dd_forward_lanes(gpu, dims, kw):
+    """DD projections with four lanes per LOR (calls of up to 196608) against
+    one (a call of all; the largest image from bricks), also of 1, 15 and 65 LORs
+    and of images of fewer slices than lanes.  Sums of the same positive terms, some
+    10^3 to 10^4, in two orders: 100 x 6e-8 of rounding."""
+    im = yrtmi.ImageParams(*dims, nt=max(1, kw.get("frames", 0)))
+    n = 540_000 if dims[0] > 100 else 196_609
+    ctx, p, L, _ = setup(im, n, proj="DD", gpu=gpu, **kw)
+    x = 0.5 + torch.rand(im.shape, device=gpu, generator=torch.Generator(gpu).manual_seed(2))
+    y, z = torch.full((n,), -1.0, device=gpu), torch.full((n,), -1.0, device=gpu)
+    ctx.forward(p, im, x, L, y)
+    at = 0
+    for k in (1, 15, 65, 196_527, 196_608, n):
+        b = min(n, at + k)
+        if b > at:
+            ctx.forward(p, im, x, L.slice(at, b), z[at:b])
+        at = b
+    torch.cuda.synchronize()
+    y, z = y.cpu().numpy(), z.cpu().numpy()
+    print(f"lanes rel L2 {rel_l2(z, y):.2e}", flush=True)
+    assert np.abs(y).sum() > 0 and rel_l2(z, y) <= 1e-5
+    assert ((y == 0) == (z == 0)).all()

@@ -369,7 +369,7 @@ int brickDone(yrtmi_ctx* c, const KArgs& a)
 
 constexpr int64_t kBrickRays = 4;  // voxels a ray above which it is not
 
-// A forward projection of `rays` Siddon rays of image `im` reads a bricked
+// A forward projection of `rays` rays of image `im` reads a bricked
 // copy of it (a.xb, in c->fwd), where the copy, ~3 ps
 // a voxel, is worth it: a bricked ray saves ~60 ps of 270 (1 M TOF LORs x 4
 // rays at 200 x 200 x 128: 1.08 -> 0.76 ms).
@@ -379,8 +379,7 @@ bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, in
 {
 	*status = YRTMI_OK;
 	const int64_t bvox = brickFrameVoxels(im.nx, im.ny, im.nz);
-	if (a.pr.type == YRTMI_PROJ_DD || !useBricks(im.nvox * im.nt) ||
-	    rays * kBrickRays < im.nvox * im.nt ||
+	if (!useBricks(im.nvox * im.nt) || rays * kBrickRays < im.nvox * im.nt ||
 	    !reserve(c, c->fwd, sizeof(float) * (size_t)(bvox * im.nt)))
 		return false;
 	*status = acquire(c, c->fwd);
@@ -532,7 +531,6 @@ int sensValue(yrtmi_ctx* c, KArgs a, float* v)
 	int r = YRTMI_OK;
 	a.xb = nullptr;
 	KArgs s = a;
-	s.pr.type = YRTMI_PROJ_SIDDON;  // (attenuation is a Siddon ray's)
 	const bool bricks = a.att != nullptr && brickForward(c, s, a.attIm, a.att, a.L.n, &r);
 	if (r)
 		return r;
@@ -1252,14 +1250,17 @@ int yrtmi_forward(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	if (img == nullptr || out == nullptr)
 		return fail(YRTMI_EINVAL, "forward: null image or output");
 	a.x = img;
-	if (brickForward(c, a, a.im, img, l->n * (int64_t)a.pr.numRays, &r))
+	const bool bricks = brickForward(c, a, a.im, img, l->n * (int64_t)a.pr.numRays, &r);
+	if (r)
+		return r;
+	// (3 M DD LORs of 200 x 200 x 128 from bricks: TOF 4.3 -> 2.7 ms, without
+	// 9.0 -> 5.9; few of them by the lanes per LOR of the ratio's kernel)
+	if (bricks || (a.pr.type == YRTMI_PROJ_DD && l->n <= kDDLanesUpTo))
 	{
 		a.plain = 1;
 		HIP_TRY(launchEmRatio(a, p->lpe, out, c->stream));
-		return release(c, c->fwd);
+		return bricks ? release(c, c->fwd) : YRTMI_OK;
 	}
-	if (r)
-		return r;
 	a.out = out;
 	HIP_TRY(launchEvents(MODE_FWD, a, p->lpe, p->block, p->grid, c->stream));
 	return YRTMI_OK;

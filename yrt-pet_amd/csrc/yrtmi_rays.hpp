@@ -1419,11 +1419,11 @@ constexpr int DD_ZW = 4;
 template <bool TOF, bool PRE, bool TAB, bool BRICK, class Fn>
 __device__ __forceinline__ void ddVisitX(const DImage& P, const DDRay& R, const DProj& pr,
                                          int xlo, int xhi, int ylo, int yhi, int zlo, int zhi,
-                                         const float* __restrict__ img, Fn&& fn)
+                                         const float* __restrict__ img, Fn&& fn, int xstep = 1)
 {
 #pragma clang fp contract(off)
 	const int x0 = max(R.xy_i_0, xlo), x1 = min(R.xy_i_1, xhi);
-	for (int xyi = x0; xyi <= x1; xyi++)
+	for (int xyi = x0; xyi <= x1; xyi += xstep)
 	{
 		DDSlice q;
 		ddSlice<TOF>(P, R, pr, xyi, q);
@@ -1534,14 +1534,16 @@ __device__ __forceinline__ void ddVisit(const DImage& P, const DDRay& R, const D
 }
 
 // Forward sweep of a set-up DD LOR over the whole image: the sum of w * x
-// in the sweep's voxel order.
+// in the sweep's voxel order; with `step` lanes per LOR, lane `first`'s share of
+// its slices.
 template <bool TOF, bool TAB = false, bool BRICK = false>
 __device__ __forceinline__ float ddSweepFwd(const DImage& P, const float* __restrict__ img,
-                                            const DDRay& R, const DProj& pr)
+                                            const DDRay& R, const DProj& pr, int first = 0,
+                                            int step = 1)
 {
 	float acc = 0.f;
-	ddVisitX<TOF, true, TAB, BRICK>(P, R, pr, 0, 1 << 30, 0, 1 << 30, 0, 1 << 30, img,
-	                    [&](int, int, int, int, float w, float xv) { acc = fmaf(w, xv, acc); });
+	ddVisitX<TOF, true, TAB, BRICK>(P, R, pr, max(R.xy_i_0, 0) + first, 1 << 30, 0, 1 << 30, 0, 1 << 30, img,
+	                    [&](int, int, int, int, float w, float xv) { acc = fmaf(w, xv, acc); }, step);
 	return acc;
 }
 

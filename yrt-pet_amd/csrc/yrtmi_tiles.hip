@@ -990,21 +990,26 @@ kEmRatio(KArgs a, float* __restrict__ v)
 	}
 }
 
-// DD: one lane per LOR, its set-up read from the plan's table (TAB) or made
+// DD: LPE lanes per LOR, its set-up read from the plan's table (TAB) or made
 // from the resolved LOR.  BRICK: gathers from the bricked copy of x, as the
 // Siddon forward: a brick serves 4 slices of the sweep whichever the major
 // axis, where rows along x serve one of y (4 M bins of 16 frames at 128 x 128 x 96:
 // 15.8 -> 12.1 ms).
-template <bool TOF, bool S64, bool TAB, bool BRICK>
+// LPE: lanes per LOR, each on every LPE-th slice (a lane per LOR leaves the
+// chip idle in calls of few LORs: the forward of 150 k TOF LORs of 95 x 97 x
+// 47 with a PSF 0.49 -> 0.40 ms); one where there are LORs enough.
+template <bool TOF, bool S64, bool TAB, bool BRICK, int LPE>
 __global__ void __launch_bounds__(256) kEmRatioDD(KArgs a, float* __restrict__ v)
 {
 	extern __shared__ float4 psfLds[];
 	const float4* psfL = psfStage(a.pr.psf, false, psfLds);
 	__syncthreads();
 	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-	for (int64_t e = xcdRange(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; e < a.L.n;
-	     e += stride)
+	for (int64_t t = xcdRange(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; t < a.L.n * LPE;
+	     t += stride)
 	{
+		const int64_t e = t / LPE;
+		const int lane = (int)(t & (LPE - 1));
 		const float m = a.c.meas ? a.c.meas[e] : 1.0f;
 		const float sf = a.c.sens ? a.c.sens[e] : 1.0f;
 		const float af = a.c.att ? a.c.att[e] : 1.0f;
@@ -1022,7 +1027,7 @@ __global__ void __launch_bounds__(256) kEmRatioDD(KArgs a, float* __restrict__ v
 			frame = l.frame;
 		}
 		const bool skip = (m == 0.f || sf == 0.f || af == 0.f || frame < 0);
-		float out = 0.f;
+		float s = 0.f;
 		if (!skip)
 		{
 			DDRay D;
@@ -1043,17 +1048,19 @@ __global__ void __launch_bounds__(256) kEmRatioDD(KArgs a, float* __restrict__ v
 			const float* img = BRICK ? a.xb + (int64_t)frame * a.bvox
 			                         : a.x + (int64_t)frame * a.im.nvox;
 			// (two copies of the sweep: one reads the PSF segments from LDS)
-			float s;
 			if (psfL != nullptr)
 			{
 				D.ptab = psfL + D.psfRow * psfSegments(a.pr.psf.K);
-				s = ddSweepFwd<TOF, true, BRICK>(a.im, img, D, a.pr);
+				s = ddSweepFwd<TOF, true, BRICK>(a.im, img, D, a.pr, lane, LPE);
 			}
 			else
-				s = ddSweepFwd<TOF, false, BRICK>(a.im, img, D, a.pr);
-			out = emRatioOut(a, e, s, m, sf, af);
+				s = ddSweepFwd<TOF, false, BRICK>(a.im, img, D, a.pr, lane, LPE);
 		}
-		v[e] = out;
+#pragma unroll
+		for (int o = 1; o < LPE; o <<= 1)
+			s += __shfl_xor(s, o, LPE);
+		if (lane == 0)
+			v[e] = skip ? 0.f : emRatioOut(a, e, s, m, sf, af);
 	}
 }
 
@@ -1453,12 +1460,16 @@ static hipError_t ratioT(const KArgs& a, int lpe, dim3 g, float* v, hipStream_t 
 	if (a.pr.type == 1)
 	{
 		auto go = [&](auto k) { k<<<g, 256, a.pr.psf.ldsBytes, st>>>(a, v); };
+		auto lanes = [&](auto tab, auto brick) {
+			constexpr bool T = decltype(tab)::value, B = decltype(brick)::value;
+			lpe == 4 ? go(kEmRatioDD<TOF, S64, T, B, 4>) : go(kEmRatioDD<TOF, S64, T, B, 1>);
+		};
+		using Y = std::true_type;
+		using N = std::false_type;
 		if (a.xb != nullptr)
-			a.rays != nullptr ? go(kEmRatioDD<TOF, S64, true, true>)
-			                  : go(kEmRatioDD<TOF, S64, false, true>);
+			a.rays != nullptr ? lanes(Y{}, Y{}) : lanes(N{}, Y{});
 		else
-			a.rays != nullptr ? go(kEmRatioDD<TOF, S64, true, false>)
-			                  : go(kEmRatioDD<TOF, S64, false, false>);
+			a.rays != nullptr ? lanes(Y{}, N{}) : lanes(N{}, N{});
 		return hipGetLastError();
 	}
 	return a.xb != nullptr ? ratioLpe<TOF, S64, true>(a, lpe, g, v, st)
@@ -1498,7 +1509,7 @@ hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st)
 	if (a.xb != nullptr && a.bvox != brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz))
 		return hipErrorInvalidValue;
 	if (a.pr.type == 1)
-		lpe = 1;
+		lpe = a.L.n <= kDDLanesUpTo ? 4 : 1;
 	const int64_t threads = a.L.n * lpe;
 	int64_t nb = (threads + 255) / 256;
 	if (nb > 0x7ffffff0)

@@ -224,6 +224,12 @@ hipError_t launchClearWords(unsigned int* p, int64_t words, hipStream_t st);
 hipError_t launchStreamScan(const DPlan& pl, int64_t* tileOff, int nTiles, int64_t cap,
                             TileChunk* chunks, StreamState* s, hipStream_t st);
 
+// LORs up to which a DD forward takes four lanes per LOR (3 waves for each of
+// the chip's 1024 SIMDs at one).  96 x 96 x 48, four lanes against one: 65536
+// LORs 94 / 172 us, 196608 205 / 212, 262144 260 / 254; 200 x 200 x 128 TOF:
+// 116 / 220, 252 / 302, 336 / 425.
+constexpr int64_t kDDLanesUpTo = 196608;
+
 // LDS of the fill pass: an int counter and a 32-bit base per bin.
 inline size_t binLdsBytes(int nB)
 {
