@@ -1254,8 +1254,10 @@ int yrtmi_forward(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	if (r)
 		return r;
 	// (3 M DD LORs of 200 x 200 x 128 from bricks: TOF 4.3 -> 2.7 ms, without
-	// 9.0 -> 5.9; few of them by the lanes per LOR of the ratio's kernel)
-	if (bricks || (a.pr.type == YRTMI_PROJ_DD && l->n <= kDDLanesUpTo))
+	// 9.0 -> 5.9; few LORs by the ratio's kernel for its lanes per LOR or ray)
+	if (bricks ||
+	    (a.pr.type == YRTMI_PROJ_DD ? l->n <= kDDLanesUpTo
+	                                : !a.pr.setup64 && l->n * (int64_t)a.pr.numRays <= kSplitRays))
 	{
 		a.plain = 1;
 		HIP_TRY(launchEmRatio(a, p->lpe, out, c->stream));

@@ -469,6 +469,75 @@ __device__ __forceinline__ bool sidPlaneShift(const DImage& P, const SidRay& r, 
 	return sidFirst<S64>(P, r, vx, vy, vz, dx, dy, dz);
 }
 
+// One axis of an FP32 ray in plane numbers, as sidPieces and sidPart cut it
+// (kept as floats, exact to 2^24)
+struct SidAxis
+{
+	float start, sv, p, inv;  // plane q: (start + q sv - p) inv
+	float gs, g0;             // planes passed at alpha m: gs m + g0
+	float k, kt, kend;        // next plane, the tile's face, the image's
+	float dirf, off;          // voxel whose far face is plane q: dirf q + off
+	float T;
+	__device__ __forceinline__ float plane(float q) const
+	{
+#pragma clang fp contract(off)
+		const float c = start + q * sv;
+		return (c - p) * inv;
+	}
+	__device__ __forceinline__ int voxel(float q) const { return (int)(q * dirf + off); }
+	// the first plane after alpha m, from plane k on (at: the alpha of
+	// the tile's face, which is passed if not after m: every round of
+	// the loop leaves a tile, whatever the numbers)
+	__device__ __forceinline__ float after(float m, float at, bool coarse) const
+	{
+#pragma clang fp contract(off)
+		float q = fminf(fmaxf(floorf(fmaf(m, gs, g0)) + 1.f, k), kt + 1.f);
+		const float lo = plane(q - 1.f), hi = plane(q);
+		q += (hi <= m) ? 1.f : ((lo > m && q > k) ? -1.f : 0.f);
+		if (coarse)
+		{
+			while (q > k && plane(q - 1.f) > m)
+				q -= 1.f;
+			while (q < kend + 16.f && plane(q) <= m)
+				q += 1.f;
+		}
+		return (at <= m) ? fmaxf(q, kt + 1.f) : q;
+	}
+};
+
+__device__ __forceinline__ SidAxis sidAxis(float len, float v, float p1, float p2, float inv,
+                                           int dir, int n, int l, int sh, int vox)
+{
+#pragma clang fp contract(off)
+	const float FMAX = 3.402823466e+38f;
+	SidAxis a;
+	const bool flat = p1 == p2;
+	const float rv = (dir > 0) ? 1.0f / v : -1.0f / v;
+	a.start = (dir > 0) ? -len * 0.5f : len * 0.5f;
+	a.sv = (float)dir * v;
+	a.p = flat ? -FMAX : p1;
+	a.inv = flat ? 1.f : inv;
+	a.k = (float)(((dir > 0) ? vox + 1 : n - vox) + sh);
+	a.gs = (p2 - p1) * rv;
+	a.g0 = flat ? a.k - 1.f : (p1 - a.start) * rv;
+	const int t = vox >> l;
+	a.kt = (float)((dir > 0 ? min((t + 1) << l, n) : n - (t << l)) + sh);
+	a.kend = (float)(n + sh);
+	a.dirf = (float)dir;
+	a.off = (float)(dir > 0 ? -1 - sh : n + sh);
+	a.T = (float)(1 << l);
+	return a;
+}
+
+// Voxels below a millionth of the scanner: a position may be planes off.
+__device__ __forceinline__ bool sidCoarse(const DImage& P, const SidRay& r, const SidAxis& X,
+                                          const SidAxis& Y, const SidAxis& Z)
+{
+	return fmaxf(fmaxf(fabsf(X.gs), fabsf((r.p1.x - X.start) / P.vx)),
+	             fmaxf(fmaxf(fabsf(Y.gs), fabsf((r.p1.y - Y.start) / P.vy)),
+	                   fmaxf(fabsf(Z.gs), fabsf((r.p1.z - Z.start) / P.vz)))) > 1e6f;
+}
+
 // The pieces of an FP32 ray's walk in tiles of 2^lx x 2^ly x 2^lz voxels,
 // without walking its segments: fn(a0, vx, vy, vz, segs) for each tile the
 // walk passes through, in its order, a0 the alpha and (vx, vy, vz) the voxel
@@ -500,69 +569,13 @@ __device__ __forceinline__ void sidPieces(const DImage& P, const SidRay& r, int 
                                           int dz, Fn&& fn)
 {
 #pragma clang fp contract(off)
-	// plane numbers are kept as floats (exact: at most 1024 voxels an axis)
-	struct Axis
-	{
-		float start, sv, p, inv;  // plane q: (start + q sv - p) inv
-		float gs, g0;             // planes passed at alpha m: gs m + g0
-		float k, kt, kend;        // next plane, the tile's face, the image's
-		float dirf, off;          // voxel whose far face is plane q: dirf q + off
-		float T;
-		__device__ __forceinline__ float plane(float q) const
-		{
-			const float c = start + q * sv;
-			return (c - p) * inv;
-		}
-		__device__ __forceinline__ int voxel(float q) const { return (int)(q * dirf + off); }
-		// the first plane after alpha m, from plane k on (at: the alpha of
-		// the tile's face, which is passed if not after m: every round of
-		// the loop leaves a tile, whatever the numbers)
-		__device__ __forceinline__ float after(float m, float at, bool coarse) const
-		{
-			float q = fminf(fmaxf(floorf(fmaf(m, gs, g0)) + 1.f, k), kt + 1.f);
-			const float lo = plane(q - 1.f), hi = plane(q);
-			q += (hi <= m) ? 1.f : ((lo > m && q > k) ? -1.f : 0.f);
-			if (coarse)
-			{
-				while (q > k && plane(q - 1.f) > m)
-					q -= 1.f;
-				while (q < kend + 16.f && plane(q) <= m)
-					q += 1.f;
-			}
-			return (at <= m) ? fmaxf(q, kt + 1.f) : q;
-		}
-	};
-	const float FMAX = 3.402823466e+38f;
-	auto axis = [&](float len, float v, float p1, float p2, float inv, int dir, int n, int l,
-	                int sh, int vox) {
-		Axis a;
-		const bool flat = p1 == p2;
-		const float rv = (dir > 0) ? 1.0f / v : -1.0f / v;
-		a.start = (dir > 0) ? -len * 0.5f : len * 0.5f;
-		a.sv = (float)dir * v;
-		a.p = flat ? -FMAX : p1;
-		a.inv = flat ? 1.f : inv;
-		a.k = (float)(((dir > 0) ? vox + 1 : n - vox) + sh);
-		a.gs = (p2 - p1) * rv;
-		a.g0 = flat ? a.k - 1.f : (p1 - a.start) * rv;
-		const int t = vox >> l;
-		a.kt = (float)((dir > 0 ? min((t + 1) << l, n) : n - (t << l)) + sh);
-		a.kend = (float)(n + sh);
-		a.dirf = (float)dir;
-		a.off = (float)(dir > 0 ? -1 - sh : n + sh);
-		a.T = (float)(1 << l);
-		return a;
-	};
 	if ((unsigned)vx >= (unsigned)P.nx || (unsigned)vy >= (unsigned)P.ny ||
 	    (unsigned)vz >= (unsigned)P.nz)
 		return;
-	Axis X = axis(P.lx, P.vx, r.p1.x, r.p2.x, r.invx, r.dirx, P.nx, lx, dx, vx);
-	Axis Y = axis(P.ly, P.vy, r.p1.y, r.p2.y, r.invy, r.diry, P.ny, ly, dy, vy);
-	Axis Z = axis(P.lz, P.vz, r.p1.z, r.p2.z, r.invz, r.dirz, P.nz, lz, dz, vz);
-	const bool coarse =
-	    fmaxf(fmaxf(fabsf(X.gs), fabsf((r.p1.x - X.start) / P.vx)),
-	          fmaxf(fmaxf(fabsf(Y.gs), fabsf((r.p1.y - Y.start) / P.vy)),
-	                fmaxf(fabsf(Z.gs), fabsf((r.p1.z - Z.start) / P.vz)))) > 1e6f;
+	SidAxis X = sidAxis(P.lx, P.vx, r.p1.x, r.p2.x, r.invx, r.dirx, P.nx, lx, dx, vx);
+	SidAxis Y = sidAxis(P.ly, P.vy, r.p1.y, r.p2.y, r.invy, r.diry, P.ny, ly, dy, vy);
+	SidAxis Z = sidAxis(P.lz, P.vz, r.p1.z, r.p2.z, r.invz, r.dirz, P.nz, lz, dz, vz);
+	const bool coarse = sidCoarse(P, r, X, Y, Z);
 	float a0 = r.a_cur;
 	for (;;)
 	{
@@ -884,6 +897,59 @@ __device__ __forceinline__ void sidWalk(const DImage& P, const SidRay& r,
 	sidWalk<TOF, S64, false>(P, r, tof, B, first, vx, vy, vz, fn, [](uint32_t) {});
 }
 
+// The sum of w * x over a walk.
+template <bool TOF, bool S64, bool BRICK>
+__device__ __forceinline__ float sidForward(const DImage& P, const SidRay& r, const DTof& tof,
+                                            const float* __restrict__ img, bool first, int vx,
+                                            int vy, int vz)
+{
+	// one FMA per segment in the walk's order, a segment behind the walk,
+	// and the voxel's value fetched a segment ahead: its gather has two
+	// steps to arrive (8.4 M attenuation rays at 256 x 256 x 128 3.5 ->
+	// 3.1 ms, 1 M unordered TOF LORs x 4 rays at 200 x 200 x 128 0.85 ->
+	// 0.76; a third step spills: slower)
+	float acc = 0.f, xv = 0.f, w1 = 0.f, x1 = 0.f;
+	sidWalk<TOF, S64, BRICK>(
+	    P, r, tof, imageBox(P), first, vx, vy, vz,
+	    [&](int, int, int, uint32_t, float, float w, uint32_t nidx) {
+		    acc = fmaf(w1, x1, acc);
+		    w1 = w;
+		    x1 = xv;
+		    xv = img[nidx];
+	    },
+	    [&](uint32_t idx) { xv = img[idx]; });
+	acc = fmaf(w1, x1, acc);
+	return acc;
+}
+
+// The start of stretch `part` > 0 of `parts` of an FP32 ray's walk: its alpha,
+// or amax if the stretch is empty, and in (vx, vy, vz), the walk's first voxel
+// before, its first.  The walk's alphas are cut in equal lengths; a stretch
+// starts with the first crossing after its cut (found as sidPieces finds a
+// tile's), so segments stay whole and their weights the walk's.
+__device__ __forceinline__ float sidPart(const DImage& P, const SidRay& r, int part, int parts,
+                                         int& vx, int& vy, int& vz, int dx, int dy, int dz)
+{
+#pragma clang fp contract(off)
+	const float FMAX = 3.402823466e+38f;
+	// (one tile of the whole image: its faces are the image's)
+	SidAxis X = sidAxis(P.lx, P.vx, r.p1.x, r.p2.x, r.invx, r.dirx, P.nx, 20, dx, vx);
+	SidAxis Y = sidAxis(P.ly, P.vy, r.p1.y, r.p2.y, r.invy, r.diry, P.ny, 20, dy, vy);
+	SidAxis Z = sidAxis(P.lz, P.vz, r.p1.z, r.p2.z, r.invz, r.dirz, P.nz, 20, dz, vz);
+	const bool coarse = sidCoarse(P, r, X, Y, Z);
+	const float cut = r.a_cur + (r.amax - r.a_cur) * ((float)part / (float)parts);
+	X.k = X.after(cut, FMAX, coarse);
+	Y.k = Y.after(cut, FMAX, coarse);
+	Z.k = Z.after(cut, FMAX, coarse);
+	const float start = fminf(X.plane(X.k), fminf(Y.plane(Y.k), Z.plane(Z.k)));
+	const float qx = X.after(start, FMAX, coarse), qy = Y.after(start, FMAX, coarse),
+	            qz = Z.after(start, FMAX, coarse);
+	vx = X.voxel(qx);
+	vy = Y.voxel(qy);
+	vz = Z.voxel(qz);
+	return (start < r.amax && qx <= X.kend && qy <= Y.kend && qz <= Z.kend) ? start : r.amax;
+}
+
 // Siddon ray over the whole image.  `img` points at the frame's voxels.
 // MODE_FWD returns the line integral; MODE_BACK adds val*w atomically;
 // MODE_COUNT counts applied segments.
@@ -900,22 +966,7 @@ __device__ __forceinline__ float siddonRay(const DImage& P,
 		return 0.f;
 	if constexpr (MODE == MODE_FWD)
 	{
-		// one FMA per segment in the walk's order, a segment behind the walk,
-		// and the voxel's value fetched a segment ahead: its gather has two
-		// steps to arrive (8.4 M attenuation rays at 256 x 256 x 128 3.5 ->
-		// 3.1 ms, 1 M unordered TOF LORs x 4 rays at 200 x 200 x 128 0.85 ->
-		// 0.76; a third step spills: slower)
-		float acc = 0.f, xv = 0.f, w1 = 0.f, x1 = 0.f;
-		sidWalk<TOF, S64, BRICK>(
-		    P, r, tof, imageBox(P), true, 0, 0, 0,
-		    [&](int, int, int, uint32_t, float, float w, uint32_t nidx) {
-			    acc = fmaf(w1, x1, acc);
-			    w1 = w;
-			    x1 = xv;
-			    xv = img[nidx];
-		    },
-		    [&](uint32_t idx) { xv = img[idx]; });
-		acc = fmaf(w1, x1, acc);
+		const float acc = sidForward<TOF, S64, BRICK>(P, r, tof, img, true, 0, 0, 0);
 		return acc * r.ws;
 	}
 	const float vs = val * r.ws;

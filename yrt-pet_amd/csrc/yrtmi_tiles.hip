@@ -947,20 +947,49 @@ __device__ __forceinline__ float emRatioOut(const KArgs& a, int64_t e, float s, 
 	return out;
 }
 
+// The line integral of an FP32 ray's stretch `part` of PARTS (sidPart), by one
+// of PARTS neighbouring lanes, all of them here with the same ray; it ends where
+// the next one starts.
+template <bool TOF, bool BRICK, int PARTS>
+__device__ __forceinline__ float siddonPart(const DImage& P, const float* __restrict__ img,
+                                            float3 p1, float3 p2, const DTof& tof, float tofv,
+                                            int part)
+{
+	SidRay r;
+	int vx, vy, vz, dx, dy, dz;
+	auto outside = [&]() {
+		return (unsigned)vx >= (unsigned)P.nx || (unsigned)vy >= (unsigned)P.ny ||
+		       (unsigned)vz >= (unsigned)P.nz;
+	};
+	if (!sidSetup<TOF, false>(P, p1, p2, tof, tofv, r) ||
+	    !sidFirst<false>(P, r, vx, vy, vz, dx, dy, dz) || outside())
+		return 0.f;
+	const float start = part > 0 ? sidPart(P, r, part, PARTS, vx, vy, vz, dx, dy, dz) : r.a_cur;
+	const float next = __shfl_down(start, 1, PARTS);
+	if (part < PARTS - 1)
+		r.amax = next;
+	if (!(start < r.amax) || outside())
+		return 0.f;
+	sidRestart<false>(P, r, start, vx, vy, vz, dx, dy, dz);
+	return sidForward<TOF, false, BRICK>(P, r, tof, img, false, vx, vy, vz) * r.ws;
+}
+
 // Siddon: LPE lanes per LOR splitting its rays, made from the resolved LOR
 // (the LUT stays in L2; a plan's ray table, read from HBM, measured slower).
 // BRICK: gathers from the bricked copy of x (a.xb; useBricks), else from x.
-template <bool TOF, int LPE, bool S64, bool BRICK>
+// PARTS: lanes per ray, in turn along it (kSplitRays; the FP32 set-up's).
+template <bool TOF, int LPE, bool S64, bool BRICK, int PARTS>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(S64 ? 4 : 5, 8)))
 kEmRatio(KArgs a, float* __restrict__ v)
 {
-	const int64_t total = a.L.n * LPE;
+	constexpr int lanes = LPE * PARTS;
+	const int64_t total = a.L.n * lanes;
 	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
 	for (int64_t t = xcdRange(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; t < total;
 	     t += stride)
 	{
-		const int64_t e = t / LPE;
-		const int lane = (int)(t & (LPE - 1));
+		const int64_t e = t / lanes;
+		const int lane = (int)(t & (lanes - 1));
 		const Lor l = fetchLor(a.sc, a.L, e, a.im.nt);
 		const float m = a.c.meas ? a.c.meas[e] : 1.0f;
 		const float sf = a.c.sens ? a.c.sens[e] : 1.0f;
@@ -971,20 +1000,24 @@ kEmRatio(KArgs a, float* __restrict__ v)
 		{
 			const float* img = BRICK ? a.xb + (int64_t)l.frame * a.bvox
 			                         : a.x + (int64_t)l.frame * a.im.nvox;
-			for (int r = lane; r < a.pr.numRays; r += LPE)
+			for (int r = lane / PARTS; r < a.pr.numRays; r += LPE)
 			{
 				float3 q1, q2;
 				rayLine(a.pr, l, r, q1, q2);
 				q1 = make_float3(q1.x - a.im.ox, q1.y - a.im.oy, q1.z - a.im.oz);
 				q2 = make_float3(q2.x - a.im.ox, q2.y - a.im.oy, q2.z - a.im.oz);
 				uint32_t c = 0;
-				s += siddonRay<MODE_FWD, TOF, S64, BRICK>(a.im, const_cast<float*>(img), q1, q2,
-				                                          0.f, a.pr.tof, l.tof, c);
+				if constexpr (PARTS > 1)
+					s += siddonPart<TOF, BRICK, PARTS>(a.im, img, q1, q2, a.pr.tof, l.tof,
+					                                   lane & (PARTS - 1));
+				else
+					s += siddonRay<MODE_FWD, TOF, S64, BRICK>(a.im, const_cast<float*>(img), q1,
+					                                          q2, 0.f, a.pr.tof, l.tof, c);
 			}
 		}
 #pragma unroll
-		for (int o = 1; o < LPE; o <<= 1)
-			s += __shfl_xor(s, o, LPE);
+		for (int o = 1; o < lanes; o <<= 1)
+			s += __shfl_xor(s, o, lanes);
 		if (lane == 0)
 			v[e] = skip ? 0.f : emRatioOut(a, e, s, m, sf, af);
 	}
@@ -1432,21 +1465,31 @@ hipError_t launchTileBack(const KArgs& a, const DTiles& T, const DPlanRead& pl,
 }
 
 template <bool TOF, bool S64, bool BRICK>
-static hipError_t ratioLpe(const KArgs& a, int lpe, dim3 g, float* v, hipStream_t st)
+static hipError_t ratioLpe(const KArgs& a, int lpe, int parts, dim3 g, float* v, hipStream_t st)
 {
+	auto go = [&](auto lanes) {
+		constexpr int N = decltype(lanes)::value;
+		if constexpr (!S64)
+			if (parts > 1)
+			{
+				kEmRatio<TOF, N, S64, BRICK, kRayParts><<<g, 256, 0, st>>>(a, v);
+				return;
+			}
+		kEmRatio<TOF, N, S64, BRICK, 1><<<g, 256, 0, st>>>(a, v);
+	};
 	switch (lpe)
 	{
 	case 1:
-		kEmRatio<TOF, 1, S64, BRICK><<<g, 256, 0, st>>>(a, v);
+		go(std::integral_constant<int, 1>{});
 		break;
 	case 2:
-		kEmRatio<TOF, 2, S64, BRICK><<<g, 256, 0, st>>>(a, v);
+		go(std::integral_constant<int, 2>{});
 		break;
 	case 4:
-		kEmRatio<TOF, 4, S64, BRICK><<<g, 256, 0, st>>>(a, v);
+		go(std::integral_constant<int, 4>{});
 		break;
 	case 8:
-		kEmRatio<TOF, 8, S64, BRICK><<<g, 256, 0, st>>>(a, v);
+		go(std::integral_constant<int, 8>{});
 		break;
 	default:
 		return hipErrorInvalidValue;
@@ -1455,7 +1498,7 @@ static hipError_t ratioLpe(const KArgs& a, int lpe, dim3 g, float* v, hipStream_
 }
 
 template <bool TOF, bool S64>
-static hipError_t ratioT(const KArgs& a, int lpe, dim3 g, float* v, hipStream_t st)
+static hipError_t ratioT(const KArgs& a, int lpe, int parts, dim3 g, float* v, hipStream_t st)
 {
 	if (a.pr.type == 1)
 	{
@@ -1472,8 +1515,8 @@ static hipError_t ratioT(const KArgs& a, int lpe, dim3 g, float* v, hipStream_t 
 			a.rays != nullptr ? lanes(Y{}, N{}) : lanes(N{}, N{});
 		return hipGetLastError();
 	}
-	return a.xb != nullptr ? ratioLpe<TOF, S64, true>(a, lpe, g, v, st)
-	                       : ratioLpe<TOF, S64, false>(a, lpe, g, v, st);
+	return a.xb != nullptr ? ratioLpe<TOF, S64, true>(a, lpe, parts, g, v, st)
+	                       : ratioLpe<TOF, S64, false>(a, lpe, parts, g, v, st);
 }
 
 // One workgroup per row of bricks (y, z), its threads along it: no division
@@ -1510,7 +1553,11 @@ hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st)
 		return hipErrorInvalidValue;
 	if (a.pr.type == 1)
 		lpe = a.L.n <= kDDLanesUpTo ? 4 : 1;
-	const int64_t threads = a.L.n * lpe;
+	const int parts = a.pr.type == 0 && !a.pr.setup64 &&
+	                          a.L.n * (int64_t)a.pr.numRays <= kSplitRays
+	                      ? kRayParts
+	                      : 1;
+	const int64_t threads = a.L.n * lpe * parts;
 	int64_t nb = (threads + 255) / 256;
 	if (nb > 0x7ffffff0)
 		nb = 0x7ffffff0;
@@ -1520,10 +1567,10 @@ hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st)
 	const dim3 g((unsigned)nb);
 	const bool tof = a.pr.useTof != 0;
 	if (a.pr.setup64)
-		return tof ? ratioT<true, true>(a, lpe, g, v, st)
-		           : ratioT<false, true>(a, lpe, g, v, st);
-	return tof ? ratioT<true, false>(a, lpe, g, v, st)
-	           : ratioT<false, false>(a, lpe, g, v, st);
+		return tof ? ratioT<true, true>(a, lpe, parts, g, v, st)
+		           : ratioT<false, true>(a, lpe, parts, g, v, st);
+	return tof ? ratioT<true, false>(a, lpe, parts, g, v, st)
+	           : ratioT<false, false>(a, lpe, parts, g, v, st);
 }
 
 hipError_t launchSensValue(const KArgs& a, float* v, hipStream_t st)

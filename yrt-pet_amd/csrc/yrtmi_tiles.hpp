@@ -230,6 +230,14 @@ hipError_t launchStreamScan(const DPlan& pl, int64_t* tileOff, int nTiles, int64
 // 116 / 220, 252 / 302, 336 / 425.
 constexpr int64_t kDDLanesUpTo = 196608;
 
+// Rays up to which a Siddon forward takes kRayParts lanes per ray (FP32 set-up):
+// a walk is a chain of steps and gathers, and these fill 4 waves for each of the
+// chip's SIMDs at most.  One lane against four, us: 4096 rays of 200 x 200 x 128
+// 65 / 23 (TOF 22 / 12), 65536 77 / 47 (36 / 31), 98304 78 / 76 (39 / 48); of 96 x
+// 96 x 48 27 / 12, 23 / 20, 28 / 28.
+constexpr int kRayParts = 4;
+constexpr int64_t kSplitRays = 65536;
+
 // LDS of the fill pass: an int counter and a 32-bit base per bin.
 inline size_t binLdsBytes(int nB)
 {
