@@ -426,12 +426,12 @@ int yrtmi_permute(yrtmi_ctx* ctx, const void* src, int elem_bytes,
  * OSEM_GPU::computeEMUpdateImage,
  * OSEM_GPU::generateSensitivityImageForCurrentSubset).
  *
- * Siddon: a plan bins the walk of every (LOR, ray) of `lors` by the image
- * tiles it crosses, recording where it enters each (12 bytes per record,
+ * Siddon: a plan bins every (LOR, ray) of `lors` by the image tiles its
+ * walk crosses, recording where it enters each (12 bytes per record,
  * records of a tile ordered by the length of their piece), and keeps each
- * ray's end points, TOF value and frame (32 bytes per LOR and ray), plus,
- * with the FP32 set-up, the ray's walk set-up (inverse direction, exit
- * parameter, TOF terms: 64 bytes per LOR and ray in all), so that the
+ * ray's end points and frame (32 bytes per LOR and ray; TOF value or first
+ * voxel), plus, with the FP32 set-up, the ray's walk set-up (inverse direction,
+ * exit parameter, TOF terms: 64 bytes per LOR and ray in all), so that the
  * backprojection reads one table entry per record instead of resolving the
  * LOR and redoing its set-up.
  * DD: a plan keeps each LOR's footprint set-up (128 bytes per LOR) and one
@@ -534,10 +534,11 @@ int yrtmi_em_subset_planned(yrtmi_ctx* ctx, const yrtmi_proj* p,
  * EM ratio of LOR i (m / corrected forward projection, times the
  * multiplicative corrections), 0 where the reference skips the LOR.
  * yrtmi_em_subset_planned = yrtmi_em_ratio_planned + yrtmi_back_planned(v).
- * Siddon projects a bricked copy of x made at each call into a buffer the
- * context keeps (4 x 4 x 2-voxel bricks; same values, same sums): it grows
- * on the first call of a larger image, or when a plan is created, which a
- * caller recording a graph must do before recording.
+ * Images of 2^21 voxels and more are projected from a bricked copy of x made
+ * at each call into a buffer the context keeps (4 x 4 x 2-voxel bricks; same
+ * values, same sums): it grows on the first call of a larger image, or when a
+ * plan is created, which a caller recording a graph of a Siddon ratio must do
+ * before recording (a DD ratio reads x itself where there is no buffer).
  * Replaces the forward half of OSEM_CPU::computeEMUpdateImage
  * (src/recon/OSEM_CPU.cpp:329-374). */
 int yrtmi_em_ratio(yrtmi_ctx* ctx, const yrtmi_proj* p, const yrtmi_image* im,
