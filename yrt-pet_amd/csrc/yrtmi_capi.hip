@@ -1454,6 +1454,7 @@ int yrtmi_sensitivity(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 		if (r)
 			return r;
 		a.attIm = toDImage(att_im);
+		a.attIm.nt = 1;  // (a dynamic descriptor's frame 0 is the image)
 		a.att = att_img;
 	}
 	a.y = img;
@@ -2320,6 +2321,7 @@ int yrtmi_sensitivity_planned(yrtmi_ctx* c, const yrtmi_proj* p,
 		if (r)
 			return r;
 		a.attIm = toDImage(att_im);
+		a.attIm.nt = 1;  // (a dynamic descriptor's frame 0 is the image)
 		a.att = att_img;
 	}
 	a.vals = sens;
