@@ -316,8 +316,17 @@ __global__ void __launch_bounds__(kBinThreads) kBin(DImage im, DProj pr, int64_t
 		}
 		return;
 	}
-	if (pl.skip != nullptr && *pl.skip != 0)
-		return;
+	if (pl.skip != nullptr)
+	{
+		// read once for the workgroup: another one may be setting it now
+		if (threadIdx.x == 0)
+			cnt[0] = *pl.skip;
+		__syncthreads();
+		const int skip = cnt[0];
+		__syncthreads();
+		if (skip != 0)
+			return;
+	}
 	for (int i = threadIdx.x; i < nB; i += blockDim.x)
 	{
 		const int c = (int)myCnt[i];
