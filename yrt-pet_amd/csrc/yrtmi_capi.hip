@@ -345,7 +345,7 @@ bool reserve(yrtmi_ctx* c, Scratch& w, size_t bytes)
 // never allocate.
 int brickImage(yrtmi_ctx* c, KArgs& a)
 {
-	if (!useBricks(a.im.nvox * a.im.nt))
+	if (!useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt))
 		return YRTMI_OK;
 	const int64_t bvox = brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz);
 	if (!reserve(c, c->em, sizeof(float) * (size_t)(bvox * a.im.nt)))
@@ -381,7 +381,7 @@ bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, in
 {
 	*status = YRTMI_OK;
 	const int64_t bvox = brickFrameVoxels(im.nx, im.ny, im.nz);
-	if (!useBricks(im.nvox) || rays * kBrickRays < im.nvox * im.nt ||
+	if (!useBricks(im.nx, im.ny, im.nz, 1) || rays * kBrickRays < im.nvox * im.nt ||
 	    !reserve(c, c->fwd, sizeof(float) * (size_t)(bvox * im.nt)))
 		return false;
 	*status = acquire(c, c->fwd);
@@ -481,7 +481,7 @@ bool streamShape(yrtmi_ctx* c, const KArgs& a, bool em, StreamShape& s)
 	// records are not bounded so (a batch of more takes the direct kernel)
 	s.recPer = s.dd ? std::min<int64_t>(128, 8 * std::max(s.T.ntx, s.T.nty))
 	                : std::min<int64_t>(64, s.T.ntx + s.T.nty + s.T.ntz - 2);
-	s.brick = (em && useBricks(a.im.nvox * a.im.nt)) ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt : 0;
+	s.brick = (em && useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt)) ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt : 0;
 	return true;
 }
 
@@ -1919,7 +1919,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	const bool dd = p->d.type == YRTMI_PROJ_DD;
 	if (im->nx > 1024 || im->ny > 1024 || im->nz > 1024)
 		return fail(YRTMI_EINVAL, "plan: image dimensions above 1024");
-	if (useBricks(a.im.nvox * a.im.nt))
+	if (useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt))
 	{
 		// the bricked image of the planned EM ratio, sized here
 		if (!reserve(c, c->em,

@@ -262,7 +262,13 @@ hipError_t launchTileBack(const KArgs& a, const DTiles& T, const DPlanRead& pl,
 // A smaller image is in L2 anyway, and the bricked walk's extra instructions
 // show: 1 M TOF rays of 96 x 96 x 48 111 us from rows and 140 bricked, of 200
 // x 200 x 128 190 and 163.
-inline bool useBricks(int64_t voxels) { return voxels >= (int64_t(1) << 21); }
+// (A frame's bricks are indexed in 32 bits, padding included, which a frame
+// of few voxels along one axis, or of just below 2^31, may exceed.)
+inline bool useBricks(int64_t nx, int64_t ny, int64_t nz, int64_t frames)
+{
+	return nx * ny * nz * frames >= (int64_t(1) << 21) &&
+	       brickFrameVoxels((int)nx, (int)ny, (int)nz) < (int64_t(1) << 31);
+}
 // xb (nt frames of brickFrameVoxels floats) = bricked copy of x (nt frames
 // of the image's voxels), padding voxels 0.
 hipError_t launchToBricks(const DImage& im, const float* x, float* xb, hipStream_t st);
