@@ -156,7 +156,14 @@ int yrtmi_ctx_own_stream(yrtmi_ctx* ctx, void** stream);
  * Calls that allocate, copy or synchronise (plan_create, count_segments,
  * histo_subset_nonzero, lor_order, copy, device_alloc/free, lut / histo /
  * motion uploads, and a first per-XCD backprojection that would allocate its
- * partial images or scratch) fail with YRTMI_ESTATE while recording. */
+ * partial images or scratch) fail with YRTMI_ESTATE while recording.
+ * A graph may be launched through any context of its device, while the
+ * context that recorded it lives (its tables are read); launches and other
+ * calls that use the same scratch are ordered on the device.  Calls captured
+ * by the caller itself (the context's stream in a capture of its own) use no
+ * scratch of the context but a Siddon EM ratio's bricked image, if there is
+ * one, and the per-XCD partial images: the caller orders replays that use
+ * these with the context's other calls. */
 typedef struct yrtmi_graph yrtmi_graph;
 int yrtmi_graph_begin(yrtmi_ctx* ctx);
 int yrtmi_graph_end(yrtmi_ctx* ctx, yrtmi_graph** out);

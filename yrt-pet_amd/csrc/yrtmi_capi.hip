@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -50,18 +51,28 @@ int hipFail(hipError_t e, const char* what)
 
 }  // namespace
 
-// Device scratch of a context, used in stream order: a call on another
-// stream than the last one's waits for it.  Scratch that a graph refers to
-// stays until the context goes when it is grown.
+// Device scratch, used in stream order: each use waits for the last one's
+// event and records its own.  Held by the context that made it, which
+// replaces it by a larger one, and by the graphs recorded with it, whose
+// replays may come through other contexts and threads: the mutex is held from
+// a use's wait to its record.  A thread that holds several takes them in the
+// order of `rank`.
 struct Scratch
 {
+	int device = 0, rank = 0;
 	void* p = nullptr;
 	size_t bytes = 0;
-	hipEvent_t event = nullptr;  // the last use, on `stream`
-	hipStream_t stream = nullptr;
-	bool used = false, captured = false;
-	std::vector<void*> retired;
+	hipEvent_t event = nullptr;  // the last use
+	bool used = false;
+	std::mutex m;
+	~Scratch()
+	{
+		poolFree(device, p, poolQuiesce(device));
+		if (event != nullptr)
+			(void)hipEventDestroy(event);
+	}
 };
+using ScratchPtr = std::shared_ptr<Scratch>;
 
 struct yrtmi_ctx
 {
@@ -86,11 +97,15 @@ struct yrtmi_ctx
 	float* part = nullptr;
 	int64_t partStride = 0;
 	int nxcc = 1;
-	Scratch em;   // the bricked image that EM ratios project
-	Scratch ws;   // of the backprojections binned by tiles without a plan (streamBack)
-	Scratch fwd;  // the bricked image of forward and sensitivity projections
+	// (null until needed; ranks 0, 1, 2)
+	ScratchPtr em;   // the bricked image that EM ratios project
+	ScratchPtr ws;   // of the backprojections binned by tiles without a plan (streamBack)
+	ScratchPtr fwd;  // the bricked image of forward and sensitivity projections
 	hipStream_t owned = nullptr;  // stream created by yrtmi_ctx_own_stream
 	bool capturing = false;       // between yrtmi_graph_begin and _end
+	// scratch that the calls being recorded use; scratch that calls captured
+	// by the caller use (their graph is not known here: kept to the end)
+	std::vector<ScratchPtr> recorded, kept;
 };
 
 struct yrtmi_graph
@@ -98,6 +113,7 @@ struct yrtmi_graph
 	int device = 0;
 	hipGraph_t graph = nullptr;
 	hipGraphExec_t exec = nullptr;
+	std::vector<ScratchPtr> scratch;  // what its calls use, by rank
 };
 
 struct yrtmi_proj
@@ -291,80 +307,117 @@ int ensurePartials(yrtmi_ctx* c, int64_t n)
 	return YRTMI_OK;
 }
 
-// Before and after a call's use of the scratch.
-int acquire(yrtmi_ctx* c, Scratch& w)
+// Whether the context's stream is being captured other than by
+// yrtmi_graph_begin.
+bool callerCaptures(yrtmi_ctx* c)
 {
-	if (!c->capturing && w.used && w.stream != c->stream)
-		HIP_TRY(hipStreamWaitEvent(c->stream, w.event, 0));
-	return YRTMI_OK;
-}
-
-int release(yrtmi_ctx* c, Scratch& w)
-{
-	if (c->capturing)
-	{
-		w.captured = true;
-		return YRTMI_OK;
-	}
-	if (w.event == nullptr)
-		HIP_TRY(hipEventCreateWithFlags(&w.event, hipEventDisableTiming));
-	HIP_TRY(hipEventRecord(w.event, c->stream));
-	w.stream = c->stream;
-	w.used = true;
-	return YRTMI_OK;
-}
-
-// At least `bytes` of scratch; false where there is no memory for it, or the
-// context is recording and has less.
-bool reserve(yrtmi_ctx* c, Scratch& w, size_t bytes)
-{
-	if (w.bytes >= bytes)
-		return true;
 	if (c->capturing)
 		return false;
-	void* q = nullptr;
-	bytes = std::max(bytes, w.bytes + w.bytes / 2);
-	if (poolAlloc(c->device, &q, bytes) != hipSuccess)
+	hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+	if (hipStreamIsCapturing(c->stream, &st) == hipSuccess)
+		return st != hipStreamCaptureStatusNone;
+	(void)hipGetLastError();
+	return false;
+}
+
+// One call's use of a scratch buffer on its context's stream, from begin()
+// before its first launch to end() after its last (or, where the call fails
+// between them, to the destructor).  Recorded uses are ordered by the launch
+// of their graph instead; uses captured by the caller cannot be ordered here.
+class ScratchUse
+{
+public:
+	ScratchUse() = default;
+	ScratchUse(const ScratchUse&) = delete;
+	ScratchUse(ScratchUse&& o) noexcept
+	    : m_stream(o.m_stream), m_s(std::move(o.m_s)), m_lock(std::move(o.m_lock))
+	{
+	}
+	~ScratchUse() { (void)end(); }
+	int begin(yrtmi_ctx* c, const ScratchPtr& s)
+	{
+		if (c->capturing || callerCaptures(c))
+		{
+			auto& held = c->capturing ? c->recorded : c->kept;
+			if (std::find(held.begin(), held.end(), s) == held.end())
+				held.push_back(s);
+			return YRTMI_OK;
+		}
+		m_lock = std::unique_lock<std::mutex>(s->m);
+		m_stream = c->stream;
+		m_s = s;
+		if (s->event == nullptr)
+			HIP_TRY(hipEventCreateWithFlags(&s->event, hipEventDisableTiming));
+		if (s->used)
+			HIP_TRY(hipStreamWaitEvent(m_stream, s->event, 0));
+		return YRTMI_OK;
+	}
+	int end()
+	{
+		if (m_s == nullptr)
+			return YRTMI_OK;
+		const ScratchPtr s = std::move(m_s);
+		const std::unique_lock<std::mutex> lk = std::move(m_lock);
+		if (s->event != nullptr)
+		{
+			HIP_TRY(hipEventRecord(s->event, m_stream));
+			s->used = true;
+		}
+		return YRTMI_OK;
+	}
+
+private:
+	hipStream_t m_stream = nullptr;
+	ScratchPtr m_s;
+	std::unique_lock<std::mutex> m_lock;  // (of m_s: released before it)
+};
+
+// At least `bytes` of scratch; false where there is no memory for it, or the
+// context's stream is being captured and there is less.
+bool reserve(yrtmi_ctx* c, ScratchPtr& w, int rank, size_t bytes)
+{
+	const size_t have = w ? w->bytes : 0;
+	if (have >= bytes)
+		return true;
+	if (c->capturing || callerCaptures(c))
+		return false;
+	auto q = std::make_shared<Scratch>();
+	q->device = c->device;
+	q->rank = rank;
+	q->bytes = std::max(bytes, have + have / 2);
+	if (poolAlloc(c->device, &q->p, q->bytes) != hipSuccess)
 	{
 		(void)hipGetLastError();
 		return false;
 	}
-	if (w.captured)
-		w.retired.push_back(w.p);
-	else
-		poolFree(c->device, w.p, w.p == nullptr || poolQuiesce(c->device));
-	w.p = q;
-	w.bytes = bytes;
+	w = std::move(q);
 	return true;
 }
 
 // The bricked copy of a.x for the EM ratio's forward; small images are read
 // as they are, and so is a DD call's while recording without the buffer
-// (Siddon refuses that).  The caller releases it after its launch
-// (brickDone).  Tile plans reserve it for their image, so planned EM calls
-// never allocate.
-int brickImage(yrtmi_ctx* c, KArgs& a)
+// (Siddon refuses that), or captured by the caller.  The caller ends the use
+// after its launch.  Tile plans reserve the buffer for their image, so planned
+// EM calls never allocate.
+int brickImage(yrtmi_ctx* c, KArgs& a, ScratchUse& use)
 {
 	if (!useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt))
 		return YRTMI_OK;
 	const int64_t bvox = brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz);
-	if (!reserve(c, c->em, sizeof(float) * (size_t)(bvox * a.im.nt)))
-		return a.pr.type == YRTMI_PROJ_DD
+	const bool dd = a.pr.type == YRTMI_PROJ_DD;
+	if ((dd && callerCaptures(c)) ||
+	    !reserve(c, c->em, 0, sizeof(float) * (size_t)(bvox * a.im.nt)))
+		return dd
 		           ? YRTMI_OK
 		           : notCapturing(c,
 		                          "bricked image (run one EM ratio of this size before recording)");
-	const int r = acquire(c, c->em);
+	const int r = use.begin(c, c->em);
 	if (r)
 		return r;
-	HIP_TRY(launchToBricks(a.im, a.x, (float*)c->em.p, c->stream));
-	a.xb = (const float*)c->em.p;
+	HIP_TRY(launchToBricks(a.im, a.x, (float*)c->em->p, c->stream));
+	a.xb = (const float*)c->em->p;
 	a.bvox = bvox;
 	return YRTMI_OK;
-}
-
-int brickDone(yrtmi_ctx* c, const KArgs& a)
-{
-	return a.xb != nullptr ? release(c, c->em) : YRTMI_OK;
 }
 
 constexpr int64_t kBrickRays = 4;  // voxels a ray above which it is not
@@ -375,25 +428,27 @@ constexpr int64_t kBrickRays = 4;  // voxels a ray above which it is not
 // rays at 200 x 200 x 128: 1.08 -> 0.76 ms).  The size is a frame's: LORs in
 // locality order read one frame at a time (8 frames of 128 x 128 x 64, 160 M
 // LORs: 98.7 ms from bricks, 87.5 from rows; in no order 1.6 M 1.29 / 1.41).
-// The caller releases c->fwd after its launch.
+// Not where the caller captures the stream: a forward used no scratch of the
+// context before it used bricks, and the graph's replays cannot be ordered
+// with the context's other calls.  The caller ends the use after its launch.
 bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, int64_t rays,
-                  int* status)
+                  ScratchUse& use, int* status)
 {
 	*status = YRTMI_OK;
 	const int64_t bvox = brickFrameVoxels(im.nx, im.ny, im.nz);
 	if (!useBricks(im.nx, im.ny, im.nz, 1) || rays * kBrickRays < im.nvox * im.nt ||
-	    !reserve(c, c->fwd, sizeof(float) * (size_t)(bvox * im.nt)))
+	    callerCaptures(c) || !reserve(c, c->fwd, 2, sizeof(float) * (size_t)(bvox * im.nt)))
 		return false;
-	*status = acquire(c, c->fwd);
+	*status = use.begin(c, c->fwd);
 	if (*status != YRTMI_OK)
 		return false;
-	const hipError_t e = launchToBricks(im, img, (float*)c->fwd.p, c->stream);
+	const hipError_t e = launchToBricks(im, img, (float*)c->fwd->p, c->stream);
 	if (e != hipSuccess)
 	{
 		*status = hipFail(e, "bricked image");
 		return false;
 	}
-	a.xb = (const float*)c->fwd.p;
+	a.xb = (const float*)c->fwd->p;
 	a.bvox = bvox;
 	return true;
 }
@@ -503,26 +558,27 @@ DLors sliceLors(const DLors& L, int64_t b, int64_t e)
 // LORs per batch that the scratch has room for.
 int64_t streamBatch(const yrtmi_ctx* c, const StreamShape& s, int64_t n)
 {
-	if (c->ws.bytes <= s.fixedBytes())
+	if (c->ws == nullptr || c->ws->bytes <= s.fixedBytes())
 		return 0;
-	int64_t b = (int64_t)((c->ws.bytes - s.fixedBytes()) / s.lorBytes());
+	int64_t b = (int64_t)((c->ws->bytes - s.fixedBytes()) / s.lorBytes());
 	// keys and record numbers are 32 bits
 	b = std::min(b, ((int64_t(1) << 31) / std::max<int64_t>(1, s.recPer)) / s.R);
 	return std::min(b, n);
 }
 
 // Whether a backprojection of a.L goes through streamBack, its scratch then
-// made ready.
+// made ready (not where the caller captures the stream, as brickForward).
 bool streamReady(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a, bool em, StreamShape& s)
 {
 	const int64_t n = a.L.n, rays = n * (int64_t)a.pr.numRays, least = streamMinRays(a);
-	if (p->accum != YRTMI_ACCUM_XCD || rays < least || !streamShape(c, a, em, s))
+	if (p->accum != YRTMI_ACCUM_XCD || rays < least || callerCaptures(c) ||
+	    !streamShape(c, a, em, s))
 		return false;
 	const size_t want =
 	    std::max(s.fixedBytes() + (size_t)std::min<int64_t>(n, 1 << 26) * s.lorBytes(), size_t(1));
 	const size_t cap = std::max(std::min(want, kStreamBytes + (size_t)s.brick * 4),
 	                            s.fixedBytes() + (size_t)((least + s.R) / s.R) * s.lorBytes());
-	(void)reserve(c, c->ws, cap);  // else what there is
+	(void)reserve(c, c->ws, 1, cap);  // else what there is
 	const int64_t b = streamBatch(c, s, n);
 	return b == n || b * s.R >= least;
 }
@@ -533,12 +589,14 @@ int sensValue(yrtmi_ctx* c, KArgs a, float* v)
 	int r = YRTMI_OK;
 	a.xb = nullptr;
 	KArgs s = a;
-	const bool bricks = a.att != nullptr && brickForward(c, s, a.attIm, a.att, a.L.n, &r);
+	ScratchUse use;
+	if (a.att != nullptr)
+		(void)brickForward(c, s, a.attIm, a.att, a.L.n, use, &r);
 	if (r)
 		return r;
 	a.xb = s.xb;
 	HIP_TRY(launchSensValue(a, v, c->stream));
-	return bricks ? release(c, c->fwd) : YRTMI_OK;
+	return use.end();
 }
 
 enum StreamKind
@@ -551,12 +609,13 @@ enum StreamKind
 int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamShape& s,
                StreamKind kind, float* y, const float* vals)
 {
-	int r = acquire(c, c->ws);
+	ScratchUse use;
+	int r = use.begin(c, c->ws);
 	if (r)
 		return r;
 	hipStream_t st = c->stream;
 	const int64_t n = a0.L.n, batch = streamBatch(c, s, n);
-	char* at = (char*)c->ws.p;
+	char* at = (char*)c->ws->p;
 	auto take = [&](size_t bytes) {
 		char* q = at;
 		at += (bytes + 255) / 256 * 256;
@@ -646,7 +705,7 @@ int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamS
 		a.y = y;
 		HIP_TRY(launchBackIf(a, rd.err, st));
 	}
-	return release(c, c->ws);
+	return use.end();
 }
 
 // Set up per-XCD accumulation for a backprojection of n voxels into y, or
@@ -657,8 +716,8 @@ int setupAccum(yrtmi_ctx* c, const yrtmi_proj* p, KArgs& a, int64_t n)
 	if (p->accum != YRTMI_ACCUM_XCD || c->nxcc <= 1)
 		return YRTMI_OK;
 	// recording, no partial images yet, but a call before made the scratch
-	// of streamBack instead of them: straight into y
-	if (c->capturing && c->ws.p != nullptr && c->partStride < n)
+	// of streamBack instead of them, or captured by the caller: straight into y
+	if (c->partStride < n && ((c->capturing && c->ws != nullptr) || callerCaptures(c)))
 		return YRTMI_OK;
 	int r = ensurePartials(c, n);
 	if (r)
@@ -738,18 +797,11 @@ int yrtmi_ctx_destroy(yrtmi_ctx* c)
 	(void)hipFree(c->gatherErr);
 	(void)hipFree(c->counter);
 	(void)hipFree(c->part);
-	for (Scratch* w : {&c->em, &c->ws, &c->fwd})
-	{
-		if (w->p != nullptr)
-		{
-			const bool idle = poolQuiesce(c->device);
-			poolFree(c->device, w->p, idle);
-			for (void* p : w->retired)
-				poolFree(c->device, p, idle);
-		}
-		if (w->event != nullptr)
-			(void)hipEventDestroy(w->event);
-	}
+	// (graphs recorded with it keep the scratch that they use)
+	for (ScratchPtr* w : {&c->em, &c->ws, &c->fwd})
+		w->reset();
+	c->recorded.clear();
+	c->kept.clear();
 	if (c->owned != nullptr)
 		(void)hipStreamDestroy(c->owned);
 	poolRelease(c->device);
@@ -796,6 +848,8 @@ int yrtmi_graph_end(yrtmi_ctx* c, yrtmi_graph** out)
 	if (!c->capturing)
 		return fail(YRTMI_ESTATE, "graph_end: not recording");
 	c->capturing = false;
+	std::vector<ScratchPtr> scratch;
+	scratch.swap(c->recorded);
 	hipGraph_t g = nullptr;
 	HIP_TRY(hipStreamEndCapture(c->stream, &g));
 	if (out == nullptr)
@@ -814,6 +868,9 @@ int yrtmi_graph_end(yrtmi_ctx* c, yrtmi_graph** out)
 	q->device = c->device;
 	q->graph = g;
 	q->exec = x;
+	std::sort(scratch.begin(), scratch.end(),
+	          [](const ScratchPtr& a, const ScratchPtr& b) { return a->rank < b->rank; });
+	q->scratch = std::move(scratch);
 	*out = q;
 	return YRTMI_OK;
 }
@@ -828,12 +885,13 @@ int yrtmi_graph_launch(yrtmi_ctx* c, const yrtmi_graph* g)
 	r = notCapturing(c, "graph_launch");
 	if (r)
 		return r;
-	for (Scratch* w : {&c->em, &c->ws, &c->fwd})
-		if (w->captured && (r = acquire(c, *w)) != YRTMI_OK)
+	std::vector<ScratchUse> uses(g->scratch.size());
+	for (size_t i = 0; i < uses.size(); i++)
+		if ((r = uses[i].begin(c, g->scratch[i])) != YRTMI_OK)
 			return r;
 	HIP_TRY(hipGraphLaunch(g->exec, c->stream));
-	for (Scratch* w : {&c->em, &c->ws, &c->fwd})
-		if (w->captured && (r = release(c, *w)) != YRTMI_OK)
+	for (ScratchUse& u : uses)
+		if ((r = u.end()) != YRTMI_OK)
 			return r;
 	return YRTMI_OK;
 }
@@ -1252,7 +1310,8 @@ int yrtmi_forward(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	if (img == nullptr || out == nullptr)
 		return fail(YRTMI_EINVAL, "forward: null image or output");
 	a.x = img;
-	const bool bricks = brickForward(c, a, a.im, img, l->n * (int64_t)a.pr.numRays, &r);
+	ScratchUse use;
+	const bool bricks = brickForward(c, a, a.im, img, l->n * (int64_t)a.pr.numRays, use, &r);
 	if (r)
 		return r;
 	// (3 M DD LORs of 200 x 200 x 128 from bricks: TOF 4.3 -> 2.7 ms, without
@@ -1263,7 +1322,7 @@ int yrtmi_forward(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	{
 		a.plain = 1;
 		HIP_TRY(launchEmRatio(a, p->lpe, out, c->stream));
-		return bricks ? release(c, c->fwd) : YRTMI_OK;
+		return use.end();
 	}
 	a.out = out;
 	HIP_TRY(launchEvents(MODE_FWD, a, p->lpe, p->block, p->grid, c->stream));
@@ -1922,7 +1981,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	if (useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt))
 	{
 		// the bricked image of the planned EM ratio, sized here
-		if (!reserve(c, c->em,
+		if (!reserve(c, c->em, 0,
 		             sizeof(float) *
 		                 (size_t)(brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt)))
 			return fail(YRTMI_ENOMEM, "plan: bricked image");
@@ -2232,11 +2291,12 @@ int yrtmi_em_ratio(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 		return fail(YRTMI_EINVAL, "em_ratio: null image or output");
 	a.x = x;
 	setCorr(a, corr);
-	r = brickImage(c, a);
+	ScratchUse use;
+	r = brickImage(c, a, use);
 	if (r)
 		return r;
 	HIP_TRY(launchEmRatio(a, p->lpe, v, c->stream));
-	return brickDone(c, a);
+	return use.end();
 }
 
 int yrtmi_em_ratio_planned(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
@@ -2257,11 +2317,12 @@ int yrtmi_em_ratio_planned(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image*
 	a.x = x;
 	setCorr(a, corr);
 	a.rays = planRays(q);
-	r = brickImage(c, a);
+	ScratchUse use;
+	r = brickImage(c, a, use);
 	if (r)
 		return r;
 	HIP_TRY(launchEmRatio(a, p->lpe, v, c->stream));
-	return brickDone(c, a);
+	return use.end();
 }
 
 int yrtmi_em_subset_planned(yrtmi_ctx* c, const yrtmi_proj* p,
@@ -2283,11 +2344,12 @@ int yrtmi_em_subset_planned(yrtmi_ctx* c, const yrtmi_proj* p,
 	a.x = x;
 	setCorr(a, corr);
 	a.rays = planRays(q);
-	r = brickImage(c, a);
+	ScratchUse use;
+	r = brickImage(c, a, use);
 	if (r)
 		return r;
 	HIP_TRY(launchEmRatio(a, p->lpe, q->v, c->stream));
-	r = brickDone(c, a);
+	r = use.end();
 	if (r)
 		return r;
 	HIP_TRY(launchTileBack(a, q->T, planRead(q), q->v, u, q->persistent, c->stream));
@@ -2647,11 +2709,10 @@ int yrtmi_autotune(yrtmi_ctx* c, yrtmi_proj* p, const yrtmi_image* im,
 	a.x = x;
 	a.c.g = 1.0f;
 	a.c.denomThr = 1e-35f;
-	{
-		const int rb = brickImage(c, a);
-		if (rb)
-			return done(rb);
-	}
+	ScratchUse use;
+	r = brickImage(c, a, use);
+	if (r)
+		return done(r);
 	// time fn(): one untimed run, then the mean of two timed runs
 	auto timeIt = [&](auto&& fn, float& ms) -> hipError_t {
 		hipError_t e = fn();
@@ -2689,7 +2750,7 @@ int yrtmi_autotune(yrtmi_ctx* c, yrtmi_proj* p, const yrtmi_image* im,
 		}
 	}
 	p->lpe = best->lanes_per_event;
-	r = brickDone(c, a);
+	r = use.end();
 	if (r)
 		return done(r);
 	// v now holds the EM ratios of x: backproject them through each shape
