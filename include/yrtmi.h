@@ -154,7 +154,7 @@ int yrtmi_ctx_own_stream(yrtmi_ctx* ctx, void** stream);
  * fill / axpby / gather / subset_interleaved / permute / forward_f64 /
  * back_f64.
  * Calls that allocate, copy or synchronise (plan_create, count_segments,
- * histo_subset_nonzero, lor_order, copy, device_alloc/free, lut / histo /
+ * histo_subset_nonzero, lor_order, copy, device_alloc/free, mem_trim, lut / histo /
  * motion uploads, and a first per-XCD backprojection that would allocate its
  * partial images or scratch) fail with YRTMI_ESTATE while recording.
  * A graph may be launched through any context of its device, while the
@@ -347,8 +347,13 @@ int yrtmi_device_alloc(yrtmi_ctx* ctx, int64_t bytes, void** out);
 /* Free and total device memory of the context's device, bytes (HOST
  * pointers, nullable): globals::getAvailableVRAM's cudaMemGetInfo
  * (src/utils/GPUUtils.cu:77), from which OSEM_GPU sizes its batches
- * (getMemAvailable, src/recon/OSEM_GPU.cu:583-591). */
+ * (getMemAvailable, src/recon/OSEM_GPU.cu:583-591).  Memory that the library
+ * keeps for reuse counts as free.  A query only: allowed while recording. */
 int yrtmi_mem_info(yrtmi_ctx* ctx, int64_t* free_bytes, int64_t* total_bytes);
+/* The library keeps up to 16 GiB per device of what plans and its own scratch
+ * gave back, for the next ones; other allocators of the process do not see
+ * it.  Returns it to the driver, as the end of the device's last context does. */
+int yrtmi_mem_trim(yrtmi_ctx* ctx);
 int yrtmi_device_free(yrtmi_ctx* ctx, void* p);
 int yrtmi_copy(yrtmi_ctx* ctx, void* dst, const void* src, int64_t bytes,
                int kind);

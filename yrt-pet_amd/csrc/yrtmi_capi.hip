@@ -2404,14 +2404,26 @@ int yrtmi_mem_info(yrtmi_ctx* c, int64_t* free_bytes, int64_t* total_bytes)
 	int r = setDev(c);
 	if (r)
 		return r;
-	// what the library keeps for reuse counts as free: it goes back first
-	poolTrim(c->device);
 	size_t fr = 0, tot = 0;
 	HIP_TRY(hipMemGetInfo(&fr, &tot));
+	// what the library keeps for reuse counts as free: its own allocations
+	// take it, or give it back where they fail
 	if (free_bytes != nullptr)
-		*free_bytes = (int64_t)fr;
+		*free_bytes = (int64_t)(fr + poolKept(c->device));
 	if (total_bytes != nullptr)
 		*total_bytes = (int64_t)tot;
+	return YRTMI_OK;
+}
+
+int yrtmi_mem_trim(yrtmi_ctx* c)
+{
+	int r = setDev(c);
+	if (r)
+		return r;
+	r = notCapturing(c, "mem_trim");
+	if (r)
+		return r;
+	poolTrim(c->device);
 	return YRTMI_OK;
 }
 

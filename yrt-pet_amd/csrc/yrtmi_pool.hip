@@ -23,6 +23,7 @@ struct Device
 	int contexts = 0;
 	size_t kept = 0;
 	std::list<Block> blocks;  // longest unused first
+	std::vector<void*> unfreed;  // hipFree refused them: tried again
 };
 
 struct Pool
@@ -45,10 +46,19 @@ size_t rounded(size_t b)
 	return (b + g - 1) / g * g;
 }
 
-void freeAll(const std::vector<void*>& v)
+// Gives v back to the driver.  Where that is refused (a thread is recording a
+// graph) the memory is kept for a later try, and no error is left behind for
+// the next call to find.
+void freeAll(int device, const std::vector<void*>& v)
 {
 	for (void* p : v)
-		(void)hipFree(p);
+		if (hipFree(p) != hipSuccess)
+		{
+			(void)hipGetLastError();
+			Pool& P = pool();
+			std::lock_guard<std::mutex> lk(P.m);
+			P.dev[device].unfreed.push_back(p);
+		}
 }
 
 // under the mutex
@@ -56,7 +66,9 @@ void takeAll(Device& d, std::vector<void*>& out)
 {
 	for (const Block& b : d.blocks)
 		out.push_back(b.p);
+	out.insert(out.end(), d.unfreed.begin(), d.unfreed.end());
 	d.blocks.clear();
+	d.unfreed.clear();
 	d.kept = 0;
 }
 
@@ -79,7 +91,7 @@ void poolRelease(int device)
 		if (--d.contexts <= 0)
 			takeAll(d, drop);
 	}
-	freeAll(drop);
+	freeAll(device, drop);
 }
 
 void poolTrim(int device)
@@ -90,7 +102,14 @@ void poolTrim(int device)
 		std::lock_guard<std::mutex> lk(P.m);
 		takeAll(P.dev[device], drop);
 	}
-	freeAll(drop);
+	freeAll(device, drop);
+}
+
+size_t poolKept(int device)
+{
+	Pool& P = pool();
+	std::lock_guard<std::mutex> lk(P.m);
+	return P.dev[device].kept;
 }
 
 hipError_t poolMalloc(int device, void** out, size_t bytes)
@@ -166,7 +185,7 @@ void poolFree(int device, void* p, bool idle)
 			}
 		}
 	}
-	freeAll(drop);
+	freeAll(device, drop);
 }
 
 bool poolQuiesce(int device)
@@ -175,6 +194,8 @@ bool poolQuiesce(int device)
 	(void)hipGetDevice(&cur);
 	(void)hipSetDevice(device);
 	const hipError_t e = hipDeviceSynchronize();
+	if (e != hipSuccess)
+		(void)hipGetLastError();
 	(void)hipSetDevice(cur);
 	return e == hipSuccess;
 }

@@ -7,10 +7,13 @@
 // GPU work ran at 100 ms a round once clean memory had run out.  Blocks given
 // back here are handed out again instead.
 //
-// Per device: at most kPoolBytes are kept (the longest unused go first), all
-// of them return to the driver with the device's last context, before
-// yrtmi_mem_info reports free memory, and when an allocation fails.  Any
-// thread may call; the mutex covers the lists only.
+// Per device: at most kPoolBytes are kept (the longest unused go first); all
+// of them return to the driver with the device's last context, with
+// yrtmi_mem_trim, and when an allocation of the library fails.  Other
+// allocators of the process do not see them.  A block is kept once the device
+// has finished with it (poolQuiesce, or the stream that used it waited for),
+// so it may be handed to any stream.  Any thread may call; the mutex covers the
+// lists only.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -50,5 +53,7 @@ void poolFree(int device, void* p, bool idle);
 bool poolQuiesce(int device);
 // The kept blocks of `device` return to the driver.
 void poolTrim(int device);
+// Bytes of them.
+size_t poolKept(int device);
 
 }  // namespace yrtmi

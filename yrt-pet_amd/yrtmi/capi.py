@@ -125,6 +125,7 @@ _SIGS = {
     "yrtmi_histo_pair_bins": (C.c_int, [_P, _P, _P, C.c_int64, _P]),
     "yrtmi_fill_i32": (C.c_int, [_P, _P, C.c_int64, C.c_int32]),
     "yrtmi_mem_info": (C.c_int, [_P, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
+    "yrtmi_mem_trim": (C.c_int, [_P]),
     "yrtmi_time_average_move": (C.c_int, [_P, C.POINTER(Image), _P, _P, _P, _P, C.c_int]),
     "yrtmi_count_segments": (C.c_int, [_P, _P, C.POINTER(Image), C.POINTER(Lors),
                                        C.POINTER(C.c_int64)]),

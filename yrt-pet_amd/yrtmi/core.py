@@ -395,6 +395,11 @@ class Context:
     def synchronize(self):
         capi.check(capi.lib().yrtmi_ctx_synchronize(self.h))
 
+    def mem_trim(self):
+        """Return the device memory the library keeps for reuse to the driver,
+        e.g. before a large torch allocation (yrtmi_mem_trim)."""
+        capi.check(capi.lib().yrtmi_mem_trim(self.h))
+
     def projector(self, params, with_tof=True):
         return Projector(self, params, with_tof)
 
