@@ -208,8 +208,8 @@ int yrtmi_proj_set_launch(yrtmi_proj* p, int lanes_per_event,
                           int block_size, int grid_blocks);
 /* How backprojections accumulate.  YRTMI_ACCUM_XCD (default): calls of many
  * rays (32768 to 131072 and more, by projector and image size) are binned by
- * image tiles on the device, batch by batch, and summed in LDS as a tile
- * plan's; the context keeps their scratch (at most 1 GiB and, for EM
+ * image tiles on the device, batch by batch, and summed in LDS in FP64 (terms
+ * in FP32, as the atomics'); the context keeps their scratch (at most 1 GiB and, for EM
  * subsets, a copy of the image) between calls.  In smaller calls each XCD
  * adds into its own private copy of the target image (chosen by the hardware
  * XCC id), and the copies are folded into the target by one streaming pass

@@ -3,7 +3,7 @@ tiles on the device: against the same calls with direct accumulation (global
 atomics, never binned).
 
 Bar 1e-5 relative L2, the projector tests' (dyadic voxels: the tile sums are
-exact, the direct ones sum some 10^4 FP32 terms a voxel, whose rounding grows
+FP64, the direct ones sum some 10^4 FP32 terms a voxel, whose rounding grows
 as the square root: 100 x 6e-8).  Below and above the
 rule's thresholds; one, two and many batches; every LOR source; a batch with more records
 than there is room for (it takes the direct kernel)."""
@@ -44,16 +44,16 @@ def setup(im, n, proj="Siddon", rays=1, tof=None, psf=False, fp64=False, frames=
     return ctx, ctx.projector(pp), L, rng
 
 
-def pair(gpu, im, proj, call):
+def pair(gpu, im, proj, call, base=2.0 ** -12):
     """call(img) with per-XCD accumulation (binned) and with direct atomics,
     each into an image that already holds something."""
     out = []
     for xcd in (True, False):
         proj.set_accumulation(xcd)
-        img = torch.full(im.shape, 2.0 ** -12, device=gpu)
+        img = torch.full(im.shape, base, device=gpu)
         call(img)
         torch.cuda.synchronize()
-        out.append((img - 2.0 ** -12).cpu().numpy())
+        out.append((img - base).cpu().numpy())
     r = rel_l2(out[0], out[1])
     print(f"binned vs direct rel L2 {r:.2e}, sum {out[1].sum():.4e}", flush=True)
     assert np.abs(out[1]).sum() > 0
@@ -90,6 +90,28 @@ def test_back_and_em(gpu, case):
          for k in ("meas", "sens", "att", "randoms", "scatter")}
     c["meas"][::5] = 0.0
     pair(gpu, im, p, lambda u: ctx.em_subset(p, im, x, u, L, global_scale=1.5, **c))
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(tof=250.0, rays=4), dict(fp64=True, rays=2),
+                                dict(proj="DD", tof=300.0)], ids=str)
+def test_values_of_different_scales(gpu, kw):
+    """Each term keeps FP32's 24 bits whatever its size beside the call's other
+    values: values over 60 binades in one call and a frame 1e-15 of the
+    others, every voxel against the FP32 atomics.  Bar: some 10^3 terms of one
+    sign a voxel, each rounding 6e-8 of the sum in FP32: 6e-5 at most."""
+    frames = 3
+    im = yrtmi.ImageParams(64, 64, 32, 4.0, 4.0, 2.0, nt=frames)
+    n = 140_000
+    ctx, p, L, rng = setup(im, n, gpu=gpu, frames=frames, **kw)
+    v = 2.0 ** rng.uniform(-60.0, 0.0, n)
+    v = np.where(L.frame.cpu().numpy() == 1, 1e-15 * rng.uniform(0.5, 1.0, n), v)
+    v = torch.from_numpy(v.astype(np.float32)).to(gpu)
+    a, b = pair(gpu, im, p, lambda u: ctx.back(p, im, u, L, v), base=0.0)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    assert (b.reshape(frames, -1).max(1) > 0).all()
+    r = np.abs(a - b)[b > 0] / b[b > 0]
+    print(f"largest relative difference of a voxel {r.max():.2e}", flush=True)
+    assert ((a > 0) == (b > 0)).all() and r.max() <= 6e-5
 
 
 @pytest.mark.parametrize("dd", [False, True])

@@ -463,7 +463,7 @@ bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, in
 // backprojection of 1 M TOF LORs x 4 rays into 200 x 200 x 128 took 19.4 ms
 // and takes 1.4, 150 k DD TOF LORs into 95 x 97 x 47 took 5.6 and take 1.0,
 // an EM subset of 2 M corrected LORs into 181 x 173 x 109 took 35.3 and takes
-// 4.0 (of which its forward 1.6).  The binned path's fixed cost (nine
+// 4.1 (of which its forward 1.6).  The binned path's fixed cost (eight
 // launches a batch, the scan, a pass over the touched tiles) is 70 to 100 us;
 // the direct one's is the fold of its partial images, 30 us at 96 x 96 x 48
 // and 90 us at 200 x 200 x 128.  The lines (streamMinRays) lie where the two
@@ -649,7 +649,6 @@ int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamS
 	rd.rec = pl.rec;
 	rd.ray = table;
 	rd.queue = state->queue;
-	rd.vexp = reinterpret_cast<const int*>(state->queue + 2);
 	rd.nChunksDev = &state->nChunks;
 	rd.err = &state->err;
 	KArgs a = a0;

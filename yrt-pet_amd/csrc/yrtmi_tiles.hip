@@ -500,16 +500,23 @@ hipError_t launchChunkSort(bool dd, const DPlan& pl, const TileChunk* chunks, in
 // can overflow the tile.  The 32^3 shape (whose 64-bit tile would need
 // 256 KB of LDS) accumulates in FP32.
 //
+// SUM64: the tile is summed in FP64 instead (ds_add_f64: any term, no scale,
+// sums good to 2^-53 of their largest partial sum, rounded once at the flush):
+// DD, and calls without a plan (pl.vexp null), whose FP32 atomics kept 24 bits
+// of every term: one 2^-15 of the fixed-point scale and smaller keeps fewer, one
+// below 2^-39 none.  An EM subset of 2 M corrected LORs into 181 x 173 x 109
+// takes 4.08 ms so (fixed point: 3.83; atomics: 35.4), 1 M TOF LORs x 4 rays
+// forward and back at 200 x 200 x 128 2.22 (2.08; 20.5).
+//
 // DD records (DD = true) hold the LOR alone: its table entry (ddEntry) is set
 // up (ddSetup) and its footprint swept over the slices, minor-axis voxels and
 // z planes of the tile (ddVisit), the voxel weights exactly those of the
-// direct sweep.  A footprint's weights have no bound of a few instructions, so
-// DD tiles are summed in FP64 (ds_add_f64: any term, no scale, sums good to
-// 2^-53, rounded once at the flush): the per-term range test and its global
-// atomic, in fixed point, cost more than the slower LDS add (4 M bins of 16
-// frames at 128 x 128 x 96, projection PSF: 28.2 -> 14.1 ms, with the PSF
-// segment table 34.5 before).  Siddon, with more adds an instruction, loses
-// by it: 6.0 -> 7.5 ms for 10 M TOF LORs x 4 rays.
+// direct sweep.  A footprint's weights have no bound of a few instructions, and
+// the per-term range test and its global atomic, in fixed point, cost more
+// than the slower FP64 LDS add (4 M bins of 16 frames at 128 x 128 x 96,
+// projection PSF: 28.2 -> 14.1 ms, with the PSF segment table 34.5 before).
+// Planned Siddon, with more adds an instruction, would lose by it: 6.0 -> 7.5
+// ms for 10 M TOF LORs x 4 rays.
 // The projector's PSF segment tables of one direction (flip: the
 // backprojection's), made in the workgroup's dynamic LDS (DPsf::ldsBytes,
 // given by the DD kernels' launches) by all its threads; the caller waits at
@@ -530,7 +537,7 @@ __device__ __forceinline__ const float4* psfStage(const DPsf& P, bool flip, floa
 	return l;
 }
 
-template <bool DD, bool TOF, bool S64, int SHAPE>
+template <bool DD, bool TOF, bool S64, int SHAPE, bool SUM64>
 __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
                                           const DPlanRead& pl, const TileChunk ch,
                                           const float* __restrict__ v,
@@ -567,9 +574,8 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 	// fixed-point scale of this chunk (uniform)
 	int fixed = 0, k = 0;
 	float climit = 0.f, wbound = 0.f;
-	if constexpr (SHAPE != 2 && !DD)
+	if constexpr (SHAPE != 2 && !SUM64)
 	{
-		if (pl.vexp != nullptr)
 		{
 			// largest voxel weight: a segment is at most the voxel diagonal
 			float wmax = 1.01f * sqrtf(a.im.vx * a.im.vx + a.im.vy * a.im.vy +
@@ -805,9 +811,8 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 	const double scale = ldexp(1.0, k);
 	constexpr double kBias = 6755399441055744.0;  // 1.5 * 2^52
 	constexpr unsigned long long kBiasBits = 0x4338000000000000ull;
-	if constexpr (DD && SHAPE != 2)
+	if constexpr (SUM64)
 	{
-		// DD: FP64 sums
 		wordBytes(8);
 		auto addD = [&](uint32_t idx, int, int, int, float c) {
 			__hip_atomic_fetch_add(
@@ -848,7 +853,7 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 		const int lx = i % TX, ly = (i / TX) % TY, lz = i / (TX * TY);
 		const int gx = B.x0 + lx, gy = B.y0 + ly, gz = B.z0 + lz;
 		float s;
-		if constexpr (DD && SHAPE != 2)
+		if constexpr (SUM64)
 			s = (float)__longlong_as_double((long long)acc64[i]);
 		else
 			s = fixed ? ldexpf((float)(long long)acc64[i], -k) : acc[i];
@@ -861,12 +866,12 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 // One workgroup per chunk (pl.queue == null), or a persistent grid taking
 // chunks from the plan's queue until it is empty.  Every workgroup leaves
 // once the queue index passes the chunk count, so the grid always drains.
-template <bool DD, bool TOF, bool S64, int SHAPE>
+template <bool DD, bool TOF, bool S64, int SHAPE, bool SUM64>
 __global__ void __launch_bounds__(tileThreads(SHAPE))
     kTileBack(KArgs a, DTiles T, DPlanRead pl, const float* __restrict__ v,
               float* __restrict__ y)
 {
-	// NV 64-bit words (fixed point), or NV floats for the 32^3 shape
+	// NV 64-bit words (fixed point or FP64), or NV floats for the 32^3 shape
 	constexpr int NV = tileDim(SHAPE, 0) * tileDim(SHAPE, 1) * tileDim(SHAPE, 2);
 	__shared__ unsigned long long acc[SHAPE == 2 ? NV / 2 : NV];
 	extern __shared__ float4 psfLds[];
@@ -878,7 +883,7 @@ __global__ void __launch_bounds__(tileThreads(SHAPE))
 	}
 	if (pl.queue == nullptr)
 	{
-		tileChunk<DD, TOF, S64, SHAPE>(a, T, pl, pl.chunks[blockIdx.x], v, y, acc, psfL);
+		tileChunk<DD, TOF, S64, SHAPE, SUM64>(a, T, pl, pl.chunks[blockIdx.x], v, y, acc, psfL);
 		return;
 	}
 	if (pl.err != nullptr && *pl.err != 0)
@@ -896,7 +901,7 @@ __global__ void __launch_bounds__(tileThreads(SHAPE))
 		__syncthreads();
 		if (c >= nChunks)
 			break;
-		tileChunk<DD, TOF, S64, SHAPE>(a, T, pl, pl.chunks[c], v, y, acc, psfL);
+		tileChunk<DD, TOF, S64, SHAPE, SUM64>(a, T, pl, pl.chunks[c], v, y, acc, psfL);
 	}
 	if (threadIdx.x == 0)
 	{
@@ -1207,8 +1212,16 @@ template <bool DD, bool TOF, bool S64, int SHAPE>
 static void tileBackT(const KArgs& a, const DTiles& T, const DPlanRead& pl,
                       const float* v, float* y, unsigned grid, hipStream_t st)
 {
-	kTileBack<DD, TOF, S64, SHAPE>
-	    <<<grid, tileThreads(SHAPE), DD ? a.pr.psf.ldsBytes : 0, st>>>(a, T, pl, v, y);
+	auto go = [&](auto k) {
+		k<<<grid, tileThreads(SHAPE), DD ? a.pr.psf.ldsBytes : 0, st>>>(a, T, pl, v, y);
+	};
+	if constexpr (SHAPE == 2)
+		go(kTileBack<DD, TOF, S64, SHAPE, false>);
+	else if constexpr (DD)
+		go(kTileBack<DD, TOF, S64, SHAPE, true>);
+	else
+		pl.vexp == nullptr ? go(kTileBack<DD, TOF, S64, SHAPE, true>)
+		                   : go(kTileBack<DD, TOF, S64, SHAPE, false>);
 }
 
 template <bool DD, bool TOF, bool S64>
