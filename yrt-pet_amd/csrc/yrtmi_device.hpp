@@ -150,14 +150,15 @@ struct DPsf
 	int32_t ldsBytes;
 };
 
-// Segments of a row's interpolant: from each tap, -1 and K - 1 included, to
-// the next.
-__host__ __device__ constexpr int psfSegments(int K) { return K + 1; }
+// Entries of a row's segment table (psfSegment): from each tap, -2 and K
+// included, to the next, and one that holds the whole integral.
+__host__ __device__ constexpr int psfSegments(int K) { return K + 4; }
 
 // Row stride of DPsf::k and DPsf::kflip.
 __host__ __device__ constexpr int psfRowTaps(int K) { return K + 4; }
-// LDS tables of at most this many bytes are staged.
-constexpr int kPsfLdsMax = 21504;
+// LDS tables of at most this many bytes are staged: beside the largest tile, of
+// 128 KB, in the 160 KB of a CU.
+constexpr int kPsfLdsMax = 28672;
 
 struct DProj
 {
@@ -516,40 +517,58 @@ __device__ __forceinline__ float psfWeight(const DPsf& P, const float* kp, const
 	return out;
 }
 
-// psfWeight from the row's segment table: segment s (from tap s - 1) holds
-// {the integral up to it (FP64, two words), ks tap(s - 1), ks (tap(s) -
-// tap(s - 1)) / 2}, so the integral up to x = (s - 1 - half + f) ks is c + f
-// (a + f h): one 16-byte read an end, and 30 VALU an integral where the
-// trapezoids at both ends and the clamps of six reads took ~50.  x / ks is the
-// correctly rounded quotient, as in psfWeight; whole segments are summed in
-// FP64, the parts of the end segments in FP32.
-__device__ __forceinline__ void psfSegment(const float* kp, const double* cum, float ks, int s,
+// psfWeight from the row's segment table: segment e holds the tap at its
+// start, tap e - 2, the next one, and the integral up to it (FP64, two words);
+// taps outside [0, K) are 0, and so is the interpolant in the first and the last
+// segment, which stand for all beyond them.  One 16-byte read an end and the
+// integral up to the segment after x0's, where psfWeight clamps and makes six
+// reads (4 M bins of 16 frames at 128 x 128 x 96: kTileBack 34.5 -> 28.2 ms).
+// The parts at both ends are trapezoids from the crossed tap on, as in
+// psfWeight, and an integral within one segment is one trapezoid: sums of
+// positive terms, so a weight is good to FP32's rounding also where it is a
+// small part of a segment (differences of the integrals up to x1 and x0 are not).
+// x / ks is the correctly rounded quotient, whole segments are summed in FP64.
+__device__ __forceinline__ void psfSegment(const float* kp, const double* cum, int K, int e,
                                            float4* out)
 {
-	const double c = cum[s];
-	const float a = kp[s + 1], b = kp[s + 2];
-	const unsigned long long u = __builtin_bit_cast(unsigned long long, c);
-	*out = make_float4(__uint_as_float((uint32_t)u), __uint_as_float((uint32_t)(u >> 32)), ks * a,
-	                   0.5f * ks * (b - a));
+	const unsigned long long u =
+	    __builtin_bit_cast(unsigned long long, cum[max(min(e - 1, K + 1), 0)]);
+	*out = make_float4(__uint_as_float((uint32_t)u), __uint_as_float((uint32_t)(u >> 32)),
+	                   e < K + 3 ? kp[e] : 0.f, e < K + 3 ? kp[e + 1] : 0.f);
 }
 
 __device__ __forceinline__ float psfWeightTab(const DPsf& P, const float4* tab, float x0, float x1)
 {
 #pragma clang fp contract(off)
 	const int half = (P.K - 1) / 2;
-	const float lim = (float)(half + 1);
-	auto end = [&](float x, double& c) {
-		const float q = fminf(fmaxf(divByRecip(x, P.kSpacing, P.rks), -lim), lim);
-		const float s = fminf(floorf(q), (float)half);
-		const float f = q - s;
-		const float4 e = tab[(int)s + half + 1];
-		c = __builtin_bit_cast(double, ((unsigned long long)__float_as_uint(e.y) << 32) |
-		                                   (unsigned long long)__float_as_uint(e.x));
-		return f * fmaf(f, e.w, e.z);
+	const float lo = (float)(-half - 2), hi = (float)(half + 1);
+	struct End
+	{
+		float s, f, g, v;  // segment, place in it from its start and end, value
+		float4 t;
+		int e;
 	};
-	double c0, c1;
-	const float p0 = end(x0, c0), p1 = end(x1, c1);
-	return x0 < x1 ? (float)(c1 - c0) + (p1 - p0) : 0.f;
+	auto end = [&](float x) {
+		End n;
+		const float q = divByRecip(x, P.kSpacing, P.rks);
+		n.s = floorf(q);
+		n.f = q - n.s;
+		n.g = 1.f - n.f;
+		n.e = (int)fminf(fmaxf(n.s, lo), hi) + half + 2;
+		n.t = tab[n.e];
+		n.v = fmaf(n.t.z, n.g, n.t.w * n.f);
+		return n;
+	};
+	auto upTo = [](const float4& t) {
+		return __builtin_bit_cast(double, ((unsigned long long)__float_as_uint(t.y) << 32) |
+		                                      (unsigned long long)__float_as_uint(t.x));
+	};
+	const End a = end(x0), b = end(x1);
+	const float mid = (float)(upTo(b.t) - upTo(tab[a.e + 1]));
+	const float ends = fmaf(a.v + a.t.w, a.g, (b.t.z + b.v) * b.f);
+	const float w = (a.s == b.s) ? (a.v + b.v) * (0.5f * (x1 - x0))
+	                             : fmaf(0.5f * P.kSpacing, ends, mid);
+	return x0 < x1 ? w : 0.f;
 }
 
 }  // namespace yrtmi

@@ -532,7 +532,7 @@ __device__ __forceinline__ const float4* psfStage(const DPsf& P, bool flip, floa
 	for (int i = threadIdx.x; i < P.numS * ns; i += blockDim.x)
 	{
 		const int row = i / ns;
-		psfSegment(k + row * psfRowTaps(P.K), c + row * (P.K + 2), P.kSpacing, i - row * ns, l + i);
+		psfSegment(k + row * psfRowTaps(P.K), c + row * (P.K + 2), P.K, i - row * ns, l + i);
 	}
 	return l;
 }
@@ -863,11 +863,20 @@ __device__ __forceinline__ void tileChunk(const KArgs& a, const DTiles& T,
 	__syncthreads();  // acc is reused by the next chunk
 }
 
+// Waves a SIMD that a DD tile's LDS leaves room for (16^3 and 32 x 32 x 8: 16 a
+// CU and more); at 131 registers one 32 x 32 x 8 workgroup a CU was left of two
+// (150 k TOF LORs with a PSF at 95 x 97 x 47, forward and back: 1.29 ms, now 1.14).
+__host__ __device__ constexpr int kDDTileWaves(int shape)
+{
+	return shape == 1 ? 2 : 4;
+}
+
 // One workgroup per chunk (pl.queue == null), or a persistent grid taking
 // chunks from the plan's queue until it is empty.  Every workgroup leaves
 // once the queue index passes the chunk count, so the grid always drains.
 template <bool DD, bool TOF, bool S64, int SHAPE, bool SUM64>
 __global__ void __launch_bounds__(tileThreads(SHAPE))
+    __attribute__((amdgpu_waves_per_eu(DD ? kDDTileWaves(SHAPE) : tileThreads(SHAPE) / 256, 8)))
     kTileBack(KArgs a, DTiles T, DPlanRead pl, const float* __restrict__ v,
               float* __restrict__ y)
 {
@@ -1045,8 +1054,11 @@ kEmRatio(KArgs a, float* __restrict__ v)
 // LPE: lanes per LOR, each on every LPE-th slice (a lane per LOR leaves the
 // chip idle in calls of few LORs: the forward of 150 k TOF LORs of 95 x 97 x
 // 47 with a PSF 0.49 -> 0.40 ms); one where there are LORs enough.
+// Four waves a SIMD where that needs no spill.
 template <bool TOF, bool S64, bool TAB, bool BRICK, int LPE>
-__global__ void __launch_bounds__(256) kEmRatioDD(KArgs a, float* __restrict__ v)
+__global__ void __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu((TAB || (!S64 && BRICK)) ? 4 : 1, 8)))
+kEmRatioDD(KArgs a, float* __restrict__ v)
 {
 	extern __shared__ float4 psfLds[];
 	const float4* psfL = psfStage(a.pr.psf, false, psfLds);
