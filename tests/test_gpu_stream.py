@@ -114,6 +114,48 @@ def test_values_of_different_scales(gpu, kw):
     assert ((a > 0) == (b > 0)).all() and r.max() <= 6e-5
 
 
+@pytest.mark.parametrize("kw", [dict(rays=4, tof=250.0), dict(rays=3, frames=2, fp64=True),
+                                dict(proj="DD", tof=300.0)], ids=str)
+@pytest.mark.parametrize("keep", [0.0, 3e-5, 0.03, 1.0])
+def test_em_subset_of_few_nonzero_lors(gpu, kw, keep):
+    """EM subsets that skip most of their LORs (measurement, sensitivity or
+    attenuation 0), or all, or none: the others are listed first."""
+    im = yrtmi.ImageParams(64, 60, 30, 4.0, 4.5, 2.0, nt=max(1, kw.get("frames", 0)))
+    n = 300_001
+    ctx, p, L, _ = setup(im, n, gpu=gpu, **kw)
+    g = torch.Generator(gpu).manual_seed(5)
+    x = 0.5 + torch.rand(im.shape, device=gpu, generator=g)
+    c = {k: 0.2 + torch.rand(n, device=gpu, generator=g)
+         for k in ("meas", "sens", "att", "randoms", "scatter")}
+    for k in ("meas", "sens", "att"):
+        c[k][torch.rand(n, device=gpu, generator=g) >= keep ** (1 / 3)] = 0.0
+    on = int(((c["meas"] != 0) & (c["sens"] != 0) & (c["att"] != 0)).sum())
+    print(f"{on} of {n} LORs", flush=True)
+    if on == 0:
+        u = torch.zeros(im.shape, device=gpu)
+        ctx.em_subset(p, im, x, u, L, **c)
+        assert float(u.abs().max()) == 0.0
+    else:
+        pair(gpu, im, p, lambda u: ctx.em_subset(p, im, x, u, L, **c))
+        pair(gpu, im, p, lambda u: ctx.em_subset(p, im, x, u, L, att=c["att"]))
+
+
+def test_em_subset_listed_in_two_parts(gpu):
+    """More LORs than are listed at a time (2^24), batches ending inside both."""
+    im = yrtmi.ImageParams(64, 60, 30, 4.0, 4.5, 2.0)
+    n = (1 << 24) + 1_234_567
+    ctx, p, _, _ = setup(im, 10, gpu=gpu)
+    g = torch.Generator(gpu).manual_seed(5)
+    d = [torch.randint(0, 128 * 24, (n,), device=gpu, generator=g, dtype=torch.int32)
+         for _ in range(2)]
+    L = yrtmi.LorSet.pairs(*d)
+    meas = torch.rand(n, device=gpu, generator=g)
+    meas[::2] = 0.0
+    meas[100_000:200_000] = 0.0
+    x = 0.5 + torch.rand(im.shape, device=gpu, generator=g)
+    pair(gpu, im, p, lambda u: ctx.em_subset(p, im, x, u, L, meas=meas))
+
+
 @pytest.mark.parametrize("dd", [False, True])
 @pytest.mark.parametrize("att", [False, True])
 def test_sensitivity_of_histogram_subset(gpu, dd, att):

@@ -476,6 +476,8 @@ bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, in
 // ---------------------------------------------------------------------------
 constexpr size_t kStreamBytes = size_t(1) << 30;  // scratch per context
 constexpr int kStreamBinGroups = 1024;
+// LORs of which an EM subset lists those it does not skip, at a time (64 MiB).
+constexpr int64_t kStreamList = int64_t(1) << 24;
 
 int64_t streamMinRays(const KArgs& a)
 {
@@ -496,10 +498,12 @@ struct StreamShape
 	int persistent = 0;  // tile kernel workgroups
 	bool dd = false;
 	int64_t brick = 0;   // floats of the bricked image (EM)
+	int64_t list = 0;    // LORs listed at a time (EM with factors that may be 0)
 	size_t fixedBytes() const
 	{
 		return sizeof(StreamState) + (size_t)nB * 20 + (size_t)kStreamBinGroups * nB * 4 +
-		       (size_t)(T.nTiles + 2048) * sizeof(TileChunk) + (size_t)brick * 4 + 16 * 256;
+		       (size_t)(T.nTiles + 2048) * sizeof(TileChunk) + (size_t)brick * 4 +
+		       (list > 0 ? ((size_t)list + kListWaves + 1) * 4 : 0) + 16 * 256;
 	}
 	size_t lorBytes() const
 	{
@@ -537,6 +541,7 @@ bool streamShape(yrtmi_ctx* c, const KArgs& a, bool em, StreamShape& s)
 	s.recPer = s.dd ? std::min<int64_t>(128, 8 * std::max(s.T.ntx, s.T.nty))
 	                : std::min<int64_t>(64, s.T.ntx + s.T.nty + s.T.ntz - 2);
 	s.brick = (em && useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt)) ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt : 0;
+	s.list = (em && (a.c.meas || a.c.sens || a.c.att)) ? std::min(a.L.n, kStreamList) : 0;
 	return true;
 }
 
@@ -636,6 +641,9 @@ int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamS
 	pl.err = &state->err;
 	pl.skip = &state->err;
 	float* brick = (float*)take((size_t)s.brick * 4);
+	uint32_t* list = (uint32_t*)take((size_t)s.list * 4);
+	uint32_t* listPart = (uint32_t*)take(s.list > 0 ? (kListWaves + 1) * 4 : 0);
+	uint32_t* listed = listPart + kListWaves;
 	float* v = (float*)take((size_t)batch * 4);
 	float4* table = (float4*)take((size_t)batch * s.R * s.tabVec * sizeof(float4));
 	const int64_t cap = batch * s.R * s.recPer;
@@ -666,10 +674,37 @@ int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamS
 		a.bvox = brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz);
 	}
 	auto shift = [](const float* q, int64_t b) { return q ? q + b : nullptr; };
-	for (int64_t b = 0; b < n; b += batch)
+	// an EM subset with factors: the LORs it does not skip are listed first and
+	// the batches taken from the list (those past its end find nothing to do), so
+	// a subset of mostly zero bins costs what its others do.  13.6 M bins x 4
+	// rays at 200 x 200 x 128, all / 1 in 100 / 1 in 1000 not 0: direct 169 / 3.6 /
+	// 0.93 ms, every bin in the batches 25.7 / 12.4 / 10.3, listed 26.2 / 1.8 / 1.2
+	const int64_t span = s.list > 0 ? s.list : n;
+	for (int64_t b = 0, l0 = 0; b < n; b = std::min(std::min(n, l0 + span), b + batch))
 	{
-		const int64_t e = std::min(n, b + batch);
-		a.L = sliceLors(a0.L, b, e);
+		if (b == l0 + span)
+			l0 = b;
+		const int64_t lEnd = std::min(n, l0 + span), e = std::min(lEnd, b + batch);
+		a.L = sliceLors(a0.L, s.list > 0 ? l0 : b, e);
+		a.L.n = e - b;
+		if (kind == STREAM_EM)
+		{
+			const int64_t first = s.list > 0 ? l0 : b;
+			a.c.meas = shift(a0.c.meas, first);
+			a.c.sens = shift(a0.c.sens, first);
+			a.c.att = shift(a0.c.att, first);
+			a.c.randoms = shift(a0.c.randoms, first);
+			a.c.scatter = shift(a0.c.scatter, first);
+			a.c.precorr = shift(a0.c.precorr, first);
+		}
+		if (s.list > 0)
+		{
+			if (b == l0)
+				HIP_TRY(launchLorList(a.c, lEnd - l0, listPart, list, listed, st));
+			a.list = list;
+			a.listed = pl.listed = listed;
+			a.listFirst = pl.listFirst = b - l0;
+		}
 		const int64_t rays = a.L.n * (int64_t)s.R;
 		const int grid =
 		    (int)std::min<int64_t>((rays + kBinThreads - 1) / kBinThreads, kStreamBinGroups);
@@ -690,12 +725,6 @@ int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamS
 		}
 		else
 		{
-			a.c.meas = shift(a0.c.meas, b);
-			a.c.sens = shift(a0.c.sens, b);
-			a.c.att = shift(a0.c.att, b);
-			a.c.randoms = shift(a0.c.randoms, b);
-			a.c.scatter = shift(a0.c.scatter, b);
-			a.c.precorr = shift(a0.c.precorr, b);
 			a.rays = s.dd ? table : nullptr;
 			HIP_TRY(launchEmRatio(a, p->lpe, v, st));
 		}

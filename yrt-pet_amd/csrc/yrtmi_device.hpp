@@ -238,7 +238,24 @@ struct KArgs
 	const float* xb;
 	int64_t bvox;
 	int32_t plain;  // the EM ratio kernels write the projection itself
+	// With `list`, the call's LOR i is L's (and c's) element list[i]: the LORs
+	// that an EM subset does not skip (launchLorList), of which there are
+	// *listed, from element listFirst on, at most L.n.
+	const uint32_t* list;
+	const uint32_t* listed;
+	int64_t listFirst;
 };
+
+// The number of LORs of the call, and the element of L and c that is LOR i.
+__device__ __forceinline__ int64_t lorCount(const KArgs& a)
+{
+	return a.list == nullptr ? a.L.n
+	                         : min(a.L.n, max((int64_t)0, (int64_t)*a.listed - a.listFirst));
+}
+__device__ __forceinline__ int64_t lorElement(const KArgs& a, int64_t i)
+{
+	return a.list == nullptr ? i : (int64_t)a.list[a.listFirst + i];
+}
 
 // Hardware id of the XCD (accelerator complex die) running this wave.
 __device__ __forceinline__ uint32_t xccId()

@@ -196,9 +196,10 @@ __global__ void __launch_bounds__(256) kBackIf(KArgs a, const int* __restrict__ 
 		return;
 	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
 	uint32_t cnt = 0;
-	for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < a.L.n; e += stride)
+	const int64_t n = lorCount(a);
+	for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += stride)
 	{
-		const Lor l = fetchLor(a.sc, a.L, e, a.im.nt);
+		const Lor l = fetchLor(a.sc, a.L, lorElement(a, e), a.im.nt);
 		if (l.frame >= 0 && a.vals[e] != 0.f)
 			backLane<TYPE, TOF, 1, S64, MODE_BACK>(a, l, 0, a.y + (int64_t)l.frame * a.im.nvox,
 			                                       a.vals[e], cnt);

@@ -55,13 +55,13 @@ template <bool DD, bool TOF, bool S64>
 __global__ void __launch_bounds__(256) kRayPrep(KArgs a, float4* __restrict__ tab, int* err)
 {
 	const int R = a.pr.numRays;
-	const int64_t total = a.L.n * (int64_t)R;
+	const int64_t total = lorCount(a) * (int64_t)R;
 	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
 	for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride)
 	{
 		const int64_t e = t / R;
 		const int r = (int)(t - e * R);
-		const Lor l = fetchLor(a.sc, a.L, e, a.im.nt);
+		const Lor l = fetchLor(a.sc, a.L, lorElement(a, e), a.im.nt);
 		if (DD)
 		{
 			if (l.frame < 0)
@@ -287,6 +287,8 @@ __global__ void __launch_bounds__(kBinThreads) kBin(DImage im, DProj pr, int64_t
 	const int nB = T.nTiles * pl.C;
 	int* cnt = sm;
 	uint32_t* base = reinterpret_cast<uint32_t*>(sm + nB);
+	if (pl.listed != nullptr)
+		nRays = min(nRays, max((int64_t)0, (int64_t)*pl.listed - pl.listFirst) * pl.R);
 	const int64_t per = (nRays + gridDim.x - 1) / gridDim.x;
 	const int64_t tEnd = min(nRays, (int64_t)(blockIdx.x + 1) * per);
 	const int64_t t0 = (int64_t)blockIdx.x * per + threadIdx.x;
@@ -1001,17 +1003,18 @@ __device__ __forceinline__ float siddonPart(const DImage& P, const float* __rest
 // (the LUT stays in L2; a plan's ray table, read from HBM, measured slower).
 // BRICK: gathers from the bricked copy of x (a.xb; useBricks), else from x.
 // PARTS: lanes per ray, in turn along it (kSplitRays; the FP32 set-up's).
-template <bool TOF, int LPE, bool S64, bool BRICK, int PARTS>
+// LIST: of listed LORs (KArgs::list; two registers more, which at 96 spill).
+template <bool TOF, int LPE, bool S64, bool BRICK, int PARTS, bool LIST>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(S64 ? 4 : 5, 8)))
 kEmRatio(KArgs a, float* __restrict__ v)
 {
 	constexpr int lanes = LPE * PARTS;
-	const int64_t total = a.L.n * lanes;
+	const int64_t total = (LIST ? lorCount(a) : a.L.n) * lanes;
 	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
 	for (int64_t t = xcdRange(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; t < total;
 	     t += stride)
 	{
-		const int64_t e = t / lanes;
+		const int64_t e = LIST ? lorElement(a, t / lanes) : t / lanes;
 		const int lane = (int)(t & (lanes - 1));
 		const Lor l = fetchLor(a.sc, a.L, e, a.im.nt);
 		const float m = a.c.meas ? a.c.meas[e] : 1.0f;
@@ -1042,7 +1045,7 @@ kEmRatio(KArgs a, float* __restrict__ v)
 		for (int o = 1; o < lanes; o <<= 1)
 			s += __shfl_xor(s, o, lanes);
 		if (lane == 0)
-			v[e] = skip ? 0.f : emRatioOut(a, e, s, m, sf, af);
+			v[LIST ? t / lanes : e] = skip ? 0.f : emRatioOut(a, e, s, m, sf, af);
 	}
 }
 
@@ -1055,7 +1058,8 @@ kEmRatio(KArgs a, float* __restrict__ v)
 // chip idle in calls of few LORs: the forward of 150 k TOF LORs of 95 x 97 x
 // 47 with a PSF 0.49 -> 0.40 ms); one where there are LORs enough.
 // Four waves a SIMD where that needs no spill.
-template <bool TOF, bool S64, bool TAB, bool BRICK, int LPE>
+// LIST: as for Siddon.
+template <bool TOF, bool S64, bool TAB, bool BRICK, int LPE, bool LIST>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu((TAB || (!S64 && BRICK)) ? 4 : 1, 8)))
 kEmRatioDD(KArgs a, float* __restrict__ v)
@@ -1064,10 +1068,11 @@ kEmRatioDD(KArgs a, float* __restrict__ v)
 	const float4* psfL = psfStage(a.pr.psf, false, psfLds);
 	__syncthreads();
 	const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-	for (int64_t t = xcdRange(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; t < a.L.n * LPE;
+	const int64_t total = (LIST ? lorCount(a) : a.L.n) * LPE;
+	for (int64_t t = xcdRange(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; t < total;
 	     t += stride)
 	{
-		const int64_t e = t / LPE;
+		const int64_t i = t / LPE, e = LIST ? lorElement(a, i) : i;
 		const int lane = (int)(t & (LPE - 1));
 		const float m = a.c.meas ? a.c.meas[e] : 1.0f;
 		const float sf = a.c.sens ? a.c.sens[e] : 1.0f;
@@ -1077,7 +1082,7 @@ kEmRatioDD(KArgs a, float* __restrict__ v)
 		float4 de[kDDVec];
 		if (TAB)
 		{
-			de[5] = a.rays[kDDVec * e + 5];
+			de[5] = a.rays[kDDVec * i + 5];
 			frame = ddFrame(de[5]);
 		}
 		else
@@ -1093,9 +1098,9 @@ kEmRatioDD(KArgs a, float* __restrict__ v)
 			if (TAB)
 			{
 #pragma unroll
-				for (int i = 0; i < kDDVec; i++)
-					if (i != 5)
-						de[i] = a.rays[kDDVec * e + i];
+				for (int k = 0; k < kDDVec; k++)
+					if (k != 5)
+						de[k] = a.rays[kDDVec * i + k];
 				ddLoad(a.im, a.pr, de, false, D);
 			}
 			else
@@ -1119,7 +1124,7 @@ kEmRatioDD(KArgs a, float* __restrict__ v)
 		for (int o = 1; o < LPE; o <<= 1)
 			s += __shfl_xor(s, o, LPE);
 		if (lane == 0)
-			v[e] = skip ? 0.f : emRatioOut(a, e, s, m, sf, af);
+			v[i] = skip ? 0.f : emRatioOut(a, e, s, m, sf, af);
 	}
 }
 
@@ -1367,6 +1372,47 @@ hipError_t launchClearWords(unsigned int* p, int64_t words, hipStream_t st)
 	return hipGetLastError();
 }
 
+// The LORs that an EM subset does not skip (m, sf and af, where given, not 0):
+// one wave per stretch of the LORs (kListWaves of them), in order.
+// PASS 0 counts each stretch's into part, kListScan makes them starts, PASS 1
+// writes the list.
+__device__ __forceinline__ int64_t listStretch(int64_t n)
+{
+	return ((n + kListWaves - 1) / kListWaves + 63) / 64 * 64;
+}
+
+template <int PASS>
+__global__ void __launch_bounds__(256) kLorList(DCorr c, int64_t n, uint32_t* __restrict__ part,
+                                                uint32_t* __restrict__ list)
+{
+	const int lane = (int)(threadIdx.x & 63u);
+	const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), per = listStretch(n);
+	const int64_t b = w * per, e = min(n, b + per);
+	const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+	uint32_t at = PASS == 0 ? 0u : part[w];
+	for (int64_t i0 = b; i0 < e; i0 += 256)
+	{
+		bool on[4];
+#pragma unroll
+		for (int k = 0; k < 4; k++)
+		{
+			const int64_t i = min(i0 + 64 * k + lane, n - 1);
+			on[k] = i0 + 64 * k + lane < e && !(c.meas && c.meas[i] == 0.f) &&
+			        !(c.sens && c.sens[i] == 0.f) && !(c.att && c.att[i] == 0.f);
+		}
+#pragma unroll
+		for (int k = 0; k < 4; k++)
+		{
+			const uint64_t m = __ballot(on[k]);
+			if (PASS == 1 && on[k])
+				list[at + (uint32_t)__popcll(m & below)] = (uint32_t)(i0 + 64 * k + lane);
+			at += (uint32_t)__popcll(m);
+		}
+	}
+	if (PASS == 0 && lane == 0)
+		part[w] = at;
+}
+
 // Exclusive prefix of v over the workgroup's 1024 threads; *total, its sum.
 __device__ __forceinline__ unsigned long long scan1024(unsigned long long v,
                                                        unsigned long long* lds,
@@ -1455,6 +1501,35 @@ __global__ void __launch_bounds__(1024)
 		s->nChunks = (int64_t)(nFull + nPart);
 }
 
+__global__ void __launch_bounds__(1024) kListScan(uint32_t* __restrict__ part,
+                                                  uint32_t* __restrict__ listed)
+{
+	__shared__ unsigned long long lds[16];
+	constexpr int per = kListWaves / 1024;
+	uint32_t* p = part + per * threadIdx.x;
+	unsigned long long sum = 0, total;
+	for (int k = 0; k < per; k++)
+		sum += p[k];
+	uint32_t at = (uint32_t)scan1024(sum, lds, &total);
+	for (int k = 0; k < per; k++)
+	{
+		const uint32_t q = p[k];
+		p[k] = at;
+		at += q;
+	}
+	if (threadIdx.x == 0)
+		*listed = (uint32_t)total;
+}
+
+hipError_t launchLorList(const DCorr& c, int64_t n, uint32_t* part, uint32_t* list,
+                         uint32_t* listed, hipStream_t st)
+{
+	kLorList<0><<<kListWaves / 4, 256, 0, st>>>(c, n, part, nullptr);
+	kListScan<<<1, 1024, 0, st>>>(part, listed);
+	kLorList<1><<<kListWaves / 4, 256, 0, st>>>(c, n, part, list);
+	return hipGetLastError();
+}
+
 hipError_t launchStreamScan(const DPlan& pl, int64_t* tileOff, int nTiles, int64_t cap,
                             TileChunk* chunks, StreamState* s, hipStream_t st)
 {
@@ -1506,10 +1581,13 @@ static hipError_t ratioLpe(const KArgs& a, int lpe, int parts, dim3 g, float* v,
 		if constexpr (!S64)
 			if (parts > 1)
 			{
-				kEmRatio<TOF, N, S64, BRICK, kRayParts><<<g, 256, 0, st>>>(a, v);
+				kEmRatio<TOF, N, S64, BRICK, kRayParts, false><<<g, 256, 0, st>>>(a, v);
 				return;
 			}
-		kEmRatio<TOF, N, S64, BRICK, 1><<<g, 256, 0, st>>>(a, v);
+		if (a.list != nullptr)
+			kEmRatio<TOF, N, S64, BRICK, 1, true><<<g, 256, 0, st>>>(a, v);
+		else
+			kEmRatio<TOF, N, S64, BRICK, 1, false><<<g, 256, 0, st>>>(a, v);
 	};
 	switch (lpe)
 	{
@@ -1539,7 +1617,15 @@ static hipError_t ratioT(const KArgs& a, int lpe, int parts, dim3 g, float* v, h
 		auto go = [&](auto k) { k<<<g, 256, a.pr.psf.ldsBytes, st>>>(a, v); };
 		auto lanes = [&](auto tab, auto brick) {
 			constexpr bool T = decltype(tab)::value, B = decltype(brick)::value;
-			lpe == 4 ? go(kEmRatioDD<TOF, S64, T, B, 4>) : go(kEmRatioDD<TOF, S64, T, B, 1>);
+			if constexpr (T)
+				if (a.list != nullptr)
+				{
+					lpe == 4 ? go(kEmRatioDD<TOF, S64, T, B, 4, true>)
+					         : go(kEmRatioDD<TOF, S64, T, B, 1, true>);
+					return;
+				}
+			lpe == 4 ? go(kEmRatioDD<TOF, S64, T, B, 4, false>)
+			         : go(kEmRatioDD<TOF, S64, T, B, 1, false>);
 		};
 		using Y = std::true_type;
 		using N = std::false_type;
@@ -1587,7 +1673,9 @@ hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st)
 		return hipErrorInvalidValue;
 	if (a.pr.type == 1)
 		lpe = a.L.n <= kDDLanesUpTo ? 4 : 1;
-	const int parts = a.pr.type == 0 && !a.pr.setup64 &&
+	if (a.list != nullptr && a.pr.type == 1 && a.rays == nullptr)
+		return hipErrorInvalidValue;
+	const int parts = a.pr.type == 0 && !a.pr.setup64 && a.list == nullptr &&
 	                          a.L.n * (int64_t)a.pr.numRays <= kSplitRays
 	                      ? kRayParts
 	                      : 1;

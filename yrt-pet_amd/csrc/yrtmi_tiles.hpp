@@ -119,6 +119,8 @@ struct DPlan
 	const float4* ray;          // ray table (rayEntry + sidStore / ddStore, kRayPrep)
 	int* err;                   // set when a tile range would overflow
 	const int* skip;            // (nullable) the fill pass does nothing if set
+	const uint32_t* listed;     // (nullable) LORs there are, as KArgs::listed
+	int64_t listFirst;
 };
 
 // Cuts of a plan's length classes (DPlan::cut) for its number of classes.
@@ -218,6 +220,12 @@ struct StreamState
 };
 // Clears `words` 32-bit words.
 hipError_t launchClearWords(unsigned int* p, int64_t words, hipStream_t st);
+// list = the elements below n (> 0) of the LORs that an EM subset with these
+// corrections does not skip, in order; *listed, their number; part, kListWaves
+// words of scratch.
+constexpr int kListWaves = 4096;
+hipError_t launchLorList(const DCorr& c, int64_t n, uint32_t* part, uint32_t* list,
+                         uint32_t* listed, hipStream_t st);
 // From pl.count: pl.tileOff, the chunk table (chunkRecords of the total,
 // full chunks first) and s->nChunks; s->err |= 4 and no chunks when there
 // are more than `cap` records or an error before.  One workgroup.
