@@ -173,9 +173,9 @@ def test_sensitivity_of_histogram_subset(gpu, dd, att):
     pair(gpu, im, p, lambda u: ctx.back(p, im, u, B, v))
 
 
-def test_batch_without_room_takes_the_direct_kernel(gpu):
+def test_batch_of_high_footprints(gpu):
     """Crystals 240 voxels high over one column of 64 tiles: some 30 records
-    for each LOR that meets the image, where there is room for 8 per LOR."""
+    for each LOR that meets the image, for which there is room."""
     im = yrtmi.ImageParams(32, 32, 512, 4.0, 4.0, 0.25)
     ctx, p, L, _ = setup(im, 70_000, proj="DD", gpu=gpu,
                          sc=("t", 128.0, 60.0, 4.0, 10.0, 180.0, 128, 2))
@@ -183,6 +183,34 @@ def test_batch_without_room_takes_the_direct_kernel(gpu):
     plan = ctx.plan(p, im, L, tile_shape=3)
     assert plan.info()["records"] > 8 * L.n
     pair(gpu, im, p, lambda u: ctx.back(p, im, u, L, v))
+
+
+@pytest.mark.parametrize("kind", ["back", "em", "em_listed", "sens"])
+@pytest.mark.parametrize("kw", [dict(), dict(tof=3000.0), dict(fp64=True)], ids=str)
+def test_batch_with_more_records_than_room(gpu, kind, kw):
+    """Rays from a tall image's first ring to its last, some 100 tiles each
+    (TOF too wide to cut them), where there is room for 64: the batch takes the
+    direct kernel (kBackIf)."""
+    im = yrtmi.ImageParams(32, 32, 1024, 4.0, 4.0, 0.25)
+    n = 140_000
+    ctx, p, _, rng = setup(im, 10, gpu=gpu, sc=("t", 256.0, 4.0, 3.4, 10.0, 70.0, 128, 64), **kw)
+    i = rng.integers(0, 128, n)
+    j = (i + rng.integers(48, 81, n)) % 128
+    t = lambda a, d: torch.from_numpy(a.astype(d)).to(gpu)
+    tof = t(rng.normal(0.0, 100.0, n), np.float32) if "tof" in kw else None
+    L = yrtmi.LorSet.pairs(t(i, np.int32), t(j + 128 * 63, np.int32), tof=tof)
+    records = ctx.plan(p, im, L, tile_shape=3).info()["records"]
+    print(f"{records / n:.1f} records a ray", flush=True)
+    assert records > 64 * n
+    g = torch.Generator(gpu).manual_seed(1)
+    v = 0.5 + torch.rand(n, device=gpu, generator=g)
+    x = 0.5 + torch.rand(im.shape, device=gpu, generator=g)
+    mu = 0.01 * torch.rand(im.shape, device=gpu, generator=g)
+    pair(gpu, im, p, {
+        "back": lambda u: ctx.back(p, im, u, L, v),
+        "em": lambda u: ctx.em_subset(p, im, x, u, L),
+        "em_listed": lambda u: ctx.em_subset(p, im, x, u, L, meas=v),
+        "sens": lambda u: ctx.sensitivity(p, im, u, L, att_im=im, att_img=mu, sens=v)}[kind])
 
 
 def test_recorded_and_on_other_streams(gpu):

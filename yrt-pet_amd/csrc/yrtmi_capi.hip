@@ -536,10 +536,13 @@ bool streamShape(yrtmi_ctx* c, const KArgs& a, bool em, StreamShape& s)
 	while (s.C < 8 && s.T.nTiles * s.C * 2 <= 4096)
 		s.C *= 2;
 	s.nB = (int64_t)s.T.nTiles * s.C;
-	// a ray crosses at most one tile face per tile and axis; a footprint's
-	// records are not bounded so (a batch of more takes the direct kernel)
-	s.recPer = s.dd ? std::min<int64_t>(128, 8 * std::max(s.T.ntx, s.T.nty))
+	// a ray crosses at most one tile face per tile and axis (a batch of more than
+	// 64 a ray, steep ones in a tall image, takes the direct kernel, kBackIf)
+	s.recPer = s.dd ? ddRecordsPerLor(s.T, a.im.vx, a.im.vy, a.im.vz, a.pr.tt, a.pr.tz,
+	                                  a.pr.psf.k != nullptr ? a.pr.psf.halfWidth : 0.f)
 	                : std::min<int64_t>(64, s.T.ntx + s.T.nty + s.T.ntz - 2);
+	if (s.recPer > kStreamRecords)
+		return false;
 	s.brick = (em && useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt)) ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt : 0;
 	s.list = (em && (a.c.meas || a.c.sens || a.c.att)) ? std::min(a.L.n, kStreamList) : 0;
 	return true;

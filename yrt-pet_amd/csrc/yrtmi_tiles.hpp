@@ -159,6 +159,24 @@ inline DTiles tilesOf(int shape, int64_t nx, int64_t ny, int64_t nz, int64_t nt)
 	return T;
 }
 
+// Room for the records of one DD footprint that calls without a plan leave, on
+// the average of a batch.  An interval of l voxels at any offset meets 1 + l / T
+// tiles of T on average: in each slab of tiles along the major axis the
+// footprint's minor range, its width (crystal, PSF extent ext) and what the line
+// moves across the slab, at most a slab's length; axially its height, and over
+// all slabs what the line rises, at most the image.  8 per slab at least, up to 128
+// (footprints of a few voxels: mostly below 4).
+inline int64_t ddRecordsPerLor(const DTiles& T, float vx, float vy, float vz, float tt, float tz,
+                               float ext)
+{
+	const double slabs = std::max(T.ntx, T.nty), vMin = std::min(vx, vy), vMax = std::max(vx, vy);
+	const double minor = 1.0 + vMax / vMin + (1.5 * tt + 2.0 * ext) / vMin / T.tx;
+	const double r = minor * (slabs * (1.0 + (double)tz / vz / T.tz) + T.ntz);
+	return std::max((int64_t)std::min(128.0, 8.0 * slabs), (int64_t)std::min(r + 1.0, 1e9));
+}
+// More than this: the direct kernel.
+constexpr int64_t kStreamRecords = 512;
+
 // Ray table of a Siddon plan, rayTabVec(S64) float4 per (LOR, ray) t = lor *
 // R + ray.  The first two: the ray's end points after multi-ray offsets,
 // motion and the image offset (q1, q2, exactly as the walk sets it up) and
