@@ -223,6 +223,9 @@ int yrtmi_proj_set_accumulation(yrtmi_proj* p, int mode);
 
 /* ---- projections --------------------------------------------------------
  * Forward: out[i] = (A x)_i for each LOR of `lors` (device out, n floats).
+ * An image whose frames have 2^21 voxels and more is read from a copy in 4 x 4 x
+ * 2-voxel bricks, in a buffer the context keeps (same values, same sums), where
+ * there is a ray for every 4 voxels and memory for it.
  * Replaces OperatorProjectorDevice::applyA (OperatorProjectorDevice.cu:
  * 442-544) -> projectSiddon_kernel / projectDD_kernel<true,...>. */
 int yrtmi_forward(yrtmi_ctx* ctx, const yrtmi_proj* p, const yrtmi_image* im,

@@ -101,3 +101,37 @@ def test_free_memory_is_a_query(gpu):
     ctx.mem_trim()
     # (blocks below the driver's 2 MiB granule may stay in one with live memory)
     assert driver_free() >= held + kept - (16 << 20)
+
+
+def test_memory_bounds(gpu):
+    """A plan within a budget takes no larger kept block than it counts, and the
+    scratch of calls without a plan stays within its 1 GiB as it grows."""
+    ctx, p, im, L, _ = kept_plan(gpu, 480_000)
+    ctx.mem_trim()
+    plan = ctx.plan(p, im, L)
+    del plan  # kept: every block 1.2 times what the next plan needs
+    S = L.slice(0, 400_000)
+    free = free_bytes(ctx)
+    opt = capi.PlanOptions(0, 0, 0, 1 << 32, 0)
+    h, ci, cl, b = C.c_void_p(), im.c(), S.c(), C.c_int64()
+    capi.check(capi.lib().yrtmi_plan_create(ctx.h, p.h, C.byref(ci), C.byref(cl), C.byref(opt),
+                                            C.byref(h)))
+    capi.check(capi.lib().yrtmi_plan_info(h, None, None, C.byref(b)))
+    taken = free - free_bytes(ctx)
+    capi.lib().yrtmi_plan_destroy(h)
+    print(f"plan counts {b.value >> 20} MiB, took {taken >> 20}", flush=True)
+    assert b.value > 64 << 20 and taken <= b.value + (16 << 20)  # (five blocks' rounding)
+
+    d1 = torch.randint(0, 128 * 24, (6_000_000,), device=gpu, dtype=torch.int32)
+    d2 = d1.flip(0).contiguous()
+    v = torch.ones(d1.numel(), device=gpu)
+    u = torch.zeros(im.shape, device=gpu)
+    torch.cuda.synchronize()
+    ctx.mem_trim()
+    free = free_bytes(ctx)
+    for k in (1_450_000, 1_800_000, 6_000_000):
+        ctx.back(p, im, u, yrtmi.LorSet.pairs(d1[:k], d2[:k]), v)
+        ctx.synchronize()
+        took = free - free_bytes(ctx)
+        print(f"{k} LORs: scratch {took >> 20} MiB", flush=True)
+        assert 600 << 20 < took <= (1 << 30) + (16 << 20)

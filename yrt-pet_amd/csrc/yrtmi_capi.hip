@@ -372,9 +372,10 @@ private:
 	std::unique_lock<std::mutex> m_lock;  // (of m_s: released before it)
 };
 
-// At least `bytes` of scratch; false where there is no memory for it, or the
-// context's stream is being captured and there is less.
-bool reserve(yrtmi_ctx* c, ScratchPtr& w, int rank, size_t bytes)
+// At least `bytes` of scratch, and half as much again as there is, up to `upTo`,
+// where it has to grow; false where there is no memory for it, or the context's
+// stream is being captured and there is less.
+bool reserve(yrtmi_ctx* c, ScratchPtr& w, int rank, size_t bytes, size_t upTo = 0)
 {
 	const size_t have = w ? w->bytes : 0;
 	if (have >= bytes)
@@ -384,7 +385,7 @@ bool reserve(yrtmi_ctx* c, ScratchPtr& w, int rank, size_t bytes)
 	auto q = std::make_shared<Scratch>();
 	q->device = c->device;
 	q->rank = rank;
-	q->bytes = std::max(bytes, have + have / 2);
+	q->bytes = std::max(bytes, std::min(have + have / 2, upTo));
 	if (poolAlloc(c->device, &q->p, q->bytes) != hipSuccess)
 	{
 		(void)hipGetLastError();
@@ -474,7 +475,8 @@ bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, in
 //   DD                      32 k LORs  back 404-993 / 388-863 EM 440-1245 / 574-1313
 //                           65 k LORs  back 518-1544 / 419-938 EM 650-1901 / 591-1386
 // ---------------------------------------------------------------------------
-constexpr size_t kStreamBytes = size_t(1) << 30;  // scratch per context
+// scratch per context, beside an EM subset's copy of the image
+constexpr size_t kStreamBytes = size_t(1) << 30;
 constexpr int kStreamBinGroups = 1024;
 // LORs of which an EM subset lists those it does not skip, at a time (64 MiB).
 constexpr int64_t kStreamList = int64_t(1) << 24;
@@ -584,9 +586,8 @@ bool streamReady(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a, bool em, Str
 		return false;
 	const size_t want =
 	    std::max(s.fixedBytes() + (size_t)std::min<int64_t>(n, 1 << 26) * s.lorBytes(), size_t(1));
-	const size_t cap = std::max(std::min(want, kStreamBytes + (size_t)s.brick * 4),
-	                            s.fixedBytes() + (size_t)((least + s.R) / s.R) * s.lorBytes());
-	(void)reserve(c, c->ws, 1, cap);  // else what there is
+	const size_t most = kStreamBytes + (size_t)s.brick * 4;
+	(void)reserve(c, c->ws, 1, std::min(want, most), most);  // else what there is
 	const int64_t b = streamBatch(c, s, n);
 	return b == n || b * s.R >= least;
 }
@@ -2066,6 +2067,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	// [0] next chunk, [1] finished workgroups (persistent launches),
 	// [2] fixed-point scale exponent of the current launch, [3] workgroups
 	// done counting, [4 .. 259] exponent histogram of its values (kVExpScale)
+	const bool exact = o.max_bytes > 0;  // the memory counted is the memory taken
 	if (poolAlloc(c->device, &q->queue, 260 * sizeof(unsigned int)) != hipSuccess ||
 	    hipMemsetAsync(q->queue, 0, 260 * sizeof(unsigned int), c->stream) != hipSuccess)
 	{
@@ -2073,7 +2075,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 		return fail(YRTMI_ENOMEM, "plan: chunk queue");
 	}
 	if (l->n > 0)
-		if (poolAlloc(c->device, &q->v, sizeof(float) * l->n) != hipSuccess)
+		if (poolAlloc(c->device, &q->v, sizeof(float) * l->n, exact) != hipSuccess)
 		{
 			freePlan(q);
 			return fail(YRTMI_ENOMEM, "plan: value buffer");
@@ -2121,7 +2123,7 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	    poolAlloc(c->device, &dOff, sizeof(int64_t) * nB) != hipSuccess ||
 	    poolAlloc(c->device, &dErr, sizeof(int)) != hipSuccess)
 		return cleanup(fail(YRTMI_ENOMEM, "plan: build scratch"));
-	if (poolAlloc(c->device, &q->ray, tabVec * sizeof(float4) * rays) != hipSuccess)
+	if (poolAlloc(c->device, &q->ray, tabVec * sizeof(float4) * rays, exact) != hipSuccess)
 		return cleanup(fail(YRTMI_ENOMEM, "plan: ray table"));
 	q->bytes += rays * tabVec * (int64_t)sizeof(float4);
 	hipError_t e = hipMemsetAsync(dCount, 0, sizeof(unsigned long long) * nB, c->stream);
@@ -2197,8 +2199,10 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	if (total > 0)
 	{
 		// records of 12 B (Siddon) / 8 B (DD: no alpha)
-		if (poolAlloc(c->device, &q->rec, sizeof(uint32_t) * recWords(dd) * total) != hipSuccess ||
-		    poolAlloc(c->device, &q->chunks, sizeof(TileChunk) * chunks.size()) != hipSuccess)
+		if (poolAlloc(c->device, &q->rec, sizeof(uint32_t) * recWords(dd) * total, exact) !=
+		        hipSuccess ||
+		    poolAlloc(c->device, &q->chunks, sizeof(TileChunk) * chunks.size(), exact) !=
+		        hipSuccess)
 			return cleanup(fail(YRTMI_ENOMEM, "plan: records"));
 		q->bytes += total * (dd ? 8 : 12) + (int64_t)(sizeof(TileChunk) * chunks.size());
 		e = hipMemcpyAsync(dOff, off.data(), sizeof(int64_t) * nB,

@@ -124,16 +124,16 @@ hipError_t poolMalloc(int device, void** out, size_t bytes)
 	return e;
 }
 
-hipError_t poolAlloc(int device, void** out, size_t bytes)
+hipError_t poolAlloc(int device, void** out, size_t bytes, bool exact)
 {
 	Pool& P = pool();
-	const size_t need = rounded(bytes);
+	const size_t need = rounded(bytes), slack = exact ? 0 : need / 4 + (size_t(1) << 20);
 	{
 		std::lock_guard<std::mutex> lk(P.m);
 		Device& d = P.dev[device];
 		auto best = d.blocks.end();
 		for (auto it = d.blocks.begin(); it != d.blocks.end(); ++it)
-			if (it->bytes >= need && it->bytes <= need + need / 4 + (size_t(1) << 20) &&
+			if (it->bytes >= need && it->bytes <= need + slack &&
 			    (best == d.blocks.end() || it->bytes < best->bytes))
 				best = it;
 		if (best != d.blocks.end())

@@ -29,12 +29,14 @@ constexpr size_t kPoolBytes = size_t(16) << 30;
 // Context count of a device (create / destroy).
 void poolRetain(int device);
 void poolRelease(int device);
-// *out = at least `bytes` (> 0) bytes on `device`, which is current.
-hipError_t poolAlloc(int device, void** out, size_t bytes);
+// *out = at least `bytes` (> 0) bytes on `device`, which is current: a kept
+// block of up to a quarter (and 1 MiB) more than that, or, with `exact`, of no
+// more than the pool's rounding, else new memory.
+hipError_t poolAlloc(int device, void** out, size_t bytes, bool exact = false);
 template <class T>
-hipError_t poolAlloc(int device, T** out, size_t bytes)
+hipError_t poolAlloc(int device, T** out, size_t bytes, bool exact = false)
 {
-	return poolAlloc(device, reinterpret_cast<void**>(out), bytes);
+	return poolAlloc(device, reinterpret_cast<void**>(out), bytes, exact);
 }
 // hipMalloc, once more with the kept blocks returned where it fails: for
 // memory that is not given back through the pool.
