@@ -202,8 +202,11 @@ int yrtmi_motion_upload(yrtmi_ctx* ctx, const float* xf, int k);
 int yrtmi_proj_create(yrtmi_ctx* ctx, const yrtmi_projector_desc* d,
                       yrtmi_proj** out);
 int yrtmi_proj_destroy(yrtmi_proj* p);
-/* Launch shape: lanes cooperating on one event (1, 2, 4 or 8; they split the
- * rays), threads per block, and blocks (0 = sized from the event count). */
+/* Launch shape of forwards and of the calls without a plan that take the direct kernels:
+ * lanes cooperating on one event (1, 2, 4 or 8; they split the rays; small
+ * calls put up to 4 lanes on each ray or DD LOR besides), threads per block, and
+ * blocks (0 = sized from the event count; a forward rounds up to a multiple of
+ * 8).  EM ratios take the lanes only. */
 int yrtmi_proj_set_launch(yrtmi_proj* p, int lanes_per_event,
                           int block_size, int grid_blocks);
 /* How backprojections accumulate.  YRTMI_ACCUM_XCD (default): calls of many

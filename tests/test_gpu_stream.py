@@ -363,3 +363,33 @@ def test_forward_lanes_along_a_ray(gpu, dims, kw):
     ref, y, z = y.abs().max().item(), y.cpu().numpy()[:at], z.cpu().numpy()[:at]
     print(f"lanes rel L2 {rel_l2(z, y):.2e} max {np.abs(z - y).max() / ref:.2e}", flush=True)
     assert ref > 0 and rel_l2(z, y) <= 1e-5 and np.abs(z - y).max() <= 1e-4 * ref
+
+
+@pytest.mark.parametrize("dims", [(33, 65, 17, 4.0, 4.0, 4.0), (161, 127, 103, 1.5, 1.75, 1.0)],
+                         ids=str)
+@pytest.mark.parametrize("kw", [dict(rays=3), dict(proj="DD")], ids=str)
+def test_launch_shape_of_forwards(gpu, dims, kw):
+    """Forwards with the block and grid that the caller set, by way of small
+    calls (several lanes a ray or LOR), bricks, and neither: the same sums.  (A
+    grid far too small for the LORs is seen by its time: one block of 64
+    threads against the whole chip.)"""
+    im = yrtmi.ImageParams(*dims)
+    n = 540_000 // kw.get("rays", 1)
+    ctx, p, L, _ = setup(im, n, gpu=gpu, **kw)
+    x = 0.5 + torch.rand(im.shape, device=gpu, generator=torch.Generator(gpu).manual_seed(2))
+    for S in (L, L.slice(0, 10_001)):
+        y, z = torch.zeros(S.n, device=gpu), torch.full((S.n,), -1.0, device=gpu)
+        ctx.forward(p, im, x, S, y)
+        times = []
+        for block, grid in ((256, 0), (64, 0), (192, 24), (128, 8)):
+            p.set_launch(block=block, grid=grid)
+            t = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            t[0].record()
+            ctx.forward(p, im, x, S, z.fill_(-1.0))
+            t[1].record()
+            torch.cuda.synchronize()
+            times.append(t[0].elapsed_time(t[1]))
+            assert float(y.abs().sum()) > 0 and torch.equal(y, z)
+        p.set_launch()
+        print("ms:", " ".join(f"{k:.3f}" for k in times), flush=True)
+        assert times[3] > 2 * times[1]

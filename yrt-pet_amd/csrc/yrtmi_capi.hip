@@ -1353,7 +1353,7 @@ int yrtmi_forward(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	                                : !a.pr.setup64 && l->n * (int64_t)a.pr.numRays <= kSplitRays))
 	{
 		a.plain = 1;
-		HIP_TRY(launchEmRatio(a, p->lpe, out, c->stream));
+		HIP_TRY(launchEmRatio(a, p->lpe, out, c->stream, p->block, p->grid));
 		return use.end();
 	}
 	a.out = out;

@@ -1574,20 +1574,21 @@ hipError_t launchTileBack(const KArgs& a, const DTiles& T, const DPlanRead& pl,
 }
 
 template <bool TOF, bool S64, bool BRICK>
-static hipError_t ratioLpe(const KArgs& a, int lpe, int parts, dim3 g, float* v, hipStream_t st)
+static hipError_t ratioLpe(const KArgs& a, int lpe, int parts, dim3 g, dim3 b, float* v,
+                           hipStream_t st)
 {
 	auto go = [&](auto lanes) {
 		constexpr int N = decltype(lanes)::value;
 		if constexpr (!S64)
 			if (parts > 1)
 			{
-				kEmRatio<TOF, N, S64, BRICK, kRayParts, false><<<g, 256, 0, st>>>(a, v);
+				kEmRatio<TOF, N, S64, BRICK, kRayParts, false><<<g, b, 0, st>>>(a, v);
 				return;
 			}
 		if (a.list != nullptr)
-			kEmRatio<TOF, N, S64, BRICK, 1, true><<<g, 256, 0, st>>>(a, v);
+			kEmRatio<TOF, N, S64, BRICK, 1, true><<<g, b, 0, st>>>(a, v);
 		else
-			kEmRatio<TOF, N, S64, BRICK, 1, false><<<g, 256, 0, st>>>(a, v);
+			kEmRatio<TOF, N, S64, BRICK, 1, false><<<g, b, 0, st>>>(a, v);
 	};
 	switch (lpe)
 	{
@@ -1610,11 +1611,12 @@ static hipError_t ratioLpe(const KArgs& a, int lpe, int parts, dim3 g, float* v,
 }
 
 template <bool TOF, bool S64>
-static hipError_t ratioT(const KArgs& a, int lpe, int parts, dim3 g, float* v, hipStream_t st)
+static hipError_t ratioT(const KArgs& a, int lpe, int parts, dim3 g, dim3 b, float* v,
+                         hipStream_t st)
 {
 	if (a.pr.type == 1)
 	{
-		auto go = [&](auto k) { k<<<g, 256, a.pr.psf.ldsBytes, st>>>(a, v); };
+		auto go = [&](auto k) { k<<<g, b, a.pr.psf.ldsBytes, st>>>(a, v); };
 		auto lanes = [&](auto tab, auto brick) {
 			constexpr bool T = decltype(tab)::value, B = decltype(brick)::value;
 			if constexpr (T)
@@ -1635,8 +1637,8 @@ static hipError_t ratioT(const KArgs& a, int lpe, int parts, dim3 g, float* v, h
 			a.rays != nullptr ? lanes(Y{}, N{}) : lanes(N{}, N{});
 		return hipGetLastError();
 	}
-	return a.xb != nullptr ? ratioLpe<TOF, S64, true>(a, lpe, parts, g, v, st)
-	                       : ratioLpe<TOF, S64, false>(a, lpe, parts, g, v, st);
+	return a.xb != nullptr ? ratioLpe<TOF, S64, true>(a, lpe, parts, g, b, v, st)
+	                       : ratioLpe<TOF, S64, false>(a, lpe, parts, g, b, v, st);
 }
 
 // One workgroup per row of bricks (y, z), its threads along it: no division
@@ -1667,7 +1669,8 @@ hipError_t launchToBricks(const DImage& im, const float* x, float* xb, hipStream
 	return hipGetLastError();
 }
 
-hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st)
+hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st, int block,
+                         int64_t grid)
 {
 	if (a.xb != nullptr && a.bvox != brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz))
 		return hipErrorInvalidValue;
@@ -1680,19 +1683,19 @@ hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st)
 	                      ? kRayParts
 	                      : 1;
 	const int64_t threads = a.L.n * lpe * parts;
-	int64_t nb = (threads + 255) / 256;
+	int64_t nb = grid > 0 ? grid : (threads + block - 1) / block;
 	if (nb > 0x7ffffff0)
 		nb = 0x7ffffff0;
 	nb = (nb + kXcds - 1) / kXcds * kXcds;  // xcdRange is a bijection on [0, nb)
 	if (nb < kXcds)
 		nb = kXcds;
-	const dim3 g((unsigned)nb);
+	const dim3 g((unsigned)nb), b((unsigned)block);
 	const bool tof = a.pr.useTof != 0;
 	if (a.pr.setup64)
-		return tof ? ratioT<true, true>(a, lpe, parts, g, v, st)
-		           : ratioT<false, true>(a, lpe, parts, g, v, st);
-	return tof ? ratioT<true, false>(a, lpe, parts, g, v, st)
-	           : ratioT<false, false>(a, lpe, parts, g, v, st);
+		return tof ? ratioT<true, true>(a, lpe, parts, g, b, v, st)
+		           : ratioT<false, true>(a, lpe, parts, g, b, v, st);
+	return tof ? ratioT<true, false>(a, lpe, parts, g, b, v, st)
+	           : ratioT<false, false>(a, lpe, parts, g, b, v, st);
 }
 
 hipError_t launchSensValue(const KArgs& a, float* v, hipStream_t st)

@@ -300,8 +300,10 @@ inline bool useBricks(int64_t nx, int64_t ny, int64_t nz, int64_t frames)
 hipError_t launchToBricks(const DImage& im, const float* x, float* xb, hipStream_t st);
 // v[e] = EM ratio of LOR e (0 where skipped), or with a.plain its projection,
 // Siddon or DD (a.pr.type); Siddon reads a.xb (launchToBricks of a.x) where
-// it is given, else a.x.
-hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st);
+// it is given, else a.x.  block threads (64 to 256, full waves) and grid
+// workgroups (0: from the LORs), the latter rounded up to a multiple of 8.
+hipError_t launchEmRatio(const KArgs& a, int lpe, float* v, hipStream_t st, int block = 256,
+                         int64_t grid = 0);
 // v[e] = sensitivity value of LOR e (factor x attenuation).
 hipError_t launchSensValue(const KArgs& a, float* v, hipStream_t st);
 
