@@ -592,20 +592,15 @@ bool streamReady(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a, bool em, Str
 	return b == n || b * s.R >= least;
 }
 
-// v = the sensitivity value of each LOR of a.L.
-int sensValue(yrtmi_ctx* c, KArgs a, float* v)
+// The attenuation image for the sensitivity values of a.L: its bricked copy
+// (a.xb) where that is worth it.  The caller ends the use after the last launch.
+int sensImage(yrtmi_ctx* c, KArgs& a, ScratchUse& use)
 {
 	int r = YRTMI_OK;
 	a.xb = nullptr;
-	KArgs s = a;
-	ScratchUse use;
 	if (a.att != nullptr)
-		(void)brickForward(c, s, a.attIm, a.att, a.L.n, use, &r);
-	if (r)
-		return r;
-	a.xb = s.xb;
-	HIP_TRY(launchSensValue(a, v, c->stream));
-	return use.end();
+		(void)brickForward(c, a, a.attIm, a.att, a.L.n, use, &r);
+	return r;
 }
 
 enum StreamKind
@@ -618,7 +613,7 @@ enum StreamKind
 int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamShape& s,
                StreamKind kind, float* y, const float* vals)
 {
-	ScratchUse use;
+	ScratchUse use, attUse;
 	int r = use.begin(c, c->ws);
 	if (r)
 		return r;
@@ -670,6 +665,9 @@ int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamS
 		// frame 0 of the image, without TOF
 		a.pr.useTof = 0;
 		a.im.nt = 1;
+		r = sensImage(c, a, attUse);
+		if (r)
+			return r;
 	}
 	if (s.brick > 0)
 	{
@@ -723,9 +721,7 @@ int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamS
 		else if (kind == STREAM_SENS)
 		{
 			a.vals = shift(a0.vals, b);
-			r = sensValue(c, a, v);
-			if (r)
-				return r;
+			HIP_TRY(launchSensValue(a, v, st));
 		}
 		else
 		{
@@ -737,7 +733,8 @@ int streamBack(yrtmi_ctx* c, const yrtmi_proj* p, const KArgs& a0, const StreamS
 		a.y = y;
 		HIP_TRY(launchBackIf(a, rd.err, st));
 	}
-	return use.end();
+	r = attUse.end();
+	return r ? r : use.end();
 }
 
 // Set up per-XCD accumulation for a backprojection of n voxels into y, or
@@ -2423,7 +2420,12 @@ int yrtmi_sensitivity_planned(yrtmi_ctx* c, const yrtmi_proj* p,
 	}
 	a.vals = sens;
 	a.L.tof = nullptr;
-	r = sensValue(c, a, q->v);
+	ScratchUse use;
+	r = sensImage(c, a, use);
+	if (r)
+		return r;
+	HIP_TRY(launchSensValue(a, q->v, c->stream));
+	r = use.end();
 	if (r)
 		return r;
 	HIP_TRY(launchTileBack(a, q->T, planRead(q), q->v, img, q->persistent, c->stream));
