@@ -20,6 +20,9 @@ CASES = [
     ((40, 40, 40), (63, 63, 63), 1),
     ((5, 2, 1), (1, 3, 9), 3),
     ((48, 7, 200), (9, 9, 31), 1),
+    # more than 65535 tiles along y, and columns along z
+    ((1, 2_200_000, 2), (3, 5, 1), 1),
+    ((1_100_000, 2, 1), (1, 3, 5), 1),
 ]
 
 

@@ -74,15 +74,16 @@ __host__ __device__ constexpr int psfPitch(int hx) { return (kPsfTX + 2 * hx + 7
 
 __global__ void __launch_bounds__(256) kPsfXY(const float* __restrict__ in,
                                               float* __restrict__ out, PsfTaps tx, PsfTaps ty,
-                                              int nx, int ny, int TY)
+                                              int nx, int ny, int TY, unsigned gx)
 {
 	extern __shared__ float sm[];
 	const int hx = tx.n / 2, hy = ty.n / 2;
 	const int pitch = psfPitch(hx), rows = TY + 2 * hy;
 	float* patch = sm;
 	float* mid = sm + pitch * rows;  // rows of kPsfTX, kPsfTX + 1 apart
-	const int x0 = (int)blockIdx.x * kPsfTX, y0 = (int)blockIdx.y * TY;
-	const int64_t plane = (int64_t)blockIdx.z * nx * ny;
+	// (a plane's tiles along blockIdx.x, which alone is not held to 65535)
+	const int x0 = (int)(blockIdx.x % gx) * kPsfTX, y0 = (int)(blockIdx.x / gx) * TY;
+	const int64_t plane = (int64_t)blockIdx.y * nx * ny;
 	// util::circular (Tools.cpp:160-167): one wrap (h < n); elements that no
 	// output inside the image needs are read somewhere inside it
 	auto wrap = [](int q, int n) {
@@ -151,13 +152,14 @@ __global__ void __launch_bounds__(256) kPsfXY(const float* __restrict__ in,
 constexpr int kPsfMz = 16;
 
 __global__ void __launch_bounds__(256) kPsfZ(const float* __restrict__ in,
-                                             float* __restrict__ out, PsfTaps t, int nxy, int nz)
+                                             float* __restrict__ out, PsfTaps t, int nxy, int nz,
+                                             unsigned gc)
 {
-	const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+	const int i = (int)(blockIdx.x % gc * blockDim.x + threadIdx.x);
 	if (i >= nxy)
 		return;
-	const int z0 = (int)blockIdx.y * kPsfMz;
-	const float* p = in + (int64_t)blockIdx.z * nxy * nz + i;
+	const int z0 = (int)(blockIdx.x / gc) * kPsfMz;
+	const float* p = in + (int64_t)blockIdx.y * nxy * nz + i;
 	float acc[kPsfMz];
 	convolveLine<kPsfMz>(
 	    t,
@@ -167,7 +169,7 @@ __global__ void __launch_bounds__(256) kPsfZ(const float* __restrict__ in,
 		    return p[(int64_t)(q < nz ? q : 0) * nxy];
 	    },
 	    acc);
-	float* o = out + (int64_t)blockIdx.z * nxy * nz + i;
+	float* o = out + (int64_t)blockIdx.y * nxy * nz + i;
 #pragma unroll
 	for (int j = 0; j < kPsfMz; j++)
 		if (z0 + j < nz)
@@ -190,11 +192,11 @@ hipError_t launchPsf(const float* in, float* tmp, float* out, const PsfTaps* t, 
 	// (a grid has at most 65535 planes and frames)
 	const int64_t planes = frames * nz;
 	for (int64_t p = 0; p < planes; p += 65535)
-		kPsfXY<<<dim3(gx, gy, (unsigned)std::min<int64_t>(65535, planes - p)), 256, lds, st>>>(
-		    in + p * nxy, tmp + p * nxy, t[0], t[1], nx, ny, TY);
+		kPsfXY<<<dim3(gx * gy, (unsigned)std::min<int64_t>(65535, planes - p)), 256, lds, st>>>(
+		    in + p * nxy, tmp + p * nxy, t[0], t[1], nx, ny, TY, gx);
 	for (int64_t f = 0; f < frames; f += 65535)
-		kPsfZ<<<dim3(gc, gz, (unsigned)std::min<int64_t>(65535, frames - f)), 256, 0, st>>>(
-		    tmp + f * nz * nxy, out + f * nz * nxy, t[2], nxy, nz);
+		kPsfZ<<<dim3(gc * gz, (unsigned)std::min<int64_t>(65535, frames - f)), 256, 0, st>>>(
+		    tmp + f * nz * nxy, out + f * nz * nxy, t[2], nxy, nz, gc);
 	return hipGetLastError();
 }
 
