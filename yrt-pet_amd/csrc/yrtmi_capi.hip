@@ -2009,10 +2009,12 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 		return fail(YRTMI_EINVAL, "plan: image dimensions above 1024");
 	if (useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt))
 	{
-		// the bricked image of the planned EM ratio, sized here
+		// the bricked image of the planned EM ratio, sized here (a DD ratio does
+		// without where there is no memory for it)
 		if (!reserve(c, c->em, 0,
 		             sizeof(float) *
-		                 (size_t)(brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt)))
+		                 (size_t)(brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt)) &&
+		    !dd)
 			return fail(YRTMI_ENOMEM, "plan: bricked image");
 	}
 	const int R = p->d.numRays;
