@@ -226,9 +226,10 @@ int yrtmi_proj_set_accumulation(yrtmi_proj* p, int mode);
 
 /* ---- projections --------------------------------------------------------
  * Forward: out[i] = (A x)_i for each LOR of `lors` (device out, n floats).
- * An image whose frames have 2^21 voxels and more is read from a copy in 4 x 4 x
- * 2-voxel bricks, in a buffer the context keeps (same values, same sums), where
- * there is a ray for every 4 voxels and memory for it.
+ * A large image (2^21 voxels and more; in long calls of up to 3 rays per LOR, or
+ * DD, 2^18 or 2^20) is read from a copy in 4 x 4 x 2-voxel bricks, in a buffer the
+ * context keeps (same values, same sums), where there is a ray for every 4 voxels
+ * and memory for it.
  * Replaces OperatorProjectorDevice::applyA (OperatorProjectorDevice.cu:
  * 442-544) -> projectSiddon_kernel / projectDD_kernel<true,...>. */
 int yrtmi_forward(yrtmi_ctx* ctx, const yrtmi_proj* p, const yrtmi_image* im,
@@ -552,11 +553,12 @@ int yrtmi_em_subset_planned(yrtmi_ctx* ctx, const yrtmi_proj* p,
  * EM ratio of LOR i (m / corrected forward projection, times the
  * multiplicative corrections), 0 where the reference skips the LOR.
  * yrtmi_em_subset_planned = yrtmi_em_ratio_planned + yrtmi_back_planned(v).
- * Images of 2^21 voxels and more are projected from a bricked copy of x made
+ * Large images (as for yrtmi_forward) are projected from a bricked copy of x made
  * at each call into a buffer the context keeps (4 x 4 x 2-voxel bricks; same
  * values, same sums): it grows on the first call of a larger image, or when a
- * plan is created, which a caller recording a graph of a Siddon ratio must do
- * before recording (a DD ratio reads x itself where there is no buffer).
+ * plan is created, which a caller recording a graph of a Siddon ratio of 2^21
+ * voxels and more must do before recording (others read x itself where there is
+ * no buffer).
  * Replaces the forward half of OSEM_CPU::computeEMUpdateImage
  * (src/recon/OSEM_CPU.cpp:329-374). */
 int yrtmi_em_ratio(yrtmi_ctx* ctx, const yrtmi_proj* p, const yrtmi_image* im,

@@ -3,9 +3,9 @@
 
 extern "C" {
 
-int hw_use_bricks(int64_t nx, int64_t ny, int64_t nz, int64_t frames)
+int hw_use_bricks(int64_t nx, int64_t ny, int64_t nz, int64_t frames, int dd, int rays, int64_t n)
 {
-	return yrtmi::useBricks(nx, ny, nz, frames);
+	return yrtmi::useBricks(nx, ny, nz, frames, dd != 0, rays, n);
 }
 
 // Records per LOR that a DD backprojection without a plan has room for, with

@@ -248,25 +248,43 @@ def test_recorded_and_on_other_streams(gpu):
         assert a <= 1e-5 and b <= 1e-5
 
 
-@pytest.mark.parametrize("kw", [dict(rays=2, tof=250.0), dict(rays=3, frames=2), dict(rays=5),
-                                dict(rays=2, tof=300.0, fp64=True)], ids=str)
-def test_bricked_forward_is_the_forward(gpu, kw):
+LARGE = (161, 127, 103, 1.5, 1.75, 1.0)   # 2^21 voxels and more
+SMALL = (67, 65, 63, 4.0, 4.0, 4.0)       # 2^18 and more: bricks from 2^19 rays
+BRICKED = [(LARGE, dict(rays=1, tof=250.0)), (LARGE, dict(rays=2, tof=250.0)),
+           (LARGE, dict(rays=3, frames=2)), (LARGE, dict(rays=5)),
+           (LARGE, dict(rays=2, tof=300.0, fp64=True)), (SMALL, dict(rays=1)),
+           (SMALL, dict(rays=3, tof=250.0, frames=2))]
+
+
+@pytest.mark.parametrize("dims,kw", BRICKED, ids=str)
+def test_bricked_forward_is_the_forward(gpu, dims, kw):
     """A forward of many rays of a large image gathers from its bricked copy;
     calls of a third of its LORs do not: the same sums, bit for bit, also
-    recorded and replayed, and the attenuation of a sensitivity image too."""
+    recorded and replayed, and the EM ratio's (1 / A x without measurements)
+    against its reciprocal's rounding."""
     nt = max(1, kw.get("frames", 0))
-    im = yrtmi.ImageParams(161, 127, 103, 1.5, 1.75, 1.0, nt=nt)
-    n = (im.nvox * nt // 4) // kw["rays"] + 1000
+    R = kw["rays"]
+    im = yrtmi.ImageParams(*dims, nt=nt)
+    step = max(im.nvox * nt // 12, (1 << 19) // 3) // R + 1000
+    n = 3 * step
+    # bricked all together, rows in thirds, which are above the calls of several
+    # lanes a ray
+    if dims is LARGE:
+        assert im.nvox >= 1 << 21 and 4 * n * R >= im.nvox * nt > 4 * step * R
+    else:
+        assert im.nvox >= 1 << 18 and n * R >= 1 << 19 > step * R
+    assert step * R > 65536
     ctx, p, L, _ = setup(im, n, gpu=gpu, **kw)
     x = torch.rand(im.shape, device=gpu, generator=torch.Generator(gpu).manual_seed(2))
     y, z = torch.zeros(n, device=gpu), torch.zeros(n, device=gpu)
     ctx.forward(p, im, x, L, y)
-    step = n // 3
     for a in range(0, n, step):
-        b = min(n, a + step)
-        ctx.forward(p, im, x, L.slice(a, b), z[a:b])
+        ctx.forward(p, im, x, L.slice(a, a + step), z[a:a + step])
     torch.cuda.synchronize()
     assert float(y.abs().sum()) > 0 and torch.equal(y, z)
+    ctx.em_ratio(p, im, x, L, z)
+    on = y > 1e-6
+    assert float((z * y - 1.0)[on].abs().max()) <= 4e-7
     s = torch.cuda.Stream()
     ctx.set_stream(s)
     with ctx.graph() as g:

@@ -20,7 +20,7 @@ def hw(tmp_path_factory):
                     os.path.join(HERE, "hostwalk", "rules_host.cpp"), "-o", out],
                    check=True, capture_output=True)
     lib = C.CDLL(out)
-    lib.hw_use_bricks.argtypes = [C.c_int64] * 4
+    lib.hw_use_bricks.argtypes = [C.c_int64] * 4 + [C.c_int] * 2 + [C.c_int64]
     lib.hw_dd_records.argtypes = [C.c_int64] * 3 + [C.c_float] * 6
     lib.hw_dd_records.restype = C.c_int64
     return lib
@@ -36,7 +36,20 @@ def hw(tmp_path_factory):
     ((1, 1, (1 << 27) - 2), 1, True),
 ])
 def test_bricks_are_indexed_in_32_bits(hw, dims, frames, want):
-    assert bool(hw.hw_use_bricks(*dims, frames)) == want
+    assert bool(hw.hw_use_bricks(*dims, frames, 0, 1, 1000)) == want
+
+
+@pytest.mark.parametrize("dims,frames,dd,rays,n,want", [
+    ((128, 128, 128), 1, 0, 4, 1000, True), ((128, 128, 127), 1, 0, 4, 1 << 30, False),
+    ((128, 128, 64), 16, 0, 6, 1 << 30, False),  # a frame at a time
+    ((128, 128, 128), 1, 0, 1, 1, True), ((128, 128, 64), 2, 0, 3, 1, True),
+    ((64, 64, 64), 1, 0, 1, 1 << 19, True), ((64, 64, 64), 1, 0, 1, (1 << 19) - 1, False),
+    ((64, 64, 64), 1, 0, 2, 1 << 18, True), ((64, 64, 63), 1, 0, 3, 1 << 30, False),
+    ((128, 128, 64), 1, 1, 1, 1 << 17, True), ((128, 128, 64), 1, 1, 1, (1 << 17) - 1, False),
+    ((128, 128, 63), 1, 1, 1, 1 << 30, False), ((96, 96, 48), 16, 1, 1, 1, True),
+])
+def test_bricks_by_rays_and_length(hw, dims, frames, dd, rays, n, want):
+    assert bool(hw.hw_use_bricks(*dims, frames, dd, rays, n)) == want
 
 
 @pytest.mark.gpu

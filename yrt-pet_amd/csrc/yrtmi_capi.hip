@@ -395,20 +395,27 @@ bool reserve(yrtmi_ctx* c, ScratchPtr& w, int rank, size_t bytes, size_t upTo = 
 	return true;
 }
 
-// The bricked copy of a.x for the EM ratio's forward; small images are read
-// as they are, and so is a DD call's while recording without the buffer
-// (Siddon refuses that), or captured by the caller.  The caller ends the use
+// useBricks for the forward part of a call.
+bool callBricks(const KArgs& a, const DImage& im)
+{
+	return useBricks(im.nx, im.ny, im.nz, im.nt, a.pr.type == YRTMI_PROJ_DD, a.pr.numRays,
+	                 a.L.n);
+}
+
+// The bricked copy of a.x for the EM ratio's forward by useBricks' rule; the image
+// is read as it is while recording without the buffer (a Siddon call of 2^21
+// voxels and more is refused that) and by a DD call that the caller captures.  The caller ends the use
 // after its launch.  Tile plans reserve the buffer for their image, so planned
 // EM calls never allocate.
 int brickImage(yrtmi_ctx* c, KArgs& a, ScratchUse& use)
 {
-	if (!useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt))
+	if (!callBricks(a, a.im))
 		return YRTMI_OK;
 	const int64_t bvox = brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz);
 	const bool dd = a.pr.type == YRTMI_PROJ_DD;
 	if ((dd && callerCaptures(c)) ||
 	    !reserve(c, c->em, 0, sizeof(float) * (size_t)(bvox * a.im.nt)))
-		return dd
+		return dd || a.im.nvox * a.im.nt < kBrickVoxels
 		           ? YRTMI_OK
 		           : notCapturing(c,
 		                          "bricked image (run one EM ratio of this size before recording)");
@@ -423,21 +430,19 @@ int brickImage(yrtmi_ctx* c, KArgs& a, ScratchUse& use)
 
 constexpr int64_t kBrickRays = 4;  // voxels a ray above which it is not
 
-// A forward projection of `rays` rays of image `im` reads a bricked
-// copy of it (a.xb, in c->fwd), where the copy, ~3 ps
-// a voxel, is worth it: a bricked ray saves ~60 ps of 270 (1 M TOF LORs x 4
-// rays at 200 x 200 x 128: 1.08 -> 0.76 ms).  The size is a frame's: LORs in
-// locality order read one frame at a time (8 frames of 128 x 128 x 64, 160 M
-// LORs: 98.7 ms from bricks, 87.5 from rows; in no order 1.6 M 1.29 / 1.41).
+// A forward projection of n LORs of `rays` rays of image `im` reads a bricked copy
+// of it (a.xb, in c->fwd) by useBricks' rule, where there are rays enough for the
+// copy, ~3 ps a voxel, to be worth it.
 // Not where the caller captures the stream: a forward used no scratch of the
 // context before it used bricks, and the graph's replays cannot be ordered
 // with the context's other calls.  The caller ends the use after its launch.
-bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, int64_t rays,
+bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, bool dd, int rays,
                   ScratchUse& use, int* status)
 {
 	*status = YRTMI_OK;
 	const int64_t bvox = brickFrameVoxels(im.nx, im.ny, im.nz);
-	if (!useBricks(im.nx, im.ny, im.nz, 1) || rays * kBrickRays < im.nvox * im.nt ||
+	if (!useBricks(im.nx, im.ny, im.nz, im.nt, dd, rays, a.L.n) ||
+	    a.L.n * rays * kBrickRays < im.nvox * im.nt ||
 	    callerCaptures(c) || !reserve(c, c->fwd, 2, sizeof(float) * (size_t)(bvox * im.nt)))
 		return false;
 	*status = use.begin(c, c->fwd);
@@ -545,7 +550,9 @@ bool streamShape(yrtmi_ctx* c, const KArgs& a, bool em, StreamShape& s)
 	                : std::min<int64_t>(64, s.T.ntx + s.T.nty + s.T.ntz - 2);
 	if (s.recPer > kStreamRecords)
 		return false;
-	s.brick = (em && useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt)) ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt : 0;
+	s.brick = em && callBricks(a, a.im)
+	              ? brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt
+	              : 0;
 	s.list = (em && (a.c.meas || a.c.sens || a.c.att)) ? std::min(a.L.n, kStreamList) : 0;
 	return true;
 }
@@ -599,7 +606,7 @@ int sensImage(yrtmi_ctx* c, KArgs& a, ScratchUse& use)
 	int r = YRTMI_OK;
 	a.xb = nullptr;
 	if (a.att != nullptr)
-		(void)brickForward(c, a, a.attIm, a.att, a.L.n, use, &r);
+		(void)brickForward(c, a, a.attIm, a.att, false, 1, use, &r);
 	return r;
 }
 
@@ -1340,7 +1347,8 @@ int yrtmi_forward(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 		return fail(YRTMI_EINVAL, "forward: null image or output");
 	a.x = img;
 	ScratchUse use;
-	const bool bricks = brickForward(c, a, a.im, img, l->n * (int64_t)a.pr.numRays, use, &r);
+	const bool bricks = brickForward(c, a, a.im, img, a.pr.type == YRTMI_PROJ_DD,
+	                                 a.pr.numRays, use, &r);
 	if (r)
 		return r;
 	// (3 M DD LORs of 200 x 200 x 128 from bricks: TOF 4.3 -> 2.7 ms, without
@@ -2007,14 +2015,14 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	const bool dd = p->d.type == YRTMI_PROJ_DD;
 	if (im->nx > 1024 || im->ny > 1024 || im->nz > 1024)
 		return fail(YRTMI_EINVAL, "plan: image dimensions above 1024");
-	if (useBricks(a.im.nx, a.im.ny, a.im.nz, a.im.nt))
+	if (callBricks(a, a.im))
 	{
-		// the bricked image of the planned EM ratio, sized here (a DD ratio does
-		// without where there is no memory for it)
+		// the bricked image of the planned EM ratio, sized here (a DD ratio, and that
+		// of a smaller image, does without where there is no memory for it)
 		if (!reserve(c, c->em, 0,
 		             sizeof(float) *
 		                 (size_t)(brickFrameVoxels(a.im.nx, a.im.ny, a.im.nz) * a.im.nt)) &&
-		    !dd)
+		    !dd && a.im.nvox * a.im.nt >= kBrickVoxels)
 			return fail(YRTMI_ENOMEM, "plan: bricked image");
 	}
 	const int R = p->d.numRays;

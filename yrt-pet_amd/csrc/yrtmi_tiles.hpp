@@ -283,17 +283,40 @@ hipError_t launchChunkSort(bool dd, const DPlan& pl, const TileChunk* chunks, in
 // workgroup per chunk, or `persistent` workgroups on the chunk queue.
 hipError_t launchTileBack(const KArgs& a, const DTiles& T, const DPlanRead& pl,
                           const float* v, float* y, int persistent, hipStream_t st);
-// Whether Siddon forward projections of an image gather from its bricked
-// copy: of 2 M voxels (8 MB) and more, which an XCD's 4 MB L2 does not hold.
-// A smaller image is in L2 anyway, and the bricked walk's extra instructions
-// show: 1 M TOF rays of 96 x 96 x 48 111 us from rows and 140 bricked, of 200
-// x 200 x 128 190 and 163.
+// Whether forward projections of n LORs of `rays` rays (DD: one) gather from the
+// image's bricked copy.  A brick's line serves segments of a ray that rows split
+// over lines; the four lanes of a LOR's rays side by side share rows' lines as
+// well, and the bricked Siddon walk has a quarter more instructions.  So four rays
+// per LOR and more take bricks where an XCD's 4 MB L2 holds less than half of a
+// frame (LORs in locality order read one frame at a time), fewer rays and DD from small
+// images on, where the call is long enough for the copy (its launch, and 3 ps a
+// voxel).  Rows / bricks, us, EM ratios of list-mode events of a phantom, in
+// locality order and as acquired:
+//   2 M LORs of  96 x 96 x 48            128 x 128 x 96           4 M: 200 x 200 x 128
+//   1 ray        491 / 399  903 / 856    870 / 761  1468 / 1329  3030 / 2603  7682 / 5340
+//   1 ray, TOF   308 / 296  500 / 483    520 / 498   766 / 717   1564 / 1497  3026 / 2333
+//   3 rays, TOF  629 / 613  903 / 800   1088 / 950  1527 / 1347
+//   4 rays       968 / 1008 1100 / 1132 1462 / 1503 2284 / 1875  5177 / 4712  9923 / 6773
+//   4 rays, TOF  530 / 620  583 / 663    784 / 826  1077 / 974   2358 / 2210  3810 / 2842
+//   DD          1222 / 1295 2128 / 1796 2566 / 2055 5363 / 3717
+//   DD, TOF      828 / 698  1146 / 930  1997 / 1479 2530 / 1896
+// 4 rays at 128^3: 1479 / 1487 and 2152 / 1820 with TOF, 3067 / 3069 and 5535 / 4147
+// without; 8 frames of 128 x 128 x 64 1239 / 1369, 1401 / 1481.  Fewer LORs of 96 x
+// 96 x 48, TOF, in order: 1 ray 250 k 54 / 61, 500 k 95 / 101, 1 M 171 / 169; 3 rays
+// 125 k 51 / 61, 250 k 102 / 104; DD 125 k 70 / 70; of 64^3, 1 ray, 500 k 70 / 69.
 // (A frame's bricks are indexed in 32 bits, padding included, which a frame
 // of few voxels along one axis, or of just below 2^31, may exceed.)
-inline bool useBricks(int64_t nx, int64_t ny, int64_t nz, int64_t frames)
+constexpr int64_t kBrickVoxels = int64_t(1) << 21;
+inline bool useBricks(int64_t nx, int64_t ny, int64_t nz, int64_t frames, bool dd, int rays,
+                      int64_t n)
 {
-	return nx * ny * nz * frames >= (int64_t(1) << 21) &&
-	       brickFrameVoxels((int)nx, (int)ny, (int)nz) < (int64_t(1) << 31);
+	if (brickFrameVoxels((int)nx, (int)ny, (int)nz) >= (int64_t(1) << 31))
+		return false;
+	const int64_t frame = nx * ny * nz, all = frame * frames;
+	if (!dd && rays >= 4)
+		return frame >= kBrickVoxels;
+	return all >= kBrickVoxels || (dd ? all >= (1 << 20) && n >= (1 << 17)
+	                                  : all >= (1 << 18) && n * rays >= (1 << 19));
 }
 // xb (nt frames of brickFrameVoxels floats) = bricked copy of x (nt frames
 // of the image's voxels), padding voxels 0.
