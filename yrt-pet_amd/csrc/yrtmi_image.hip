@@ -74,16 +74,15 @@ __host__ __device__ constexpr int psfPitch(int hx) { return (kPsfTX + 2 * hx + 7
 
 __global__ void __launch_bounds__(256) kPsfXY(const float* __restrict__ in,
                                               float* __restrict__ out, PsfTaps tx, PsfTaps ty,
-                                              int nx, int ny, int TY, unsigned gx)
+                                              int nx, int ny, int TY, int ty0)
 {
 	extern __shared__ float sm[];
 	const int hx = tx.n / 2, hy = ty.n / 2;
 	const int pitch = psfPitch(hx), rows = TY + 2 * hy;
 	float* patch = sm;
 	float* mid = sm + pitch * rows;  // rows of kPsfTX, kPsfTX + 1 apart
-	// (a plane's tiles along blockIdx.x, which alone is not held to 65535)
-	const int x0 = (int)(blockIdx.x % gx) * kPsfTX, y0 = (int)(blockIdx.x / gx) * TY;
-	const int64_t plane = (int64_t)blockIdx.y * nx * ny;
+	const int x0 = (int)blockIdx.x * kPsfTX, y0 = (ty0 + (int)blockIdx.y) * TY;
+	const int64_t plane = (int64_t)blockIdx.z * nx * ny;
 	// util::circular (Tools.cpp:160-167): one wrap (h < n); elements that no
 	// output inside the image needs are read somewhere inside it
 	auto wrap = [](int q, int n) {
@@ -153,13 +152,13 @@ constexpr int kPsfMz = 16;
 
 __global__ void __launch_bounds__(256) kPsfZ(const float* __restrict__ in,
                                              float* __restrict__ out, PsfTaps t, int nxy, int nz,
-                                             unsigned gc)
+                                             int tz0)
 {
-	const int i = (int)(blockIdx.x % gc * blockDim.x + threadIdx.x);
+	const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
 	if (i >= nxy)
 		return;
-	const int z0 = (int)(blockIdx.x / gc) * kPsfMz;
-	const float* p = in + (int64_t)blockIdx.y * nxy * nz + i;
+	const int z0 = (tz0 + (int)blockIdx.y) * kPsfMz;
+	const float* p = in + (int64_t)blockIdx.z * nxy * nz + i;
 	float acc[kPsfMz];
 	convolveLine<kPsfMz>(
 	    t,
@@ -169,7 +168,7 @@ __global__ void __launch_bounds__(256) kPsfZ(const float* __restrict__ in,
 		    return p[(int64_t)(q < nz ? q : 0) * nxy];
 	    },
 	    acc);
-	float* o = out + (int64_t)blockIdx.y * nxy * nz + i;
+	float* o = out + (int64_t)blockIdx.z * nxy * nz + i;
 #pragma unroll
 	for (int j = 0; j < kPsfMz; j++)
 		if (z0 + j < nz)
@@ -185,18 +184,22 @@ hipError_t launchPsf(const float* in, float* tmp, float* out, const PsfTaps* t, 
 	};
 	const int TY = ldsOf(32) <= 65536 ? 32 : 16;
 	const size_t lds = ldsOf(TY);
-	const unsigned gx = (unsigned)((nx + kPsfTX - 1) / kPsfTX),
-	               gy = (unsigned)((ny + TY - 1) / TY);
+	const unsigned gx = (unsigned)((nx + kPsfTX - 1) / kPsfTX);
+	const int gy = (ny + TY - 1) / TY, gz = (nz + kPsfMz - 1) / kPsfMz;
 	const int nxy = nx * ny;
-	const unsigned gc = (unsigned)((nxy + 255) / 256), gz = (unsigned)((nz + kPsfMz - 1) / kPsfMz);
-	// (a grid has at most 65535 planes and frames)
+	const unsigned gc = (unsigned)((nxy + 255) / 256);
+	// (a grid has at most 65535 tiles, planes and frames on its second and third axes)
+	constexpr int64_t kAxis = 65535;
+	auto part = [&](int64_t n) { return (unsigned)std::min(kAxis, n); };
 	const int64_t planes = frames * nz;
-	for (int64_t p = 0; p < planes; p += 65535)
-		kPsfXY<<<dim3(gx * gy, (unsigned)std::min<int64_t>(65535, planes - p)), 256, lds, st>>>(
-		    in + p * nxy, tmp + p * nxy, t[0], t[1], nx, ny, TY, gx);
-	for (int64_t f = 0; f < frames; f += 65535)
-		kPsfZ<<<dim3(gc * gz, (unsigned)std::min<int64_t>(65535, frames - f)), 256, 0, st>>>(
-		    tmp + f * nz * nxy, out + f * nz * nxy, t[2], nxy, nz, gc);
+	for (int64_t p = 0; p < planes; p += kAxis)
+		for (int y = 0; y < gy; y += (int)kAxis)
+			kPsfXY<<<dim3(gx, part(gy - y), part(planes - p)), 256, lds, st>>>(
+			    in + p * nxy, tmp + p * nxy, t[0], t[1], nx, ny, TY, y);
+	for (int64_t f = 0; f < frames; f += kAxis)
+		for (int z = 0; z < gz; z += (int)kAxis)
+			kPsfZ<<<dim3(gc, part(gz - z), part(frames - f)), 256, 0, st>>>(
+			    tmp + f * nz * nxy, out + f * nz * nxy, t[2], nxy, nz, z);
 	return hipGetLastError();
 }
 
