@@ -173,6 +173,45 @@ def test_sensitivity_of_histogram_subset(gpu, dd, att):
     pair(gpu, im, p, lambda u: ctx.back(p, im, u, B, v))
 
 
+@pytest.mark.parametrize("src", ["histo", "bins", "pairs", "pairs_dd"])
+def test_batches_of_every_source(gpu, src):
+    """Several batches, the last one ragged, of each LOR source, with frames,
+    motion and every per-LOR factor: a batch starts inside each array, and
+    inside the subset iterator."""
+    dd = src == "pairs_dd"
+    frames = 0 if src == "histo" else 2
+    im = yrtmi.ImageParams(64, 60, 30, 4.0, 4.5, 2.0, nt=max(1, frames))
+    n = 4_400_001 if dd else 800_001
+    ctx, p, L, rng = setup(im, n if src[0] == "p" else 10, proj="DD" if dd else "Siddon",
+                           rays=1 if dd else 16, tof=250.0, frames=frames if src[0] == "p" else 0,
+                           motion=4 if src[0] == "p" else 0, gpu=gpu)
+    t = lambda a, d: torch.from_numpy(a.astype(d)).to(gpu)
+    if src == "histo":
+        L = yrtmi.LorSet.histo_subset(ctx, 3, 1)
+        n = L.n
+    elif src == "bins":
+        total = int(np.prod(ctx.histo_dims))
+        L = yrtmi.LorSet.bins_(t(rng.integers(0, total + 10, n), np.int32),
+                               tof=t(rng.normal(0.0, 100.0, n), np.float32),
+                               frame=t(rng.integers(-1, frames, n), np.int32))
+    # bytes a LOR: ray table (64 a ray, DD 128), records (12 a ray and tile, DD 8)
+    assert n * (256 if dd else 16 * (64 + 6 * 12)) > 1 << 30
+    g = torch.Generator(gpu).manual_seed(5)
+    v = torch.rand(n, device=gpu, generator=g)
+    pair(gpu, im, p, lambda u: ctx.back(p, im, u, L, v))
+    x = 0.5 + torch.rand(im.shape, device=gpu, generator=g)
+    c = {k: 0.2 + torch.rand(n, device=gpu, generator=g)
+         for k in ("meas", "sens", "att", "randoms", "scatter")}
+    pair(gpu, im, p, lambda u: ctx.em_subset(p, im, x, u, L, randoms=c["randoms"],
+                                             scatter=c["scatter"]))
+    c["meas"][::3] = 0.0
+    pair(gpu, im, p, lambda u: ctx.em_subset(p, im, x, u, L, **c))
+    if frames == 0:
+        mu_im = yrtmi.ImageParams(161, 127, 103, 1.5, 1.75, 1.0)  # bricked
+        mu = 0.05 * torch.rand(mu_im.shape, device=gpu, generator=g)
+        pair(gpu, im, p, lambda u: ctx.sensitivity(p, im, u, L, att_im=mu_im, att_img=mu, sens=v))
+
+
 def test_batch_of_high_footprints(gpu):
     """Crystals 240 voxels high over one column of 64 tiles: some 30 records
     for each LOR that meets the image, for which there is room."""

@@ -64,8 +64,29 @@ def lines(n, im, seed):
                                       ((256, 256, 128, 1.6, 1.6, 1.6), False)], ids=str)
 @pytest.mark.parametrize("tof", [0, 1])
 def test_pieces_are_the_walks(hw, im, exact, tile, tof):
+    check(hw, im, exact, tile, tof, lines(12000, im, 7))
+
+
+@pytest.mark.parametrize("tile", [(5, 5, 3), (3, 2, 1)], ids=str)
+@pytest.mark.parametrize("tof", [0, 1])
+def test_pieces_of_voxels_below_a_millionth_of_the_scanner(hw, tile, tof):
+    """Where a position may be planes off (sidCoarse): voxels of 2^-11 mm (short
+    binary fractions: the same pieces) under lines of 840 mm through them."""
+    im = (70, 66, 40, 2.0 ** -11, 2.0 ** -11, 2.0 ** -11)
+    rng = np.random.default_rng(3)
     n = 12000
-    p1, p2, tv = lines(n, im, 7)
+    at = rng.uniform(-0.5, 0.5, (n, 3)) * np.array(im[:3]) * im[3]
+    a, slope = rng.uniform(0, 2 * np.pi, n), rng.uniform(-1, 1, n)
+    slope[::4] = 0.0
+    d = 420 * np.stack([np.cos(a), np.sin(a), slope], 1)
+    p1, p2 = ((at + q * d).astype(np.float32) for q in (1, -1))
+    check(hw, im, True, tile, tof, (np.ascontiguousarray(p1), np.ascontiguousarray(p2),
+                                    rng.uniform(-400, 400, n).astype(np.float32)))
+
+
+def check(hw, im, exact, tile, tof, rays):
+    p1, p2, tv = rays
+    n = len(p1)
     f = np.float32
     L = [f(im[i]) * f(im[3 + i]) for i in range(3)]
     imp = np.array([*im, *L, max(L[:2]) / 2 - max(im[3:5]) / 1000], f)
