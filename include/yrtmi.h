@@ -468,15 +468,18 @@ int yrtmi_permute(yrtmi_ctx* ctx, const void* src, int elem_bytes,
  * boundaries).
  *
  * Limits: nx, ny, nz <= 1024; n * num_rays < 2^32; tiles (frames included)
- * at most the device's LDS per workgroup / 12 bytes (5459 with 64 KB).  The
+ * at most the device's LDS per workgroup / 8 bytes.  The
  * call synchronises the context's stream and allocates device memory
  * (yrtmi_plan_info's bytes); the plan owns it.
  *
- * Options (NULL: defaults): chunk_records, records per workgroup (0: 4096);
+ * Options (NULL: defaults): chunk_records, records per workgroup (0: 4096,
+ * fewer where the plan would not fill the chip);
  * tile_shape, YRTMI_TILE_16x16x16 (default), YRTMI_TILE_32x32x16,
  * YRTMI_TILE_32x32x32 or YRTMI_TILE_32x32x8 (voxels of the image held per
- * workgroup; the tile is accumulated in LDS in 64-bit fixed point, FP32 for
- * the 32x32x32 shape); persistent,
+ * workgroup; the tile is accumulated in LDS in 64-bit fixed point, DD in FP64,
+ * FP32 for the 32x32x32 shape; in fixed point a term keeps fewer than 24 bits
+ * from 2^-15 of the launch's median value times the largest segment weight
+ * down, none from 2^-39); persistent,
  * 0 for one workgroup per chunk, else that many workgroups taking chunks from
  * a device queue (changeable with yrtmi_plan_set_persistent); max_bytes, 0
  * for no limit, else the device memory the plan may hold: a plan that would

@@ -2111,8 +2111,8 @@ int yrtmi_plan_create(yrtmi_ctx* c, const yrtmi_proj* p, const yrtmi_image* im,
 	};
 	if (l->n == 0)
 		return cleanup(YRTMI_OK);
-	// length classes: up to 8, as long as tiles x classes stays within
-	// 8192 bins (64 KB of fill-pass LDS) and the LDS limit
+	// length classes: up to 8 (DD 16), as long as tiles x classes stays within
+	// kMaxBins and the device's LDS per workgroup (8 bytes a bin in the fill pass)
 	DPlan pl{};
 	pl.R = R;
 	pl.C = 1;

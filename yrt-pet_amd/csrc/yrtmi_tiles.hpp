@@ -24,8 +24,8 @@ __host__ __device__ constexpr int tileThreads(int shape)
 }
 // Binning keeps a counter (count pass) and a counter plus a 32-bit base
 // (fill pass; a plan holds fewer than 2^32 records) per (tile, length
-// class) in LDS; length classes are added while tiles x classes <=
-// kMaxBins / 2.
+// class) in LDS; length classes are added while tiles x classes <= kMaxBins
+// and the device's LDS per workgroup holds them.
 constexpr int kMaxBins = 16384;
 constexpr int kMaxClasses = 16;
 // Threads of a binning workgroup, which share its LDS counters (64 KB in the
