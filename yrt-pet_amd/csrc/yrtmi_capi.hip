@@ -467,18 +467,22 @@ bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, bo
 //
 // The direct kernels are bound by FP32 global atomics (21 G/s): a
 // backprojection of 1 M TOF LORs x 4 rays into 200 x 200 x 128 took 19.4 ms
-// and takes 1.4, 150 k DD TOF LORs into 95 x 97 x 47 took 5.6 and take 1.0,
+// and takes 1.5, 150 k DD TOF LORs into 95 x 97 x 47 took 5.6 and take 0.7,
 // an EM subset of 2 M corrected LORs into 181 x 173 x 109 took 35.3 and takes
-// 4.1 (of which its forward 1.6).  The binned path's fixed cost (eight
-// launches a batch, the scan, a pass over the touched tiles) is 70 to 100 us;
+// 4.1 (of which its forward 1.4).  The binned path's fixed cost (eight
+// launches a batch, the scan, a pass over the touched tiles) is 60 to 100 us;
 // the direct one's is the fold of its partial images, 30 us at 96 x 96 x 48
-// and 90 us at 200 x 200 x 128.  The lines (streamMinRays) lie where the two
-// meet; direct / binned, us:
-//   Siddon, 96 x 96 x 48    65 k rays  back 70-86 / 83-86  EM  88-109 / 121-128
-//   Siddon, 200 x 200 x 128 16 k rays  back 86-126 / 81-106 EM 122-221 / 142-230
-//                           32 k rays  back 110-178 / 88-109 EM 146-274 / 148-232
-//   DD                      32 k LORs  back 404-993 / 388-863 EM 440-1245 / 574-1313
-//                           65 k LORs  back 518-1544 / 419-938 EM 650-1901 / 591-1386
+// and 90 us at 200 x 200 x 128.  The lines (streamMinRays) lie where no data
+// measured is slower binned: random crystal pairs, half of which miss the image,
+// meet there; list-mode events of a phantom, long lines that crowd its atomics, from
+// 16 k to 32 k rays on.  Direct / binned, us, back and EM:
+//   random pairs, Siddon   96 x 96 x 48  65 k rays  70-86 / 83-86    88-109 / 121-128
+//                      200 x 200 x 128   32 k rays 110-178 / 88-109 146-274 / 148-232
+//                 DD                     65 k LORs 518-1544 / 419-938 650-1901 / 591-1386
+//   phantom, Siddon, TOF   96 x 96 x 48  32 k rays   98 / 70    112 / 87
+//                                       131 k rays  353 / 112   376 / 144
+//                      200 x 200 x 128   32 k rays  228 / 95    263 / 131
+//            DD, TOF       96 x 96 x 48  65 k LORs  402 / 339   446 / 371
 // ---------------------------------------------------------------------------
 // scratch per context, beside an EM subset's copy of the image
 constexpr size_t kStreamBytes = size_t(1) << 30;
