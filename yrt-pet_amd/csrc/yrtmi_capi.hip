@@ -404,9 +404,9 @@ bool callBricks(const KArgs& a, const DImage& im)
 
 // The bricked copy of a.x for the EM ratio's forward by useBricks' rule; the image
 // is read as it is while recording without the buffer (a Siddon call of 2^21
-// voxels and more is refused that) and by a DD call that the caller captures.  The caller ends the use
-// after its launch.  Tile plans reserve the buffer for their image, so planned
-// EM calls never allocate.
+// voxels and more is refused that) and by a DD call that the caller captures.
+// The caller ends the use after its launch.  Tile plans reserve the buffer for
+// their image, so planned EM calls never allocate.
 int brickImage(yrtmi_ctx* c, KArgs& a, ScratchUse& use)
 {
 	if (!callBricks(a, a.im))
@@ -474,8 +474,8 @@ bool brickForward(yrtmi_ctx* c, KArgs& a, const DImage& im, const float* img, bo
 // the direct one's is the fold of its partial images, 30 us at 96 x 96 x 48
 // and 90 us at 200 x 200 x 128.  The lines (streamMinRays) lie where no data
 // measured is slower binned: random crystal pairs, half of which miss the image,
-// meet there; list-mode events of a phantom, long lines that crowd its atomics, from
-// 16 k to 32 k rays on.  Direct / binned, us, back and EM:
+// meet there, list-mode events of a phantom at 16 k to 32 k rays.  Direct / binned,
+// us, back and EM:
 //   random pairs, Siddon   96 x 96 x 48  65 k rays  70-86 / 83-86    88-109 / 121-128
 //                      200 x 200 x 128   32 k rays 110-178 / 88-109 146-274 / 148-232
 //                 DD                     65 k LORs 518-1544 / 419-938 650-1901 / 591-1386
