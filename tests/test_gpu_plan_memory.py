@@ -4,6 +4,7 @@ dropped plan is still queued (bit for bit: with one chunk per tile each voxel
 is one exact fixed-point sum, whatever the records' order); the memory kept
 counts as free, and goes back to the driver when asked for."""
 import ctypes as C
+import gc
 
 import numpy as np
 import pytest
@@ -55,6 +56,7 @@ def test_plans_in_reused_memory(gpu):
 
 def kept_plan(gpu, n):
     """A context whose pool holds a dropped plan of n LORs."""
+    gc.collect()  # (no other test's context goes meanwhile)
     sc = yrtmi.Scanner("t", 96.0, 4.0, 4.0, 10.0, 180.0, 128, 24)
     im = yrtmi.ImageParams(64, 64, 32, 4.0, 4.0, 4.0)
     ctx = yrtmi.Context(sc)

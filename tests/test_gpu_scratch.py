@@ -4,6 +4,8 @@ GPU.  Bars: forward projections and ratios are the same sums in the same
 order, or, where a call reads rows instead of bricks, of the same values: bit
 for bit.  Backprojections 1e-5 relative L2, as in test_gpu_stream.py."""
 import ctypes as C
+import gc
+import threading
 
 import pytest
 import torch
@@ -112,8 +114,57 @@ def test_graph_launched_through_another_context(gpu):
             assert max(e) <= 1e-5
 
 
+def test_graph_and_eager_calls_from_two_threads(gpu):
+    """A graph launched through a second context by one thread while another
+    makes eager calls on the context that recorded it: each use of the scratch
+    waits for the last one, whichever thread it came from."""
+    im = yrtmi.ImageParams(64, 60, 30, 4.0, 4.5, 2.0)
+    ctx, p, L, _ = setup(im, 70_000, rays=2, tof=250.0, gpu=gpu)
+    other = setup(im, 90_000, rays=2, tof=250.0, gpu=gpu, seed=9)[2]
+    ctx2 = yrtmi.Context(ctx.scanner)
+    g = torch.Generator(gpu).manual_seed(5)
+    v, w = torch.rand(L.n, device=gpu, generator=g), torch.rand(other.n, device=gpu, generator=g)
+    refs = [torch.zeros(im.shape, device=gpu) for _ in range(2)]
+    u, u2 = (torch.zeros(im.shape, device=gpu) for _ in range(2))
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    ctx.set_stream(s1)
+    ctx2.set_stream(s2)
+    ctx.back(p, im, refs[1], other, w)
+    ctx.back(p, im, refs[0], L, v)
+    with ctx.graph() as gr:
+        ctx.fill(u, 0.0)
+        ctx.back(p, im, u, L, v)
+    torch.cuda.synchronize()
+    errors = []
+
+    def run(call):
+        try:
+            for _ in range(40):
+                call()
+        except Exception as e:  # noqa: BLE001 (reported by the test's thread)
+            errors.append(e)
+
+    def eager():
+        ctx.fill(u2, 0.0)
+        ctx.back(p, im, u2, other, w)
+
+    threads = [threading.Thread(target=run, args=(f,)) for f in
+               (lambda: capi.check(capi.lib().yrtmi_graph_launch(ctx2.h, gr.h)), eager)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    e = [rel_l2(a.cpu().numpy(), b.cpu().numpy()) for a, b in zip((u, u2), refs)]
+    print(f"replays {e[0]:.2e}, eager {e[1]:.2e}", flush=True)
+    assert max(e) <= 1e-5
+
+
 def test_scratch_of_a_graph_outlives_its_context(gpu):
     """Scratch that a graph refers to goes back with the graph, not before."""
+    gc.collect()  # (no other test's context goes meanwhile)
     im = yrtmi.ImageParams(64, 60, 30, 4.0, 4.5, 2.0)
     ctx, p, L, _ = setup(im, 70_000, rays=2, tof=250.0, gpu=gpu)
     keep = yrtmi.Context(ctx.scanner)
