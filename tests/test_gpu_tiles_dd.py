@@ -4,8 +4,9 @@ with the plan) against the direct DD backprojection and the CPU oracle.
 
 A DD plan's record is a (LOR, tile) pair; the tile kernel sweeps the LOR's
 footprint over the tile's slices with the direct sweep's arithmetic, so the
-voxel weights are bit-identical and only the summation order differs (the
-tile sums in 64-bit fixed point, then one FP32 atomic per voxel).  Bars
+voxel weights are the same up to their last bits (the PSF integral from its
+segment table) and the summation order differs (the tile sums in FP64, FP32 for
+32x32x32 tiles, then one FP32 atomic per voxel).  Bars
 (written in each test): planned vs direct <= 2e-6 relative L2; planned vs
 oracle <= 1e-5 (projection-space) / 1e-4 (EM image), as for the direct path.
 """
@@ -99,7 +100,7 @@ CASES = [
 
 def test_dd_psf_tables_beyond_lds(gpu):
     """A projection PSF of 48 rows of 57 taps (~34 KB per direction) is
-    larger than the DD kernels stage in LDS (16 KB): the planned
+    larger than the DD kernels stage in LDS (28 KB): the planned
     backprojection and EM ratio read it from global memory, and match the
     direct kernels and the oracle as the staged tables do."""
     sc = scanner()
@@ -140,8 +141,10 @@ def test_dd_psf_tables_beyond_lds(gpu):
 
 def test_dd_plan_record_order_keeps_the_image(gpu):
     """DD records ordered by footprint voxels per slice (kChunkSort) or not
-    (a single-use plan): one chunk per tile, so the fixed-point tile sums
-    and the images are bit-identical."""
+    (a single-use plan): one chunk per tile, so a voxel is one FP64 sum in two
+    orders (some 10^4 terms of one sign: within 10^4 x 2^-53, 2^-16 of an FP32
+    ulp), rounded once: the same, or where that falls on a rounding's edge one
+    ulp apart."""
     sc, im, pp, ctx, p = setup(gpu, "dyadic", None, psf=True)
     n = 40000
     ev = events(sc, n, 141, None)
@@ -158,7 +161,33 @@ def test_dd_plan_record_order_keeps_the_image(gpu):
     ctx.back(p, im, b, L, vg, plan=single)
     ctx.synchronize()
     assert np.count_nonzero(a.cpu().numpy()) > 1000
-    np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
+    np.testing.assert_array_max_ulp(a.cpu().numpy(), b.cpu().numpy(), maxulp=1)
+
+
+@pytest.mark.parametrize("shape", [0, 1, 2, 3])
+def test_dd_psf_tables_that_fill_their_lds(gpu, shape):
+    """29 rows of 57 taps take 28304 of the 28672 bytes of LDS that the DD
+    kernels stage, beside the tile (128 KB for shapes 1 and 2)."""
+    sc = scanner()
+    im = IMAGES["dyadic"]()
+    pp = yrtmi.ProjectorParams(sc, projectorType="DD")
+    k, s_step, ks = synth.gaussian_psf_row(2.0, k_spacing=0.125, num_s=29, s_step=8.0)
+    assert k.shape == (29, 57) and 29 * (57 + 4) * 16 == 28304
+    k = k * np.linspace(0.8, 1.2, 29, dtype=np.float32)[:, None]
+    k[:, :20] *= 1.3
+    pp.psf_kernels, pp.psf_s_step, pp.psf_k_spacing = k, s_step, ks
+    ctx = yrtmi.Context(sc)
+    p = ctx.projector(pp)
+    n = 3000
+    L = dev_lors(events(sc, n, 151, None), gpu)
+    vg = torch.from_numpy(np.random.default_rng(15).uniform(0.1, 1.0, n).astype(np.float32)).to(gpu)
+    plan = ctx.plan(p, im, L, tile_shape=shape)
+    a, b = (torch.zeros(im.shape, device=gpu) for _ in range(2))
+    ctx.back(p, im, a, L, vg)
+    ctx.back(p, im, b, L, vg, plan=plan)
+    ctx.synchronize()
+    assert float(a.abs().sum()) > 0
+    check(f"dd_psf_full_lds_shape{shape}", b.cpu().numpy(), a.cpu().numpy(), TOL_DIRECT)
 
 
 @pytest.mark.parametrize("name,image,tof,s64,psf,shape", CASES, ids=[c[0] for c in CASES])
